@@ -557,3 +557,66 @@ def tolerance(case: dict):
         return {"rel": 3e-3}
     # sums of products in the tensors' own precision, over up to a few thousand terms: 1e-6 seen
     return {"rel": 4e-6}
+
+
+# ------------------------------------------------------------------------------------------------- in 64 bits
+
+def _storage(t: ct.Tensor) -> torch.Tensor:
+    return t.buffer.storage.double()
+
+
+def _exact_transposed(s: _State):
+    x = _storage(s.x).t()
+    return [{"exp": torch.exp, "tanh": torch.tanh, "logistic": torch.sigmoid, "sqrt": torch.sqrt}[s.case["op"]](x)]
+
+
+def _exact_reduce(s: _State):
+    x = _storage(s.x)
+    of = {"sum": torch.sum, "mean": torch.mean, "max": torch.amax,
+          "magnitude-squared": lambda v, dim, keepdim: (v * v).sum(dim, keepdim=keepdim),
+          "magnitude": lambda v, dim, keepdim: (v * v).sum(dim, keepdim=keepdim).sqrt()}[s.case["op"]]
+    return [of(x, dim=1, keepdim=True), of(x, dim=0, keepdim=True).t()]
+
+
+def _exact_linear(s: _State):
+    weights, bias = (_storage(s.parameters[k]["buffer"]) for k in ("weights", "bias"))
+    x, gradient = _storage(s.inputs[0]["buffer"]), _storage(s.results[0]["gradient"])
+    return [weights, gradient.t() @ x, bias, gradient.sum(0), x, gradient @ weights, x @ weights.t() + bias, gradient]
+
+
+def _exact_convolution(s: _State):
+    weights, bias = (_storage(s.parameters[k]["buffer"]) for k in ("weights", "bias"))
+    x, gradient = _storage(s.inputs[0]["buffer"]), _storage(s.results[0]["gradient"])
+    window = {"kernel_size": s.case["window"], "padding": s.case["pad"], "stride": s.case["stride"]}
+    result, x_gradient = torch.empty_like(gradient), torch.empty_like(x)
+    weight_gradient = torch.zeros_like(weights)
+    for image in range(len(x)):
+        cells, g = torch.nn.functional.unfold(x[image:image + 1], **window)[0], gradient[image].flatten(1)
+        result[image] = (weights @ cells + bias[:, None]).view_as(result[image])
+        weight_gradient += g @ cells.t()
+        x_gradient[image] = torch.nn.functional.fold((weights.t() @ g)[None], x.shape[2:], **window)[0]
+    return [weights, weight_gradient, bias, gradient.sum((0, 2, 3)), x, x_gradient, result, gradient]
+
+
+def _exact_block(s: _State):
+    if s.case["norm"] != "batch":
+        return None
+    # The gradients have no such value where rounding decides which element of a window is the largest.
+    scale, bias = (_storage(s.parameters[k]["buffer"])[:, None, None] for k in ("scale", "bias"))
+    x = _storage(s.edges[0]["buffer"])
+    variance, mean = torch.var_mean(x, dim=(0, 2, 3), keepdim=True, correction=0)
+    normalized = scale * (x - mean) / torch.sqrt(variance + 1e-4) + bias
+    active = torch.clamp(normalized, min=0.0) if s.case["activation"] == "relu" else torch.tanh(normalized)
+    return [scale.flatten(), None, bias.flatten(), None, None, None, x, None, normalized, None, active, None, None, None]
+
+
+_EXACT = {"transposed": _exact_transposed, "reduce": _exact_reduce, "linear": _exact_linear,
+          "convolution": _exact_convolution, "block": _exact_block}
+
+
+def exact(case: dict, seed: int):
+    """None where a pass rounds once per stored value, in a fixed order, and is compared to the bit, and for the whole
+    training step, whose dropout mask only the library's generator gives."""
+    if case["kind"] not in _EXACT or case.get("datatype") == "int":
+        return None
+    return _EXACT[case["kind"]](prepare(case, seed))
