@@ -211,7 +211,9 @@ def check(status: int) -> None:
 
 def call(name: str, *args) -> None:
     """Calls entry point ``name`` and raises on a non-zero status."""
-    check(getattr(lib(), name)(*args))
+    status = getattr(_lib or lib(), name)(*args)
+    if status != 0:
+        check(status)
 
 
 def last_kernel() -> str:

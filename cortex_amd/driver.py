@@ -38,8 +38,11 @@ NUMPY_OF = {"byte": np.int8, "short": np.int16, "int": np.int32, "long": np.int6
 DATATYPE_OF_NUMPY = {np.dtype(v): k for k, v in NUMPY_OF.items()}
 
 
+_DTYPE_SIZES = {name: capi.DTYPE_SIZES[code] for name, code in capi.DTYPE_CODES.items()}
+
+
 def dtype_size(datatype: str) -> int:
-    return capi.DTYPE_SIZES[capi.DTYPE_CODES[datatype]]
+    return _DTYPE_SIZES[datatype]
 
 
 class DeviceBuffer:
@@ -80,11 +83,10 @@ class DeviceBuffer:
     def partially_alias(self, other: "DeviceBuffer") -> bool:
         """Overlapping byte ranges that do not start at the same address
         (``cuda/driver.clj:473-486``)."""
-        a0, a1 = self.ptr, self.ptr + self.nbytes
-        b0, b1 = other.ptr, other.ptr + other.nbytes
+        a0, b0 = self.ptr, other.ptr
         if a0 == b0:
             return False
-        return a0 < b1 and b0 < a1
+        return a0 < b0 + other.nbytes and b0 < a0 + self.nbytes
 
     def release(self) -> None:
         if self._owner is None and not self._released and self.ptr:
@@ -140,7 +142,8 @@ _DIMS_CACHE: dict = {}
 _DIMS_CACHE_LIMIT = 4096
 
 
-def _dims_struct(dims: dict) -> capi.CtDims:
+def _dims_ref(dims: dict):
+    """The ct_dims of ``dims`` as an argument of a call; the reference keeps the struct alive."""
     shape_in, strides_in = dims["shape"], dims["strides"]
     direct = True
     for entry in shape_in:
@@ -155,7 +158,7 @@ def _dims_struct(dims: dict) -> capi.CtDims:
             hit, key = None, None
         if hit is not None:
             return hit
-        made = capi.make_dims(shape_in, strides_in, None)
+        made = C.byref(capi.make_dims(shape_in, strides_in, None))
         if key is not None:
             if len(_DIMS_CACHE) >= _DIMS_CACHE_LIMIT:
                 _DIMS_CACHE.clear()
@@ -172,7 +175,7 @@ def _dims_struct(dims: dict) -> capi.CtDims:
                 raise TypeError("Index buffers must be integer tensors")
             shape.append(int(buf.ecount()))
             index.append(buf.ptr)
-    return capi.make_dims(shape, dims["strides"], index)
+    return C.byref(capi.make_dims(shape, dims["strides"], index))
 
 
 def _arg_order_indexes(arg_order: Sequence[str]):
@@ -249,82 +252,82 @@ class HipStream:
 
     # -- TensorMath (src/cortex/tensor/math.clj:14-104) ---------------------
     def assign_constant(self, buffer, dimensions, value, n_elems) -> None:
-        capi.call("ct_assign_constant", self.handle, buffer.ptr, C.byref(_dims_struct(dimensions)),
+        capi.call("ct_assign_constant", self.handle, buffer.ptr, _dims_ref(dimensions),
                   capi.DTYPE_CODES[buffer.datatype], float(value), int(n_elems))
 
     def assign(self, dest, dest_dims, src, src_dims, n_elems) -> None:
-        capi.call("ct_assign", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), capi.DTYPE_CODES[dest.datatype],
-                  src.ptr, C.byref(_dims_struct(src_dims)), capi.DTYPE_CODES[src.datatype], int(n_elems))
+        capi.call("ct_assign", self.handle, dest.ptr, _dims_ref(dest_dims), capi.DTYPE_CODES[dest.datatype],
+                  src.ptr, _dims_ref(src_dims), capi.DTYPE_CODES[src.datatype], int(n_elems))
 
     def unary_accum(self, dest, dest_dims, alpha, op, n_elems) -> None:
-        capi.call("ct_unary_accum", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), float(alpha),
+        capi.call("ct_unary_accum", self.handle, dest.ptr, _dims_ref(dest_dims), float(alpha),
                   capi.UNARY_OPS[op], capi.DTYPE_CODES[dest.datatype], int(n_elems))
 
     def unary_op(self, dest, dest_dims, x, x_dims, alpha, op, n_elems) -> None:
-        capi.call("ct_unary_op", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), x.ptr,
-                  C.byref(_dims_struct(x_dims)), float(alpha), capi.UNARY_OPS[op], capi.DTYPE_CODES[dest.datatype],
+        capi.call("ct_unary_op", self.handle, dest.ptr, _dims_ref(dest_dims), x.ptr,
+                  _dims_ref(x_dims), float(alpha), capi.UNARY_OPS[op], capi.DTYPE_CODES[dest.datatype],
                   int(n_elems))
 
     def binary_accum_constant(self, dest, dest_dims, dest_alpha, scalar, n_elems, operation, reverse_operands) -> None:
-        capi.call("ct_binary_accum_constant", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), float(dest_alpha),
+        capi.call("ct_binary_accum_constant", self.handle, dest.ptr, _dims_ref(dest_dims), float(dest_alpha),
                   float(scalar), int(n_elems), capi.BINARY_OPS[operation], int(bool(reverse_operands)),
                   capi.DTYPE_CODES[dest.datatype])
 
     def binary_op_constant(self, dest, dest_dims, x, x_dims, x_alpha, scalar, n_elems, operation, reverse_operands) -> None:
-        capi.call("ct_binary_op_constant", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), x.ptr,
-                  C.byref(_dims_struct(x_dims)), float(x_alpha), float(scalar), int(n_elems),
+        capi.call("ct_binary_op_constant", self.handle, dest.ptr, _dims_ref(dest_dims), x.ptr,
+                  _dims_ref(x_dims), float(x_alpha), float(scalar), int(n_elems),
                   capi.BINARY_OPS[operation], int(bool(reverse_operands)), capi.DTYPE_CODES[dest.datatype])
 
     def binary_accum(self, dest, dest_dims, dest_alpha, y, y_dims, y_alpha, n_elems, operation, reverse_operands,
                      dest_requires_cas) -> None:
-        capi.call("ct_binary_accum", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), float(dest_alpha), y.ptr,
-                  C.byref(_dims_struct(y_dims)), float(y_alpha), int(n_elems), capi.BINARY_OPS[operation],
+        capi.call("ct_binary_accum", self.handle, dest.ptr, _dims_ref(dest_dims), float(dest_alpha), y.ptr,
+                  _dims_ref(y_dims), float(y_alpha), int(n_elems), capi.BINARY_OPS[operation],
                   int(bool(reverse_operands)), int(bool(dest_requires_cas)), capi.DTYPE_CODES[dest.datatype])
 
     def binary_op(self, dest, dest_dims, x, x_dims, x_alpha, y, y_dims, y_alpha, n_elems, operation) -> None:
-        capi.call("ct_binary_op", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), x.ptr,
-                  C.byref(_dims_struct(x_dims)), float(x_alpha), y.ptr, C.byref(_dims_struct(y_dims)), float(y_alpha),
+        capi.call("ct_binary_op", self.handle, dest.ptr, _dims_ref(dest_dims), x.ptr,
+                  _dims_ref(x_dims), float(x_alpha), y.ptr, _dims_ref(y_dims), float(y_alpha),
                   int(n_elems), capi.BINARY_OPS[operation], capi.DTYPE_CODES[dest.datatype])
 
     def ternary_op(self, dest, dest_dims, x, x_dims, x_alpha, y, y_dims, y_alpha, z, z_dims, z_alpha, n_elems,
                    operation) -> None:
-        capi.call("ct_ternary_op", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), x.ptr,
-                  C.byref(_dims_struct(x_dims)), float(x_alpha), y.ptr, C.byref(_dims_struct(y_dims)), float(y_alpha),
-                  z.ptr, C.byref(_dims_struct(z_dims)), float(z_alpha), int(n_elems), capi.TERNARY_OPS[operation],
+        capi.call("ct_ternary_op", self.handle, dest.ptr, _dims_ref(dest_dims), x.ptr,
+                  _dims_ref(x_dims), float(x_alpha), y.ptr, _dims_ref(y_dims), float(y_alpha),
+                  z.ptr, _dims_ref(z_dims), float(z_alpha), int(n_elems), capi.TERNARY_OPS[operation],
                   capi.DTYPE_CODES[dest.datatype])
 
     def ternary_op_constant(self, dest, dest_dims, a, a_dims, a_alpha, b, b_dims, b_alpha, constant, n_elems, operation,
                             arg_order) -> None:
-        capi.call("ct_ternary_op_constant", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), a.ptr,
-                  C.byref(_dims_struct(a_dims)), float(a_alpha), b.ptr, C.byref(_dims_struct(b_dims)), float(b_alpha),
+        capi.call("ct_ternary_op_constant", self.handle, dest.ptr, _dims_ref(dest_dims), a.ptr,
+                  _dims_ref(a_dims), float(a_alpha), b.ptr, _dims_ref(b_dims), float(b_alpha),
                   float(constant), int(n_elems), capi.TERNARY_OPS[operation], _arg_order_indexes(arg_order),
                   capi.DTYPE_CODES[dest.datatype])
 
     def ternary_op_constant_constant(self, dest, dest_dims, a, a_dims, a_alpha, const_1, const_2, n_elems, operation,
                                      arg_order) -> None:
-        capi.call("ct_ternary_op_constant_constant", self.handle, dest.ptr, C.byref(_dims_struct(dest_dims)), a.ptr,
-                  C.byref(_dims_struct(a_dims)), float(a_alpha), float(const_1), float(const_2), int(n_elems),
+        capi.call("ct_ternary_op_constant_constant", self.handle, dest.ptr, _dims_ref(dest_dims), a.ptr,
+                  _dims_ref(a_dims), float(a_alpha), float(const_1), float(const_2), int(n_elems),
                   capi.TERNARY_OPS[operation], _arg_order_indexes(arg_order), capi.DTYPE_CODES[dest.datatype])
 
     def unary_reduce(self, output, output_dims, input_alpha, input, input_dims, op) -> None:
-        capi.call("ct_unary_reduce", self.handle, output.ptr, C.byref(_dims_struct(output_dims)), float(input_alpha),
-                  input.ptr, C.byref(_dims_struct(input_dims)), capi.REDUCE_OPS[op], capi.DTYPE_CODES[output.datatype])
+        capi.call("ct_unary_reduce", self.handle, output.ptr, _dims_ref(output_dims), float(input_alpha),
+                  input.ptr, _dims_ref(input_dims), capi.REDUCE_OPS[op], capi.DTYPE_CODES[output.datatype])
 
     # -- neural-network tensor ops (tensor/math.clj:176-189) ------------------
     def activation_gradient(self, input_gradient, input_grad_dims, output_gradient, output_grad_dims, output,
                             output_dims, op, element_count) -> None:
-        capi.call("ct_activation_gradient", self.handle, input_gradient.ptr, C.byref(_dims_struct(input_grad_dims)),
-                  output_gradient.ptr, C.byref(_dims_struct(output_grad_dims)), output.ptr,
-                  C.byref(_dims_struct(output_dims)), capi.ACTIVATION_OPS[op], int(element_count),
+        capi.call("ct_activation_gradient", self.handle, input_gradient.ptr, _dims_ref(input_grad_dims),
+                  output_gradient.ptr, _dims_ref(output_grad_dims), output.ptr,
+                  _dims_ref(output_dims), capi.ACTIVATION_OPS[op], int(element_count),
                   capi.DTYPE_CODES[input_gradient.datatype])
 
     def softmax_eltwise(self, output, output_dims, input, input_dims) -> None:
-        capi.call("ct_softmax_eltwise", self.handle, output.ptr, C.byref(_dims_struct(output_dims)), input.ptr,
-                  C.byref(_dims_struct(input_dims)), capi.DTYPE_CODES[output.datatype])
+        capi.call("ct_softmax_eltwise", self.handle, output.ptr, _dims_ref(output_dims), input.ptr,
+                  _dims_ref(input_dims), capi.DTYPE_CODES[output.datatype])
 
     def softmax_spatial(self, output, output_dims, input, input_dims) -> None:
-        capi.call("ct_softmax_spatial", self.handle, output.ptr, C.byref(_dims_struct(output_dims)), input.ptr,
-                  C.byref(_dims_struct(input_dims)), capi.DTYPE_CODES[output.datatype])
+        capi.call("ct_softmax_spatial", self.handle, output.ptr, _dims_ref(output_dims), input.ptr,
+                  _dims_ref(input_dims), capi.DTYPE_CODES[output.datatype])
 
     # -- convolution (tensor/math.clj:185-220); buffers are packed, the workspace is the caller's --
     def convolution_descriptor(self, datatype, out_channels, in_channels, kern_width, kern_height, pad_x, pad_y,
@@ -383,16 +386,16 @@ class HipStream:
     # -- local response normalization (tensor/math.clj:240-252); the descriptor is a plain map --
     def lrn_forward(self, output, output_dims, input, input_dims, lrn_descriptor) -> None:
         d = lrn_descriptor
-        capi.call("ct_lrn_forward", self.handle, output.ptr, C.byref(_dims_struct(output_dims)), input.ptr,
-                  C.byref(_dims_struct(input_dims)), int(d["n"]), float(d["k"]), float(d["alpha"]), float(d["beta"]),
+        capi.call("ct_lrn_forward", self.handle, output.ptr, _dims_ref(output_dims), input.ptr,
+                  _dims_ref(input_dims), int(d["n"]), float(d["k"]), float(d["alpha"]), float(d["beta"]),
                   capi.DTYPE_CODES[output.datatype])
 
     def lrn_backward(self, input_grad, input_grad_dims, output, output_dims, input, input_dims, output_grad,
                      output_grad_dims, lrn_descriptor) -> None:
         d = lrn_descriptor
-        capi.call("ct_lrn_backward", self.handle, input_grad.ptr, C.byref(_dims_struct(input_grad_dims)), output.ptr,
-                  C.byref(_dims_struct(output_dims)), input.ptr, C.byref(_dims_struct(input_dims)), output_grad.ptr,
-                  C.byref(_dims_struct(output_grad_dims)), int(d["n"]), float(d["k"]), float(d["alpha"]),
+        capi.call("ct_lrn_backward", self.handle, input_grad.ptr, _dims_ref(input_grad_dims), output.ptr,
+                  _dims_ref(output_dims), input.ptr, _dims_ref(input_dims), output_grad.ptr,
+                  _dims_ref(output_grad_dims), int(d["n"]), float(d["k"]), float(d["alpha"]),
                   float(d["beta"]), capi.DTYPE_CODES[output.datatype])
 
     # -- gemm!, gemv! (tensor/math.clj:106-123) ---------------------------------
@@ -468,7 +471,9 @@ class HipStream:
             a, b = distribution["minimum"], distribution["maximum"]
         else:
             raise ValueError(f"Unrecognized distribution: {distribution}")
-        n = int(np.prod([int(v) for v in dest_dims["shape"]], dtype=np.int64))
+        n = 1
+        for v in dest_dims["shape"]:
+            n *= int(v)
         capi.call("ct_rand", self.handle, dest.ptr, n, capi.DTYPE_CODES[dest.datatype], capi.DISTRIBUTIONS[kind],
                   float(a), float(b), self._rand_seed, self._rand_calls)
         self._rand_calls += 1

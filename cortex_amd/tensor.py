@@ -90,6 +90,9 @@ def is_tensor(x) -> bool:
 
 
 def _is_number(x) -> bool:
+    kind = type(x)
+    if kind is Tensor or kind is float or kind is int:
+        return kind is not Tensor
     return isinstance(x, (int, float, np.integer, np.floating)) and not isinstance(x, bool)
 
 
@@ -197,11 +200,11 @@ def to_vector(t: Tensor) -> Tensor:
 
 
 def as_2d_matrix(t: Tensor) -> Tensor:
-    return in_place_reshape(t, dims.to_2d_shape(t.dimensions))
+    return t._with(dimensions=dims.as_matrix(t.dimensions, dims.to_2d_shape))
 
 
 def as_batch_matrix(t: Tensor) -> Tensor:
-    return in_place_reshape(t, dims.to_batch_shape(t.dimensions))
+    return t._with(dimensions=dims.as_matrix(t.dimensions, dims.to_batch_shape))
 
 
 def transpose(t: Tensor, reorder_vec) -> Tensor:
@@ -249,13 +252,17 @@ def columns(t: Tensor):
 # ---------------------------------------------------------------- checks
 
 def _ensure_datatypes(datatype, *args) -> None:
-    if not all(a.get_datatype() == datatype for a in args):
-        raise TensorError(f"Not all arguments match required datatype {datatype}: {[a.get_datatype() for a in args]}")
+    for t in args:
+        if t.get_datatype() != datatype:
+            raise TensorError(f"Not all arguments match required datatype {datatype}: "
+                              f"{[a.get_datatype() for a in args]}")
 
 
 def _ensure_same_device(*args) -> None:
-    if not all(a.device is args[0].device for a in args[1:]):
-        raise TensorError("Tensor arguments are not all on same device")
+    device = args[0].device
+    for t in args:
+        if t.device is not device:
+            raise TensorError("Tensor arguments are not all on same device")
 
 
 def _check_partial_alias(*args) -> None:
@@ -267,6 +274,9 @@ def _check_partial_alias(*args) -> None:
 def _ensure_broadcast_rules(*args) -> None:
     """``ensure-broadcast-rules`` (``tensor.clj:592-604``): every operand
     dimension must divide the max dimension."""
+    key = dims.direct_key(*[a.dimensions for a in args])
+    if key is not None and dims.commensurate(key):
+        return
     info = dims.dimension_seq_to_max_shape(*[a.dimensions for a in args])
     max_shape = info["max-shape"]
     for d in info["dimensions"]:
