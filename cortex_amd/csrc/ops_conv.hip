@@ -368,15 +368,44 @@ int forward_t(void* stream, T* output, double output_alpha, const T* input, cons
   return CT_OK;
 }
 
-// weight_gradient = T(alpha * weight_gradient + sum over the images of partial[image]), in double
-template <class T>
+// weight_gradient = T(alpha * weight_gradient + sum over the partials of partial[p]), in double.
+// Few elements and many partials (a digit network: 4608 elements, 128 images) leave one lane
+// per element with 18 blocks and a serial chain of 128 loads, each the latency of memory.
+// SLICES lanes share an element instead, every slice taking each SLICES-th partial, and the
+// slices are added in order through LDS: [128, 4608] float 30.9 -> 4.1 us, [64, 36864]
+// 24.3 -> 4.9 us.  A handful of partials stays with one lane per element.
+template <class T, int SLICES>
 __global__ void __launch_bounds__(kBlock) conv_sum_partials_kernel(T* weight_gradient, const T* partials, uint32_t n,
-                                                                    uint32_t images, double alpha) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  double acc = alpha == 0.0 ? 0.0 : alpha * (double)weight_gradient[i];
-  for (uint32_t b = 0; b < images; ++b) acc += (double)partials[(int64_t)b * n + i];
-  weight_gradient[i] = (T)acc;
+                                                                    uint32_t count, double alpha) {
+  constexpr uint32_t COLS = kBlock / SLICES;
+  const uint32_t col = threadIdx.x % COLS, slice = threadIdx.x / COLS;
+  const uint32_t i = blockIdx.x * COLS + col;
+  double acc = 0.0;
+  if (i < n) {
+#pragma unroll 4
+    for (uint32_t p = slice; p < count; p += SLICES) acc += (double)partials[(int64_t)p * n + i];
+  }
+  if constexpr (SLICES > 1) {
+    __shared__ double slices[SLICES][COLS];
+    slices[slice][col] = acc;
+    __syncthreads();
+    if (slice != 0) return;
+#pragma unroll
+    for (int s = 1; s < SLICES; ++s) acc += slices[s][col];
+  }
+  if (i < n) weight_gradient[i] = (T)(alpha == 0.0 ? acc : alpha * (double)weight_gradient[i] + acc);
+}
+
+template <class T>
+void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t n, int64_t count, double alpha) {
+  constexpr int kSlices = 8;
+  if (count >= kSlices)
+    hipLaunchKernelGGL((conv_sum_partials_kernel<T, kSlices>),
+                       dim3((uint32_t)((n + kBlock / kSlices - 1) / (kBlock / kSlices))), dim3(kBlock), 0, s,
+                       weight_gradient, partials, (uint32_t)n, (uint32_t)count, alpha);
+  else
+    hipLaunchKernelGGL((conv_sum_partials_kernel<T, 1>), dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                       s, weight_gradient, partials, (uint32_t)n, (uint32_t)count, alpha);
 }
 
 template <class T>
@@ -411,9 +440,7 @@ int backward_weights_t(void* stream, T* weight_gradient, double alpha, const T* 
         return rc;
       ++used;
     }
-    hipLaunchKernelGGL((conv_sum_partials_kernel<T>), dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                       weight_gradient, reinterpret_cast<const T*>(scratch), (uint32_t)n, (uint32_t)(nb * used),
-                       b0 == 0 ? (double)al : 1.0);
+    sum_partials(s, weight_gradient, reinterpret_cast<const T*>(scratch), n, nb * used, b0 == 0 ? (double)al : 1.0);
   }
   note_kernel("gemm+conv_sum_partials");
   return after_launch(s);
