@@ -1,0 +1,46 @@
+// conv_products.h -- what ops_conv.hip hands to the matrix-core products of ops_conv_mfma.hip.
+#pragma once
+
+#include "common.h"
+
+namespace cthip {
+
+// The cells of a window that the products keep a mask of.
+constexpr int kConvMaskTaps = 32;
+
+// forward:       output[m][j]    = sum over k of weights[m][k] * unrolled[k][j] (+ beta * output[m][j]),
+//                                  the unrolled input written to the workspace; m out channels, k cells
+// backward-data: workspace[m][j] = sum over k of weights[k][m] * output[k][j]; m cells, k out channels
+// over the n positions j of all images, numbered on.
+struct ConvProductArgs {
+  const float* weights;
+  const float* input;
+  float* output;
+  float* workspace;
+  int64_t in_image, out_image, conv_image;
+  uint32_t m, n, k, n_rows;
+  uint32_t in_plane, in_h, in_w, kw, kh;
+  int32_t px, py, sx, sy;
+  float beta;
+  uint32_t units;
+  FastDiv m_tiles_fd, rows_fd, out_w_fd, taps_fd, kw_fd;
+};
+void conv_product(hipStream_t s, ConvProductArgs a, bool forward);
+// The tiles that such a product has.
+int64_t conv_product_units(int64_t m, int64_t n);
+
+// partials[split][m][n] = sum over the split's positions of output_gradient[m][p] * unrolled[n][p]
+struct ConvWeightArgs {
+  const float* output_gradient;
+  const float* workspace;
+  float* partials;
+  int64_t out_image, conv_image;
+  uint32_t m, n, n_rows;
+  uint32_t piece_len, pieces, pieces_per_split;   // positions of a piece; pieces of all images; of a split
+  uint32_t units;
+  FastDiv parts_fd, tiles_fd, n_tiles_fd;          // parts: pieces of one image
+};
+void conv_weight_gradient(hipStream_t s, ConvWeightArgs a, int64_t splits);
+int64_t conv_weight_tiles(int64_t m, int64_t n);   // blocks to a split
+
+}  // namespace cthip

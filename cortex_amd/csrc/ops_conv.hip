@@ -23,14 +23,17 @@
 //              that came from it, windows in increasing (row, column) order,
 //              which is the order in which that walk reaches the element: the
 //              same roundings, no atomics.  Reads the workspace once.
-//   products   ONE strided-batched rocBLAS call per method (an image's product
-//              alone leaves most of the device idle).  The weight gradient, which
+//   products   float: kernels of their own on the matrix cores (ops_conv_mfma.hip),
+//              the unrolling done inside the forward product.  double, and float
+//              where the rules below say so: ONE strided-batched rocBLAS call per
+//              method (an image's product alone leaves most of the device idle).  The weight gradient, which
 //              the reference accumulates image after image into one matrix, is
 //              formed as per-image products in the stream's scratch memory and
 //              summed over the images in double by a small kernel.
 #include <algorithm>
 
 #include "common.h"
+#include "conv_products.h"
 
 using namespace cthip;
 
@@ -353,10 +356,59 @@ void roll_back(hipStream_t s, const T* workspace, T* input_gradient, const ct_co
   }
 }
 
+// Whether a float product goes to the matrix-core kernels: where they have the tiles to fill the
+// chip, or a k so short that the chain over it is over before the library's second launch is.
+// A tile of 16 k takes about 0.9 us when a block has the unit to itself, whatever the number of
+// blocks, and the library's two launches 15 to 20 us: forward over [1, 64, 56, 56] and 64 windows
+// of 3 x 3 (k 576, 25 tiles) 43 us here, 19 there; over [3, 15, 109, 109] (k 135, 279 tiles) 28 and
+// 36; over [134, 94, 15, 15] and 145 windows (k 846, 707 tiles) 147 both; over [34, 30, 57, 57] and
+// 106 of 5 x 5 (k 750, 1493 tiles) 250 and 347.
+bool matrix_core_product(const ct_conv_desc& d, const ConvShape& sh, int64_t m, int64_t k) {
+  constexpr int64_t kFullChip = 768, kShortChain = 192;
+  return sh.in_image > 0 && d.kernel_width * d.kernel_height <= kConvMaskTaps &&
+         (k <= kShortChain || conv_product_units(m, sh.batch * sh.n_rows) >= kFullChip);
+}
+
+void run_product(hipStream_t s, float* output, float beta, const float* input, const float* weights, float* workspace,
+                 const ct_conv_desc& d, const ConvShape& sh, bool forward) {
+  ConvProductArgs a{};
+  a.weights = weights;
+  a.in_image = sh.in_image; a.out_image = sh.out_image; a.conv_image = sh.conv_image;
+  a.m = (uint32_t)(forward ? d.out_channels : sh.n_cols);
+  a.k = (uint32_t)(forward ? sh.n_cols : d.out_channels);
+  a.n_rows = (uint32_t)sh.n_rows;
+  a.in_plane = (uint32_t)(sh.in_h * sh.in_w);
+  a.in_h = (uint32_t)sh.in_h; a.in_w = (uint32_t)sh.in_w;
+  a.kw = (uint32_t)d.kernel_width; a.kh = (uint32_t)d.kernel_height;
+  a.px = d.pad_x; a.py = d.pad_y; a.sx = d.stride_x; a.sy = d.stride_y;
+  a.beta = beta;
+  a.rows_fd = FastDiv((uint32_t)sh.n_rows);
+  a.out_w_fd = FastDiv((uint32_t)sh.out_w);
+  a.taps_fd = FastDiv((uint32_t)(d.kernel_width * d.kernel_height));
+  a.kw_fd = FastDiv((uint32_t)d.kernel_width);
+  // the positions and the tiles of a launch are counted in 31 bits
+  const int64_t step = images_per_launch(sh.n_rows * (a.m / 4096 + 1));
+  for (int64_t b0 = 0; b0 < sh.batch; b0 += step) {
+    const int64_t nb = std::min(step, sh.batch - b0);
+    a.input = forward ? input + b0 * sh.in_image : nullptr;
+    a.output = output + b0 * sh.out_image;
+    a.workspace = workspace + b0 * sh.conv_image;
+    a.n = (uint32_t)(nb * sh.n_rows);
+    conv_product(s, a, forward);
+  }
+}
+
 template <class T>
 int forward_t(void* stream, T* output, double output_alpha, const T* input, const T* weights, T* workspace,
               const ct_conv_desc& d, const ConvShape& sh, int dtype) {
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if constexpr (std::is_same<T, float>::value) {
+    if (sh.n_cols >= 4 && matrix_core_product(d, sh, d.out_channels, sh.n_cols)) {
+      run_product(s, output, (float)output_alpha, input, weights, workspace, d, sh, true);
+      note_kernel("conv_product");
+      return after_launch(s);
+    }
+  }
   unroll(s, input, workspace, d, sh);
   if (int rc = after_launch(s)) return rc;
   // output[b] [out_channels, n_rows] = weights [out_channels, n_cols] x unrolled[b] [n_cols, n_rows]
@@ -408,12 +460,57 @@ void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t 
                        s, weight_gradient, partials, (uint32_t)n, (uint32_t)count, alpha);
 }
 
+// The splits of the matrix-core weight gradient: at most kWeightBlocks blocks in all, two to a
+// compute unit and none left over (64 splits of 9 tiles, 2.25 blocks to a unit, took 215 us where
+// 56 take 180), every split a run of pieces of at most kPieceLength positions.  The partials stay within what the library's
+// products take (a matrix an image, at most 256 MiB) or the megabyte that every scratch block has.
+ConvWeightArgs weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t* splits) {
+  constexpr int64_t kWeightBlocks = 512, kPieceLength = 512;
+  ConvWeightArgs a{};
+  a.out_image = sh.out_image; a.conv_image = sh.conv_image;
+  a.m = (uint32_t)d.out_channels; a.n = (uint32_t)sh.n_cols; a.n_rows = (uint32_t)sh.n_rows;
+  const int64_t parts = (sh.n_rows + kPieceLength - 1) / kPieceLength;
+  a.piece_len = (uint32_t)(((sh.n_rows + parts - 1) / parts + 63) / 64 * 64);
+  const int64_t used_parts = (sh.n_rows + a.piece_len - 1) / a.piece_len;
+  a.pieces = (uint32_t)(sh.batch * used_parts);
+  a.parts_fd = FastDiv((uint32_t)used_parts);
+  const int64_t result = (int64_t)a.m * a.n * (int64_t)sizeof(float);
+  const int64_t tiles = conv_weight_tiles(a.m, a.n);
+  const int64_t fit = std::max<int64_t>(std::min<int64_t>(sh.batch * result, int64_t(256) << 20), int64_t(1) << 20) / result;
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({kWeightBlocks / tiles, fit, (int64_t)a.pieces}));
+  a.pieces_per_split = (uint32_t)((a.pieces + want - 1) / want);
+  *splits = (a.pieces + a.pieces_per_split - 1) / a.pieces_per_split;
+  return a;
+}
+
+// Images of a few hundred positions that fall badly into tiles of 64 leave a large product to the
+// library: [32, 256, 14, 14] under 256 windows of 3 x 3 (196 positions in four tiles) 127 us
+// here, 98 there.  Rows shorter than a 16-byte load are the library's too.
+bool matrix_core_weight_gradient(int64_t result, const ConvShape& sh) {
+  constexpr double kLarge = 2e9;
+  const bool ragged = (sh.n_rows + 63) / 64 * 64 * 5 > sh.n_rows * 6;
+  return sh.n_rows >= 4 && !(ragged && 2.0 * (double)result * (double)(sh.batch * sh.n_rows) > kLarge);
+}
+
 template <class T>
 int backward_weights_t(void* stream, T* weight_gradient, double alpha, const T* output_gradient, T* workspace,
                        const ct_conv_desc& d, const ConvShape& sh, int dtype) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t n = (int64_t)d.out_channels * sh.n_cols;
   CT_REQUIRE(n <= (int64_t(1) << 31) - 1, "convolution: the weight matrix exceeds the supported range");
+  if (std::is_same<T, float>::value && matrix_core_weight_gradient(n, sh)) {
+    int64_t splits;
+    ConvWeightArgs a = weight_args(d, sh, &splits);
+    void* scratch = nullptr;
+    if (int rc = stream_scratch(s, (size_t)(splits * n) * sizeof(float), &scratch)) return rc;
+    a.output_gradient = reinterpret_cast<const float*>(output_gradient);
+    a.workspace = reinterpret_cast<const float*>(workspace);
+    a.partials = reinterpret_cast<float*>(scratch);
+    conv_weight_gradient(s, a, splits);
+    sum_partials(s, reinterpret_cast<float*>(weight_gradient), a.partials, n, splits, (double)(float)alpha);
+    note_kernel("conv_weight_gradient+conv_sum_partials");
+    return after_launch(s);
+  }
   // A product of few outputs over very many positions (a first layer: 64 x 27 outputs, 50176
   // positions) would occupy one workgroup per image: the positions are cut into pieces of about
   // kPositionsPerPiece, every piece a product of its own, and the sum takes the pieces too.
@@ -451,6 +548,14 @@ int backward_data_t(void* stream, T* input_gradient, const T* output_gradient, c
                     const ct_conv_desc& d, const ConvShape& sh, int dtype) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   // unrolled[b] [n_cols, n_rows] = weights^T [n_cols, out_channels] x output_gradient[b] [out_channels, n_rows]
+  if constexpr (std::is_same<T, float>::value) {
+    if (sh.conv_image > 0 && matrix_core_product(d, sh, sh.n_cols, d.out_channels)) {
+      run_product(s, const_cast<float*>(output_gradient), 0.f, nullptr, weights, workspace, d, sh, false);
+      roll_back(s, workspace, input_gradient, d, sh);
+      note_kernel("conv_product+conv_roll");
+      return after_launch(s);
+    }
+  }
   if (sh.conv_image > 0)
     if (int rc = gemm_strided_batched(stream, workspace, sh.n_rows, sh.conv_image, 1, 0, 1.0, weights, sh.n_cols,
                                       d.out_channels, sh.n_cols, 0, output_gradient, sh.n_rows, sh.n_rows,

@@ -37,3 +37,67 @@ def test_weight_gradient_over_many_images(P, code, batch):
     for alpha in (0.0, 2.0):
         P.run(H.convolution, "backward_weights", vec(wg), alpha, vec(og), vec(inp), vec(work), desc, batch, h, w, h, w)
         H.assert_bit_exact(wg.download(), wg.host, f"convolution-backward-weights, alpha {alpha}")
+
+
+# (batch, in channels, out channels, height, width, kernel width, kernel height, pad, stride): the edges of the tiles
+# (32, 64 and 128 rows, 128 and 64 columns, 16 k, 64 positions of a piece), of a run of sums (128 k), of the mask of taps
+# (32), of the rows (4 positions, 4 cells) and of the routes (k 192, 768 tiles)
+PRODUCT_CASES = [
+    (1, 1, 1, 2, 2, 1, 1, 0, 1),        # 4 positions, 1 cell: the product is the library's
+    (1, 1, 3, 1, 3, 1, 1, 0, 1),        # 3 positions
+    (3, 4, 2, 2, 2, 1, 1, 0, 1),        # 4 positions, 4 cells
+    (2, 5, 31, 7, 9, 3, 1, 0, 1),       # 15 cells, 49 positions of odd alignment
+    (2, 16, 32, 8, 8, 1, 1, 0, 1),      # exactly one tile of k, one piece of positions
+    (1, 17, 33, 5, 13, 1, 1, 0, 1),     # one more of each: 17 cells, 65 positions, 33 rows
+    (1, 7, 64, 9, 7, 3, 3, 1, 1),       # 63 positions and cells
+    (5, 3, 65, 11, 10, 3, 3, 1, 2),     # 65 rows, strided, 30 positions
+    (2, 14, 130, 9, 8, 3, 3, 1, 1),     # 126 cells: one run; 130 rows in tiles of 64
+    (2, 15, 128, 9, 15, 3, 3, 0, 1),    # 135 cells: two runs; tiles of 128 rows
+    (1, 21, 9, 6, 6, 3, 3, 1, 1),       # 189 cells: the last short chain
+    (1, 22, 9, 6, 6, 3, 3, 1, 1),       # 198 cells, few tiles: the library
+    (2, 3, 200, 5, 5, 3, 3, 1, 1),      # the same for backward-data, over 200 out channels
+    (1, 2, 4, 27, 19, 5, 5, 2, 1),      # 25 taps, 513 positions: two pieces
+    (1, 2, 4, 13, 12, 6, 6, 2, 1),      # 36 taps: no mask
+    (64, 23, 6, 40, 40, 3, 3, 1, 1),    # 800 tiles over 207 cells
+]
+
+
+@pytest.mark.parametrize("case", PRODUCT_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_products_at_the_edges_of_their_tiles(P, case):
+    """Whole numbers whose sums stay below 2^24: exact in any order, so everything agrees to the bit."""
+    batch, cin, cout, h, w, kw, kh, pad, stride = case
+    oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kw) // stride + 1
+    n_rows, n_cols = oh * ow, cin * kw * kh
+    desc = H.conv_desc(cin, cout, kw, kh, pad, pad, stride, stride)
+    geometry = (desc, batch, h, w, oh, ow)
+    rng = np.random.default_rng(sum(case))
+    ints = lambda n: rng.integers(-2, 3, n).astype(np.float32)
+    inp, weights, og = P.buf(ints(batch * cin * h * w)), P.buf(ints(cout * n_cols)), P.buf(ints(batch * cout * n_rows))
+    out, wg, ig = P.buf(ints(batch * cout * n_rows)), P.buf(ints(cout * n_cols)), P.buf(ints(batch * cin * h * w))
+    work = P.buf(np.full(batch * n_rows * n_cols + 5, 7.0, np.float32))
+
+    def unrolled(what):
+        n = batch * n_rows * n_cols
+        got = work.download()
+        H.assert_bit_exact(np.ascontiguousarray(got[:n].reshape(batch, n_cols, n_rows).transpose(0, 2, 1)),
+                           work.host[:n].reshape(batch, n_rows, n_cols), what)
+        assert np.all(got[n:] == 7.0), what
+
+    def route(m, k):
+        rows = 32 if m <= 32 else 64 if -(-m // 64) % 2 else 128
+        tiles = -(-m // rows) * -(-batch * n_rows // (64 if rows == 128 else 128))
+        return kw * kh <= 32 and (k <= 192 or tiles >= 768)
+
+    for alpha in (0.0, 2.0):
+        kernel = P.run(H.convolution, "forward", vec(out), alpha, vec(inp), vec(weights), vec(work), *geometry)
+        assert (kernel == "conv_product") == (n_cols >= 4 and route(cout, n_cols)), kernel
+        H.assert_bit_exact(out.download(), out.host, f"convolution-forward, alpha {alpha}")
+        unrolled("unrolled input")
+    for alpha in (0.0, 2.0):
+        kernel = P.run(H.convolution, "backward_weights", vec(wg), alpha, vec(og), vec(inp), vec(work), *geometry)
+        assert (kernel == "conv_weight_gradient+conv_sum_partials") == (n_rows >= 4), kernel
+        H.assert_bit_exact(wg.download(), wg.host, f"convolution-backward-weights, alpha {alpha}")
+    kernel = P.run(H.convolution, "backward_data", vec(ig), 0.0, vec(og), vec(weights), vec(work), *geometry)
+    assert (kernel == "conv_product+conv_roll") == route(n_cols, cout), kernel
+    H.assert_bit_exact(ig.download(), ig.host, "convolution-backward-data")
+    unrolled("unrolled gradient")
