@@ -173,6 +173,7 @@ struct BandArgs {
   uint32_t fast_div;   // float tensor and kw * kh <= kRecipTable - 1
   double recip;        // RN(1 / (kw * kh))
   FastDiv bands_fd, dest_w_fd, dest_plane_fd, sx_fd, sy_fd;
+  FastDiv row_pieces_fd, in_h_fd;   // 16-byte pieces of an input row; input rows of a plane
 };
 
 constexpr int kRecipTable = 256;
@@ -548,6 +549,94 @@ __global__ void __launch_bounds__(kBlock) pool_backward_band_kernel(const BandAr
   }
 }
 
+// The same for the maximum over K x K windows, K 2 or 3, at stride 2: which windows an input lies
+// under follows from the parity of its coordinates, so a lane takes a 16-byte piece of one input
+// row, reads the few window values and gradients above it once, and adds without loops or
+// divisions (the general form spends four divisions and a loop of its own bounds per element and
+// was bound by that).  Rows of any width: the last piece of a row goes element by element.
+// Windows in increasing (row, column) order, as above: the same bits.
+// [32, 64, 112, 112] float, 3 x 3, pad 1: 83.8 -> 69.2 us (360 MB).
+template <class T, int K>
+__global__ void __launch_bounds__(kBlock) pool_backward_max_stride2_kernel(const BandArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  T* tile_v = reinterpret_cast<T*>(smem);
+  T* tile_g = tile_v + a.cap;
+  uint32_t group, band;
+  a.bands_fd.divmod(blockIdx.x, group, band);
+  const uint32_t p0 = group * a.pb, np = min(a.pb, a.planes - p0);
+  const int32_t iy0 = (int32_t)(band * a.br), rows = min((int32_t)a.br, a.in_h - iy0);
+  int32_t oy_first = 0, n_src_rows = a.out_h;
+  if (a.pb == 1) {
+    oy_first = min(a.out_h, max(0, (iy0 + a.py - K + 2) >> 1));
+    n_src_rows = max(0, min(a.out_h, ((iy0 + rows - 1 + a.py) >> 1) + 1) - oy_first);
+  }
+  const uint32_t len = a.pb > 1 ? np * a.out_plane : (uint32_t)(n_src_rows * a.out_w);
+  const int64_t src_at = (int64_t)p0 * a.out_plane + (int64_t)oy_first * a.out_w;
+  const uint32_t lead_v = stage_linear(tile_v, reinterpret_cast<const T*>(a.out_values) + src_at, len);
+  const uint32_t lead_g = stage_linear(tile_g, reinterpret_cast<const T*>(a.out_grad) + src_at, len);
+  __syncthreads();
+  const int64_t dest_at = (int64_t)p0 * a.in_plane + (int64_t)iy0 * a.in_w;
+  T* ig = reinterpret_cast<T*>(a.dest) + dest_at;
+  const T* in = reinterpret_cast<const T*>(a.in) + dest_at;
+
+  auto add_windows = [&](auto parity) {
+    constexpr int VEC = 16 / sizeof(T), P = decltype(parity)::value;   // pieces start at P modulo 2, padding counted
+    constexpr int kFirst = K == 3 && P == 0 ? 1 : 0;                   // windows read left of the piece's own
+    constexpr int kWindows = kFirst + (P + VEC - 1) / 2 + 1;
+    const uint32_t n_pieces = np * (uint32_t)rows * a.row_pieces_fd.d;
+    for (uint32_t q = threadIdx.x; q < n_pieces; q += kBlock) {
+      uint32_t r, c, j = 0, iyl;
+      a.row_pieces_fd.divmod(q, r, c);
+      iyl = r;
+      if (a.pb > 1) a.in_h_fd.divmod(r, j, iyl);
+      const int32_t ix0 = (int32_t)c * VEC, left = a.in_w - ix0;
+      const int64_t at = (int64_t)r * a.in_w + ix0;
+      T acc[VEC], v[VEC];
+      if (left >= VEC) {
+        __builtin_memcpy(acc, ig + at, 16);
+        __builtin_memcpy(v, in + at, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          acc[e] = e < left ? ig[at + e] : (T)0;
+          v[e] = e < left ? in[at + e] : (T)0;
+        }
+      }
+      const int32_t ty = iy0 + (int32_t)iyl + a.py, oy_last = min(ty >> 1, a.out_h - 1);
+      const int32_t ox0 = ((ix0 + a.px) >> 1) - kFirst;
+      for (int32_t oy = max((ty - K + 2) >> 1, 0); oy <= oy_last; ++oy) {
+        const int32_t row_at = (int32_t)(j * a.out_plane) + (oy - oy_first) * a.out_w;
+        T wv[kWindows], wg[kWindows];
+        bool there[kWindows];
+#pragma unroll
+        for (int i = 0; i < kWindows; ++i) {
+          const int32_t ox = ox0 + i;
+          there[i] = (uint32_t)ox < (uint32_t)a.out_w;
+          const int32_t cell = row_at + (there[i] ? ox : 0);
+          wv[i] = tile_v[(int32_t)lead_v + cell];
+          wg[i] = tile_g[(int32_t)lead_g + cell];
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          constexpr int kTwo = K == 3;
+          const int t = P + e, last = kFirst + t / 2;
+          if (kTwo && t % 2 == 0 && there[last - 1] && v[e] == wv[last - 1]) acc[e] = acc[e] + wg[last - 1];
+          if (there[last] && v[e] == wv[last]) acc[e] = acc[e] + wg[last];
+        }
+      }
+      if (left >= VEC) {
+        __builtin_memcpy(ig + at, acc, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (e < left) ig[at + e] = acc[e];
+      }
+    }
+  };
+  if (a.px & 1) add_windows(std::integral_constant<int, 1>{});
+  else add_windows(std::integral_constant<int, 0>{});
+}
+
 // ------------------------------------------------------------------ 2 x 2 windows that tile the input
 
 // kernel 2 x 2, stride 2, no padding, in_h = 2 * out_h, in_w = 2 * out_w, in_w a
@@ -721,6 +810,13 @@ void launch_band(hipStream_t s, bool forward, dim3 grid, size_t lds, const BandA
 
 template <class T, int OP>
 void launch_band_window(hipStream_t s, bool forward, dim3 grid, size_t lds, const BandArgs& a) {
+  if constexpr (OP == CT_POOL_MAX) {
+    if (!forward && a.sx == 2 && a.sy == 2 && a.kw == a.kh && (a.kw == 2 || a.kw == 3)) {
+      if (a.kw == 2) hipLaunchKernelGGL((pool_backward_max_stride2_kernel<T, 2>), grid, dim3(kBlock), lds, s, a);
+      else hipLaunchKernelGGL((pool_backward_max_stride2_kernel<T, 3>), grid, dim3(kBlock), lds, s, a);
+      return;
+    }
+  }
   if (a.kw == 2 && a.kh == 2) launch_band<T, OP, 2, 2>(s, forward, grid, lds, a);
   else if (a.kw == 3 && a.kh == 3) launch_band<T, OP, 3, 3>(s, forward, grid, lds, a);
   else launch_band<T, OP, 0, 0>(s, forward, grid, lds, a);
@@ -861,6 +957,8 @@ int pool_launch(hipStream_t s, bool forward, void* dest, const void* in, const v
     a.dest_plane_fd = FastDiv((uint32_t)dest_plane);
     a.sx_fd = FastDiv((uint32_t)d.stride_x);
     a.sy_fd = FastDiv((uint32_t)d.stride_y);
+    a.row_pieces_fd = FastDiv((uint32_t)((sh.in_w + 16 / (int64_t)sizeof(T) - 1) / (16 / (int64_t)sizeof(T))));
+    a.in_h_fd = FastDiv((uint32_t)sh.in_h);
     const size_t lds = (size_t)arrays * a.cap * sizeof(T) + (size_t)kRecipTable * sizeof(double);
     note_kernel(forward ? "pool_forward_band" : "pool_backward_band");
     for (int64_t p0 = 0; p0 < sh.planes; p0 += planes_per_launch) {
