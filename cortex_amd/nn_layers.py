@@ -239,6 +239,13 @@ class Dropout:
             raise ValueError(f"Unknown dropout distribution {kind}")
         if kind == "bernoulli":
             maximum = float(np.float32(self.layer["probability"]))
+            # A driver may have the chain below as one launch that stores the same values (the mask of a digit
+            # network's 128 x 128 units: two launches of 2.4 us on the GPU, some 20 us of host time, against one).
+            fused = getattr(ct.check_stream(), "dropout_bernoulli_mask", None)
+            whole = all(ct.dense(t) and t.buffer.ecount() == t.ecount() for t in (self.mult_buffer, self.rand_buffer))
+            if fused is not None and whole and 0.0 < maximum <= 1.0:
+                fused(self.mult_buffer.buffer, self.rand_buffer.buffer, self.layer["probability"])
+                return
             distribution = ct.flat_distribution(minimum=maximum - 1.0, maximum=maximum)
         else:
             distribution = ct.gaussian_distribution(mean=1, variance=self.layer["variance"])
