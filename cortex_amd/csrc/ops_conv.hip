@@ -398,12 +398,20 @@ void run_product(hipStream_t s, float* output, float beta, const float* input, c
   }
 }
 
+bool overlap(const float* a, int64_t a_count, const float* b, int64_t b_count) {
+  const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+  return a0 < b0 + (uintptr_t)b_count * sizeof(float) && b0 < a0 + (uintptr_t)a_count * sizeof(float);
+}
+
 template <class T>
 int forward_t(void* stream, T* output, double output_alpha, const T* input, const T* weights, T* workspace,
               const ct_conv_desc& d, const ConvShape& sh, int dtype) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   if constexpr (std::is_same<T, float>::value) {
-    if (sh.n_cols >= 4 && matrix_core_product(d, sh, d.out_channels, sh.n_cols)) {
+    // The kernel gathers the input while other blocks store the output: a call in place, or on buffers that
+    // share some of their bytes, unrolls the whole input first.
+    if (sh.n_cols >= 4 && matrix_core_product(d, sh, d.out_channels, sh.n_cols) &&
+        !overlap(output, sh.batch * sh.out_image, input, sh.batch * sh.in_image)) {
       run_product(s, output, (float)output_alpha, input, weights, workspace, d, sh, true);
       note_kernel("conv_product");
       return after_launch(s);

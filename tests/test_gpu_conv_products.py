@@ -101,3 +101,19 @@ def test_products_at_the_edges_of_their_tiles(P, case):
     assert (kernel == "conv_product+conv_roll") == route(n_cols, cout), kernel
     H.assert_bit_exact(ig.download(), ig.host, "convolution-backward-data")
     unrolled("unrolled gradient")
+
+
+@pytest.mark.parametrize("shift", [0, 5])
+def test_forward_over_its_own_input(P, shift):
+    """An output that is the input, or shares some of it: the input is unrolled whole before any of the output is stored
+    (over 9 cells the product would otherwise be the kernel's that gathers the input as it goes)."""
+    batch, c, side, k = 1, 1, 40, 3
+    n = c * side * side
+    desc, geometry = H.conv_desc(c, c, k, k, 1, 1, 1, 1), (1, side, side, side, side)
+    rng = np.random.default_rng(4 + shift)
+    ints = lambda m: rng.integers(-4, 5, m).astype(np.float32)
+    both, weights, work = P.buf(ints(n + shift)), P.buf(ints(c * k * k)), P.buf(ints(n * k * k))
+    inp, out = View(both, [n]), View(both, [n], offset=shift)
+    kernel = P.run(H.convolution, "forward", out, 2.0, inp, vec(weights), vec(work), desc, *geometry)
+    assert kernel == "conv_unroll+gemm", kernel
+    H.assert_bit_exact(both.download(), both.host, "convolution-forward")
