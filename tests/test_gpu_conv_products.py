@@ -117,3 +117,53 @@ def test_forward_over_its_own_input(P, shift):
     kernel = P.run(H.convolution, "forward", out, 2.0, inp, vec(weights), vec(work), desc, *geometry)
     assert kernel == "conv_unroll+gemm", kernel
     H.assert_bit_exact(both.download(), both.host, "convolution-forward")
+
+
+def rounding_error(a, b, chain):
+    """The 2-norm of the error of a @ b against 64 bits, and that of the same product summed in float, rounded after every
+    product, in chains of so many products that are added up one after the other."""
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    exact = a64 @ b64
+    total = np.zeros(exact.shape, np.float32)
+    for k0 in range(0, a.shape[1], chain):
+        acc = np.zeros(exact.shape, np.float32)
+        for k in range(k0, min(k0 + chain, a.shape[1])):
+            acc = (acc.astype(np.float64) + a64[:, k, None] * b64[k]).astype(np.float32)
+        total = (total + acc).astype(np.float32)
+    return exact, np.linalg.norm(total - exact)
+
+
+# (batch, in channels, out channels, side): sums over 54, 144 and 45 cells; 40, 112 and 150 out channels; 64, 225 and 441
+# positions of an image
+@pytest.mark.parametrize("case", [(4, 6, 40, 8), (2, 16, 112, 15), (1, 5, 150, 21)], ids=lambda c: "x".join(map(str, c)))
+def test_products_round_as_short_chains_do(P, case):
+    """The error of a product is that of a sum in short chains, whatever the number of its terms: chains of 16 products
+    (32 for the weight gradient) leave at least as large an error.  The 2-norms are over a thousand sums or more, whose own
+    spread is then below 5 %."""
+    batch, cin, cout, side = case
+    n_rows, n_cols = side * side, cin * 9
+    desc, geometry = H.conv_desc(cin, cout, 3, 3, 1, 1, 1, 1), (batch, side, side, side, side)
+    rng = np.random.default_rng(side)
+    normal = lambda n: rng.standard_normal(n).astype(np.float32)
+    inp, weights, og = P.buf(normal(batch * cin * n_rows)), P.buf(normal(cout * n_cols)), P.buf(normal(batch * cout * n_rows))
+    out, wg, ig = P.buf(normal(batch * cout * n_rows)), P.buf(normal(cout * n_cols)), P.buf(normal(batch * cin * n_rows))
+    work = P.buf(np.zeros(batch * n_rows * n_cols, np.float32))
+    w = weights.init.reshape(cout, n_cols)
+    across = lambda buf, rows: np.concatenate(list(buf.reshape(batch, rows, n_rows)), axis=1)
+
+    kernel = P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    assert kernel == "conv_product", kernel
+    unrolled = across(work.download(), n_cols)
+    exact, bound = rounding_error(w, unrolled, 16)
+    assert np.linalg.norm(across(out.download(), cout) - exact) <= 1.05 * bound, "convolution-forward"
+
+    kernel = P.run(H.convolution, "backward_weights", vec(wg), 0.0, vec(og), vec(inp), vec(work), desc, *geometry)
+    assert kernel == "conv_weight_gradient+conv_sum_partials", kernel
+    gradient = across(og.init, cout)
+    exact, bound = rounding_error(gradient, np.ascontiguousarray(unrolled.T), 32)
+    assert np.linalg.norm(wg.download().reshape(cout, n_cols) - exact) <= 1.05 * bound, "convolution-backward-weights"
+
+    kernel = P.run(H.convolution, "backward_data", vec(ig), 0.0, vec(og), vec(weights), vec(work), desc, *geometry)
+    assert kernel == "conv_product+conv_roll", kernel
+    exact, bound = rounding_error(np.ascontiguousarray(w.T), gradient, 16)
+    assert np.linalg.norm(across(work.download(), n_cols) - exact) <= 1.05 * bound, "unrolled gradient"
