@@ -432,8 +432,11 @@ int forward_t(void* stream, T* output, double output_alpha, const T* input, cons
 // Few elements and many partials (a digit network: 4608 elements, 128 images) leave one lane
 // per element with 18 blocks and a serial chain of 128 loads, each the latency of memory.
 // SLICES lanes share an element instead, every slice taking each SLICES-th partial, and the
-// slices are added in order through LDS: [128, 4608] float 30.9 -> 4.1 us, [64, 36864]
-// 24.3 -> 4.9 us.  A handful of partials stays with one lane per element.
+// slices are added in order through LDS: [128, 4608] float 11.8 -> 4.7 us, [64, 36864]
+// 8.3 -> 4.7 us.  A handful of partials stays with one lane per element, and so do elements
+// enough to fill the chip by themselves, a lane each: slices there make for short blocks that
+// wait for one another ([34, 79500] 5.0 us with slices, 5.5 without; [38, 205375] 9.8 and 7.4;
+// [8, 1638400] 19.5 and 10.3).
 template <class T, int SLICES>
 __global__ void __launch_bounds__(kBlock) conv_sum_partials_kernel(T* weight_gradient, const T* partials, uint32_t n,
                                                                     uint32_t count, double alpha) {
@@ -459,7 +462,9 @@ __global__ void __launch_bounds__(kBlock) conv_sum_partials_kernel(T* weight_gra
 template <class T>
 void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t n, int64_t count, double alpha) {
   constexpr int kSlices = 8;
-  if (count >= kSlices)
+  constexpr int64_t kFullChip = 384 * kBlock;
+  static_assert(kFullChip * kSlices < (int64_t(1) << 31), "a launch of 2^32 lanes or more is refused");
+  if (count >= kSlices && n < kFullChip)
     hipLaunchKernelGGL((conv_sum_partials_kernel<T, kSlices>),
                        dim3((uint32_t)((n + kBlock / kSlices - 1) / (kBlock / kSlices))), dim3(kBlock), 0, s,
                        weight_gradient, partials, (uint32_t)n, (uint32_t)count, alpha);

@@ -167,3 +167,20 @@ def test_products_round_as_short_chains_do(P, case):
     assert kernel == "conv_product+conv_roll", kernel
     exact, bound = rounding_error(np.ascontiguousarray(w.T), gradient, 16)
     assert np.linalg.norm(across(work.download(), n_cols) - exact) <= 1.05 * bound, "unrolled gradient"
+
+
+@pytest.mark.parametrize("code", [capi.F32, capi.F64], ids=["float", "double"])
+@pytest.mark.parametrize("cout", [95, 96, 97])      # 97280, 98304 and 99328 weights: the sum shares elements below 98304
+def test_weight_gradient_sum_over_many_weights(P, code, cout):
+    """Whole numbers: exact in any order."""
+    batch, cin, side = 9, 1024, 3
+    desc, geometry = H.conv_desc(cin, cout, 1, 1, 0, 0, 1, 1), (batch, side, side, side, side)
+    rng = np.random.default_rng(cout)
+    ints = lambda n: rng.integers(-4, 5, n).astype(NP[code])
+    n_rows = side * side
+    inp, weights, og = P.buf(ints(batch * cin * n_rows)), P.buf(ints(cout * cin)), P.buf(ints(batch * cout * n_rows))
+    out, work, wg = P.buf(ints(batch * cout * n_rows)), P.buf(ints(batch * n_rows * cin)), P.buf(ints(cout * cin))
+    P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    for alpha in (0.0, 2.0):
+        P.run(H.convolution, "backward_weights", vec(wg), alpha, vec(og), vec(inp), vec(work), desc, *geometry)
+        H.assert_bit_exact(wg.download(), wg.host, f"convolution-backward-weights, alpha {alpha}")
