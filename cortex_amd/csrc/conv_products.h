@@ -29,18 +29,24 @@ void conv_product(hipStream_t s, ConvProductArgs a, bool forward);
 // The tiles that such a product has.
 int64_t conv_product_units(int64_t m, int64_t n);
 
-// partials[split][m][n] = sum over the split's positions of output_gradient[m][p] * unrolled[n][p]
+// The positions of a piece, the unit in which the weight gradient's sum is split.
+constexpr int kConvPiece = 64;
+
+// result[split][m][n] = alpha * result[split][m][n] + sum over the split's positions of
+//                       output_gradient[m][p] * unrolled[n][p]
 struct ConvWeightArgs {
   const float* output_gradient;
   const float* workspace;
-  float* partials;
+  float* result;                       // the weight gradient of a single split, else partial sums
+  double alpha;
   int64_t out_image, conv_image;
   uint32_t m, n, n_rows;
-  uint32_t piece_len, pieces, pieces_per_split;   // positions of a piece; pieces of all images; of a split
+  uint32_t pieces, pieces_per_split;   // of all images; of a split
   uint32_t units;
-  FastDiv parts_fd, tiles_fd, n_tiles_fd;          // parts: pieces of one image
+  FastDiv parts_fd, tiles_fd, n_tiles_fd;   // parts: pieces of one image
 };
 void conv_weight_gradient(hipStream_t s, ConvWeightArgs a, int64_t splits);
 int64_t conv_weight_tiles(int64_t m, int64_t n);   // blocks to a split
+int64_t conv_weight_waves(int64_t m, int64_t n);   // waves to a block
 
 }  // namespace cthip

@@ -473,36 +473,51 @@ void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t 
                        s, weight_gradient, partials, (uint32_t)n, (uint32_t)count, alpha);
 }
 
-// The splits of the matrix-core weight gradient: at most kWeightBlocks blocks in all, two to a
-// compute unit and none left over (64 splits of 9 tiles, 2.25 blocks to a unit, took 215 us where
-// 56 take 180), every split a run of pieces of at most kPieceLength positions.  The partials stay within what the library's
-// products take (a matrix an image, at most 256 MiB) or the megabyte that every scratch block has.
-ConvWeightArgs weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t* splits) {
-  constexpr int64_t kWeightBlocks = 512, kPieceLength = 512;
+// The splits of the matrix-core weight gradient, and whether it is taken at all.  `fit` partial
+// products may be kept.
+//
+// The positions of an image are cut into pieces of 64, a split takes a run of pieces: as many splits
+// as give two blocks to a compute unit, but no more than pieces or `fit`.  Up to three pieces stay
+// together (a piece takes a block 1.2 us, a second launch for the sum 2).  Pieces of up to 512
+// positions left the chip idle: [3, 15, 109, 109] under 84 windows of 3 x 3 58 -> 48 us,
+// [3, 5, 60, 60] under 7 15.6 -> 9.2, [134, 94, 15, 15] under 145 164 -> 139.
+//
+// The library is the faster one (its time, sum included, is the second)
+//  - over results of more than 64 tiles of 64 x 64 and images of more than two pieces, for its
+//    larger tiles load less for a product: [8, 512, 28, 28] under 512 of 3 x 3 425 and 275 us,
+//    [2, 256, 28, 28] under 256 47 and 32, [32, 256, 14, 14] under 256 134 and 94; but
+//    [32, 128, 14, 14] under 256 at stride 2 (49 positions an image) 30 and 84.  A single piece
+//    stays here: it needs no sum;
+//  - where the blocks are too few to fill the chip, their runs long, and the images of more than 400
+//    positions (the library's products are slow over fewer).  A block takes 1.4 to 1.7 us for a
+//    piece, the library 7 to 10 ns for a position of an image: [16, 64, 56, 56] under 256 of 1 x 1
+//    (64 blocks of 49 pieces) 83 and 28 us, [16, 64, 28, 28] under 64 of 3 x 3 (144 of 13) 30 and
+//    27; but [1, 64, 56, 56] under 64 (63 of 7) 19 and 24, [3, 15, 109, 109] under 84 (138 of 25)
+//    48 and 96.  Results of up to 32 rows or columns, whose blocks have half the waves, fill
+//    it for images of up to 2048 positions only: [71, 42, 77, 77] under 11 185 and 137 us,
+//    [40, 63, 60, 60] under 4 of 5 x 5 185 and 144; [34, 89, 37, 37] under 5 83 and 121.
+// Rows shorter than a 16-byte load are the library's too.
+bool weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t fit, ConvWeightArgs* args, int64_t* splits) {
+  constexpr int64_t kWeightBlocks = 512, kTogether = 3, kManyTiles = 64, kFewWaves = 1400, kPositionsPerPiece = 200,
+                    kShortImage = 400, kNarrowImage = 2048;
   ConvWeightArgs a{};
   a.out_image = sh.out_image; a.conv_image = sh.conv_image;
   a.m = (uint32_t)d.out_channels; a.n = (uint32_t)sh.n_cols; a.n_rows = (uint32_t)sh.n_rows;
-  const int64_t parts = (sh.n_rows + kPieceLength - 1) / kPieceLength;
-  a.piece_len = (uint32_t)(((sh.n_rows + parts - 1) / parts + 63) / 64 * 64);
-  const int64_t used_parts = (sh.n_rows + a.piece_len - 1) / a.piece_len;
-  a.pieces = (uint32_t)(sh.batch * used_parts);
-  a.parts_fd = FastDiv((uint32_t)used_parts);
-  const int64_t result = (int64_t)a.m * a.n * (int64_t)sizeof(float);
+  const int64_t parts = (sh.n_rows + kConvPiece - 1) / kConvPiece, pieces = sh.batch * parts;
+  a.pieces = (uint32_t)pieces;
+  a.parts_fd = FastDiv((uint32_t)parts);
   const int64_t tiles = conv_weight_tiles(a.m, a.n);
-  const int64_t fit = std::max<int64_t>(std::min<int64_t>(sh.batch * result, int64_t(256) << 20), int64_t(1) << 20) / result;
-  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({kWeightBlocks / tiles, fit, (int64_t)a.pieces}));
-  a.pieces_per_split = (uint32_t)((a.pieces + want - 1) / want);
-  *splits = (a.pieces + a.pieces_per_split - 1) / a.pieces_per_split;
-  return a;
-}
-
-// Images of a few hundred positions that fall badly into tiles of 64 leave a large product to the
-// library: [32, 256, 14, 14] under 256 windows of 3 x 3 (196 positions in four tiles) 127 us
-// here, 98 there.  Rows shorter than a 16-byte load are the library's too.
-bool matrix_core_weight_gradient(int64_t result, const ConvShape& sh) {
-  constexpr double kLarge = 2e9;
-  const bool ragged = (sh.n_rows + 63) / 64 * 64 * 5 > sh.n_rows * 6;
-  return sh.n_rows >= 4 && !(ragged && 2.0 * (double)result * (double)(sh.batch * sh.n_rows) > kLarge);
+  const int64_t want =
+      pieces <= kTogether ? 1 : std::max<int64_t>(1, std::min<int64_t>({kWeightBlocks / tiles, fit, pieces}));
+  const int64_t run = (pieces + want - 1) / want;
+  a.pieces_per_split = (uint32_t)run;
+  *splits = (pieces + run - 1) / run;
+  *args = a;
+  if (sh.n_rows < 4) return false;
+  const bool narrow = a.m <= 32 || a.n <= 32;
+  if (sh.n_rows > 2 * kConvPiece && run > 1 && (narrow ? tiles / 2 : tiles) > kManyTiles) return false;
+  const bool full = tiles * *splits * conv_weight_waves(a.m, a.n) >= kFewWaves && !(narrow && sh.n_rows > kNarrowImage);
+  return full || sh.n_rows <= kShortImage || run <= std::max<int64_t>(2, sh.n_rows / kPositionsPerPiece);
 }
 
 template <class T>
@@ -511,20 +526,7 @@ int backward_weights_t(void* stream, T* weight_gradient, double alpha, const T* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t n = (int64_t)d.out_channels * sh.n_cols;
   CT_REQUIRE(n <= (int64_t(1) << 31) - 1, "convolution: the weight matrix exceeds the supported range");
-  if (std::is_same<T, float>::value && matrix_core_weight_gradient(n, sh)) {
-    int64_t splits;
-    ConvWeightArgs a = weight_args(d, sh, &splits);
-    void* scratch = nullptr;
-    if (int rc = stream_scratch(s, (size_t)(splits * n) * sizeof(float), &scratch)) return rc;
-    a.output_gradient = reinterpret_cast<const float*>(output_gradient);
-    a.workspace = reinterpret_cast<const float*>(workspace);
-    a.partials = reinterpret_cast<float*>(scratch);
-    conv_weight_gradient(s, a, splits);
-    sum_partials(s, reinterpret_cast<float*>(weight_gradient), a.partials, n, splits, (double)(float)alpha);
-    note_kernel("conv_weight_gradient+conv_sum_partials");
-    return after_launch(s);
-  }
-  // A product of few outputs over very many positions (a first layer: 64 x 27 outputs, 50176
+  // The library: a product of few outputs over very many positions (a first layer: 64 x 27 outputs, 50176
   // positions) would occupy one workgroup per image: the positions are cut into pieces of about
   // kPositionsPerPiece, every piece a product of its own, and the sum takes the pieces too.
   constexpr int64_t kPositionsPerPiece = 4096;
@@ -533,6 +535,31 @@ int backward_weights_t(void* stream, T* weight_gradient, double alpha, const T* 
   // images per pass: partial products of at most 256 MiB
   const int64_t per_pass =
       std::max<int64_t>(1, std::min<int64_t>(sh.batch, (int64_t(256) << 20) / (pieces * n * (int64_t)sizeof(T))));
+  if constexpr (std::is_same<T, float>::value) {
+    // scratch: never more than the library's partial products take, or the megabyte that every block has
+    const int64_t fit = std::max<int64_t>(per_pass * pieces, (int64_t(1) << 20) / (n * (int64_t)sizeof(T)));
+    ConvWeightArgs a;
+    int64_t splits;
+    if (weight_args(d, sh, fit, &a, &splits)) {
+      a.output_gradient = output_gradient;
+      a.workspace = workspace;
+      a.result = weight_gradient;
+      a.alpha = (double)(float)alpha;
+      // a single split stores the gradient itself, unless other blocks may still read those bytes
+      const bool partials = splits > 1 || overlap(weight_gradient, n, output_gradient, sh.batch * sh.out_image) ||
+                            overlap(weight_gradient, n, workspace, sh.batch * sh.conv_image);
+      if (partials) {
+        void* scratch = nullptr;
+        if (int rc = stream_scratch(s, (size_t)(splits * n) * sizeof(T), &scratch)) return rc;
+        a.result = static_cast<float*>(scratch);
+        a.alpha = 0.0;
+      }
+      conv_weight_gradient(s, a, splits);
+      if (partials) sum_partials(s, weight_gradient, a.result, n, splits, (double)(float)alpha);
+      note_kernel(partials ? "conv_weight_gradient+conv_sum_partials" : "conv_weight_gradient");
+      return after_launch(s);
+    }
+  }
   void* scratch = nullptr;
   if (int rc = stream_scratch(s, (size_t)(per_pass * pieces * n) * sizeof(T), &scratch)) return rc;
   const T al = (T)alpha;

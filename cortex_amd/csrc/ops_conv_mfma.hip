@@ -47,8 +47,8 @@ __device__ __forceinline__ f32x4 load4(const float* row, uint32_t i, uint32_t n)
   __builtin_memcpy(&v, row + min(i, n - 4), 16);
   return v;
 }
-// What load4 loaded, with zeros from element `end` <= n of the row on.
-__device__ __forceinline__ f32x4 fix4(f32x4 v, uint32_t i, uint32_t n, uint32_t end) {
+// What load4 loaded, with zeros beyond the row's end.
+__device__ __forceinline__ f32x4 fix4(f32x4 v, uint32_t i, uint32_t n) {
   const uint32_t shift = i - min(i, n - 4);
   f32x4 out;
 #pragma unroll
@@ -56,7 +56,7 @@ __device__ __forceinline__ f32x4 fix4(f32x4 v, uint32_t i, uint32_t n, uint32_t 
     float x = v[e];
 #pragma unroll
     for (uint32_t d = 1; d + e < 4; ++d) x = shift == d ? v[e + d] : x;
-    out[e] = i + e < end ? x : 0.f;
+    out[e] = i + e < n ? x : 0.f;
   }
   return out;
 }
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProdu
       for (int i = 0; i < kLeft; ++i) {
         const uint32_t piece = min(i * kBlock + tid, (uint32_t)(BM * BK / 4 - 1));
         if constexpr (kForward) {
-          left_regs[i] = fix4(left_regs[i], k0 + piece % (BK / 4) * 4, a.k, a.k);
+          left_regs[i] = fix4(left_regs[i], k0 + piece % (BK / 4) * 4, a.k);
         } else {
 #pragma unroll
           for (uint32_t e = 0; e < 4; ++e) left_regs[i][e] = k0 + piece / BM * 4 + e < a.k ? left_regs[i][e] : 0.f;
@@ -300,14 +300,15 @@ __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProdu
 // ------------------------------------------------------------------------ backward-weights
 
 // partial[split][m][n] = sum over the split's positions of output_gradient[m][p] * unrolled[n][p]:
-// both operands have the positions innermost.  The positions of all images are cut into pieces
-// of at most a.piece_len, a split takes a run of consecutive pieces: the result is small (64 x
-// 576 is 9 tiles), the chip is filled by the splits.
+// both operands have the positions innermost.  The positions of every image are cut into pieces
+// of kConvPiece (the last one shorter), a split takes a run of consecutive pieces: the result is
+// small (64 x 576 is 9 tiles), the chip is filled by the splits.  A single split adds to the
+// weight gradient itself.
 // Two groups of WM x WN waves share a tile of positions and take half of it each: twice the
 // waves in flight for the same partials, which are added in LDS at the end.
 template <int WM, int WN>
 __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(const ConvWeightArgs a) {
-  constexpr int BM = 32 * WM, BN = 32 * WN, BK = 64, LD = BK + 4, THREADS = 128 * WM * WN;
+  constexpr int BM = 32 * WM, BN = 32 * WN, BK = kConvPiece, LD = BK + 4, THREADS = 128 * WM * WN;
   constexpr int kLeft = BM * BK / 4 / THREADS, kRight = BN * BK / 4 / THREADS;
   __shared__ __attribute__((aligned(16))) float left_lds[2][BM * LD];
   __shared__ __attribute__((aligned(16))) float right_lds[2][BN * LD];
@@ -321,18 +322,13 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
   const uint32_t first_piece = split * a.pieces_per_split;
   const uint32_t piece_end = min(first_piece + a.pieces_per_split, a.pieces);
 
-  // The tile that is loaded: positions [p0, p0 + BK) of a piece that ends at p_end of its image.
+  // The piece that is loaded: positions [p0, p0 + BK) of an image, as far as it has them.
   // Rows beyond the result repeat the last one and are not stored.
-  uint32_t piece = first_piece, p0 = 0, p_end = 0;
-  const float *left = nullptr, *right = nullptr;
-  auto enter_piece = [&] {
-    uint32_t image, part;
-    a.parts_fd.divmod(piece, image, part);
-    p0 = part * a.piece_len;
-    p_end = min(p0 + a.piece_len, a.n_rows);
-    left = a.output_gradient + (int64_t)image * a.out_image;
-    right = a.workspace + (int64_t)image * a.conv_image;
-  };
+  uint32_t piece = first_piece, image, part;
+  a.parts_fd.divmod(piece, image, part);
+  uint32_t p0 = part * BK;
+  const float* left = a.output_gradient + (int64_t)image * a.out_image;
+  const float* right = a.workspace + (int64_t)image * a.conv_image;
   f32x4 left_regs[kLeft], right_regs[kRight];
   auto load_tile = [&] {
 #pragma unroll
@@ -347,14 +343,14 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
     }
   };
   auto store_tile = [&](int buffer) {
-    if (p0 + BK > p_end) {
+    if (p0 + BK > a.n_rows) {
       asm volatile("");   // stays a branch: as selects it would cost every tile
 #pragma unroll
       for (int i = 0; i < kLeft; ++i)
-        left_regs[i] = fix4(left_regs[i], p0 + (i * THREADS + tid) % (BK / 4) * 4, a.n_rows, p_end);
+        left_regs[i] = fix4(left_regs[i], p0 + (i * THREADS + tid) % (BK / 4) * 4, a.n_rows);
 #pragma unroll
       for (int i = 0; i < kRight; ++i)
-        right_regs[i] = fix4(right_regs[i], p0 + (i * THREADS + tid) % (BK / 4) * 4, a.n_rows, p_end);
+        right_regs[i] = fix4(right_regs[i], p0 + (i * THREADS + tid) % (BK / 4) * 4, a.n_rows);
     }
 #pragma unroll
     for (int i = 0; i < kLeft; ++i) {
@@ -372,7 +368,6 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
   const uint32_t k_half = wave / (WM * WN) * (BK / 2);
   const uint32_t wave_m = wave / WN % WM * 32, wave_n = wave % WN * 32;
   double total[2][2][4] = {};
-  enter_piece();
   load_tile();
   store_tile(0);
   __syncthreads();
@@ -411,14 +406,14 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
       keep_order();
     }
   };
-  for (bool more = true; more;) {
-    if (p0 + BK < p_end) {
+  for (; piece < piece_end; ++piece) {
+    if (piece + 1 < piece_end) {   // else the last piece is loaded again, and not used: no load stands under a condition
       p0 += BK;
-    } else if (piece + 1 < piece_end) {
-      ++piece;
-      enter_piece();
-    } else {
-      more = false;   // the split's last tile is loaded again, and not used: no load stands under a condition
+      if (p0 >= a.n_rows) {
+        p0 = 0;
+        left += a.out_image;
+        right += a.conv_image;
+      }
     }
     load_tile();
     multiply();
@@ -446,7 +441,7 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) total[t][u][r] += shared[(t * 2 + u) * 4 + r];
 
-  float* to = a.partials + (int64_t)split * a.m * a.n;
+  float* to = a.result + (int64_t)split * a.m * a.n;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const uint32_t n = n_tile * BN + wave_n + u * 16 + row;
@@ -456,7 +451,9 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const uint32_t m = m_tile * BM + wave_m + t * 16 + 4 * group + r;
-        if (m < a.m) to[(int64_t)m * a.n + n] = (float)total[t][u][r];
+        if (m >= a.m) continue;
+        float& cell = to[(int64_t)m * a.n + n];
+        cell = (float)(a.alpha == 0.0 ? total[t][u][r] : a.alpha * (double)cell + total[t][u][r]);
       }
   }
 }
@@ -492,6 +489,8 @@ void conv_product(hipStream_t s, ConvProductArgs a, bool forward) {
 int64_t conv_weight_tiles(int64_t m, int64_t n) {
   return (m <= 32 ? 1 : (m + 63) / 64) * (n <= 32 ? 1 : (n + 63) / 64);
 }
+
+int64_t conv_weight_waves(int64_t m, int64_t n) { return (m <= 32 ? 1 : 2) * (n <= 32 ? 1 : 2) * 2; }
 
 void conv_weight_gradient(hipStream_t s, ConvWeightArgs a, int64_t splits) {
   const bool narrow_m = a.m <= 32, narrow_n = a.n <= 32;

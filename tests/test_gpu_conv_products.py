@@ -62,7 +62,42 @@ PRODUCT_CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", PRODUCT_CASES, ids=lambda c: "x".join(map(str, c)))
+def weight_route(batch, m, n, n_rows):
+    """The kernels of the weight gradient of [m, n] over n_rows positions an image."""
+    pieces, products = batch * -(-n_rows // 64), max(1, min(64, n_rows // 4096))
+    fit = max(batch * products, (1 << 20) // (4 * m * n))
+    tiles = (1 if m <= 32 else -(-m // 64)) * (1 if n <= 32 else -(-n // 64))
+    want = 1 if pieces <= 3 else max(1, min(512 // tiles, fit, pieces))
+    run = -(-pieces // want)
+    splits = -(-pieces // run)
+    waves = tiles * splits * 2 * (1 if m <= 32 else 2) * (1 if n <= 32 else 2)
+    narrow = m <= 32 or n <= 32
+    if n_rows < 4 or (n_rows > 128 and run > 1 and tiles // (2 if narrow else 1) > 64):
+        return "gemm+conv_sum_partials"
+    if n_rows > 400 and (waves < 1400 or narrow and n_rows > 2048) and run > max(2, n_rows // 200):
+        return "gemm+conv_sum_partials"
+    return "conv_weight_gradient" + ("+conv_sum_partials" if splits > 1 else "")
+
+
+# The same for the weight gradient's routes and splits
+WEIGHT_CASES = [
+    (2, 128, 250, 9, 8, 3, 3, 1, 1),    # 72 tiles, two splits of two pieces, 72 positions
+    (2, 128, 250, 9, 15, 3, 3, 1, 1),   # 72 tiles, two splits of three pieces, 135 positions: the library
+    (1, 128, 250, 7, 7, 3, 3, 1, 1),    # 72 tiles, one piece
+    (1, 406, 520, 5, 5, 3, 3, 1, 1),    # 522 tiles, one piece
+    (3, 2, 5, 8, 8, 3, 3, 1, 1),        # three pieces: one split
+    (4, 2, 5, 8, 8, 3, 3, 1, 1),        # four of them: four splits
+    (1, 20, 64, 13, 13, 3, 3, 1, 1),    # three pieces of one image, the last one of 41 positions
+    (3, 64, 64, 40, 40, 3, 3, 1, 1),    # seven splits of eleven pieces: the library
+    (2, 60, 3, 48, 48, 3, 3, 1, 1),     # 36 splits of two pieces of images of 2304 positions, few rows
+    (5, 200, 3, 48, 48, 3, 3, 1, 1),    # the same with fourteen: the library
+    (1, 64, 64, 56, 56, 3, 3, 1, 1),    # seven splits of seven pieces of one image
+    (6, 200, 128, 11, 9, 1, 1, 0, 1),   # six splits of two pieces, an image each
+    (7, 160, 128, 11, 9, 3, 3, 1, 1),   # seven partial products of 46 tiles
+]
+
+
+@pytest.mark.parametrize("case", PRODUCT_CASES + WEIGHT_CASES, ids=lambda c: "x".join(map(str, c)))
 def test_products_at_the_edges_of_their_tiles(P, case):
     """Whole numbers whose sums stay below 2^24: exact in any order, so everything agrees to the bit."""
     batch, cin, cout, h, w, kw, kh, pad, stride = case
@@ -95,7 +130,7 @@ def test_products_at_the_edges_of_their_tiles(P, case):
         unrolled("unrolled input")
     for alpha in (0.0, 2.0):
         kernel = P.run(H.convolution, "backward_weights", vec(wg), alpha, vec(og), vec(inp), vec(work), *geometry)
-        assert (kernel == "conv_weight_gradient+conv_sum_partials") == (n_rows >= 4), kernel
+        assert kernel == weight_route(batch, cout, n_cols, n_rows), kernel
         H.assert_bit_exact(wg.download(), wg.host, f"convolution-backward-weights, alpha {alpha}")
     kernel = P.run(H.convolution, "backward_data", vec(ig), 0.0, vec(og), vec(weights), vec(work), *geometry)
     assert (kernel == "conv_product+conv_roll") == route(n_cols, cout), kernel
@@ -158,7 +193,7 @@ def test_products_round_as_short_chains_do(P, case):
     assert np.linalg.norm(across(out.download(), cout) - exact) <= 1.05 * bound, "convolution-forward"
 
     kernel = P.run(H.convolution, "backward_weights", vec(wg), 0.0, vec(og), vec(inp), vec(work), desc, *geometry)
-    assert kernel == "conv_weight_gradient+conv_sum_partials", kernel
+    assert kernel.startswith("conv_weight_gradient"), kernel
     gradient = across(og.init, cout)
     exact, bound = rounding_error(gradient, np.ascontiguousarray(unrolled.T), 32)
     assert np.linalg.norm(wg.download().reshape(cout, n_cols) - exact) <= 1.05 * bound, "convolution-backward-weights"
@@ -184,3 +219,22 @@ def test_weight_gradient_sum_over_many_weights(P, code, cout):
     for alpha in (0.0, 2.0):
         P.run(H.convolution, "backward_weights", vec(wg), alpha, vec(og), vec(inp), vec(work), desc, *geometry)
         H.assert_bit_exact(wg.download(), wg.host, f"convolution-backward-weights, alpha {alpha}")
+
+
+def test_weight_gradient_over_its_own_operand(P):
+    """A weight gradient stored over the output gradient that it is formed from: one split, which otherwise stores its
+    result as soon as a block has it, here goes through scratch memory."""
+    cin, cout, side = 40, 100, 8
+    n_cols, n_rows = cin * 9, side * side
+    desc, geometry = H.conv_desc(cin, cout, 3, 3, 1, 1, 1, 1), (1, side, side, side, side)
+    rng = np.random.default_rng(5)
+    ints = lambda n: rng.integers(-4, 5, n).astype(np.float32)
+    both, inp, work = P.buf(ints(cout * n_cols)), P.buf(ints(cin * n_rows)), P.buf(ints(n_rows * n_cols))
+    out, weights = P.buf(ints(cout * n_rows)), P.buf(ints(cout * n_cols))
+    P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    og = View(both, [cout * n_rows])
+    kernel = P.run(H.convolution, "backward_weights", vec(both), 0.0, og, vec(inp), vec(work), desc, *geometry)
+    assert kernel == "conv_weight_gradient+conv_sum_partials", kernel
+    gradient = both.init[:cout * n_rows].reshape(cout, n_rows).astype(np.float64)
+    unrolled = work.download().reshape(n_cols, n_rows).astype(np.float64)
+    H.assert_bit_exact(both.download(), (gradient @ unrolled.T).astype(np.float32).reshape(-1), "convolution-backward-weights")
