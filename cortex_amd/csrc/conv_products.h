@@ -26,8 +26,9 @@ struct ConvProductArgs {
   FastDiv m_tiles_fd, rows_fd, out_w_fd, taps_fd, kw_fd;
 };
 void conv_product(hipStream_t s, ConvProductArgs a, bool forward);
-// The tiles that such a product has.
+// The tiles that such a product has, and the positions that one launch of it may have.
 int64_t conv_product_units(int64_t m, int64_t n);
+int64_t conv_product_positions(int64_t m);
 
 // The positions of a piece, the unit in which the weight gradient's sum is split.
 constexpr int kConvPiece = 64;

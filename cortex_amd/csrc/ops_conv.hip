@@ -365,7 +365,7 @@ void roll_back(hipStream_t s, const T* workspace, T* input_gradient, const ct_co
 // 106 of 5 x 5 (k 750, 1493 tiles) 250 and 347.
 bool matrix_core_product(const ct_conv_desc& d, const ConvShape& sh, int64_t m, int64_t k) {
   constexpr int64_t kFullChip = 768, kShortChain = 192;
-  return sh.in_image > 0 && d.kernel_width * d.kernel_height <= kConvMaskTaps &&
+  return sh.in_image > 0 && d.kernel_width * d.kernel_height <= kConvMaskTaps && sh.n_rows <= conv_product_positions(m) &&
          (k <= kShortChain || conv_product_units(m, sh.batch * sh.n_rows) >= kFullChip);
 }
 
@@ -386,8 +386,7 @@ void run_product(hipStream_t s, float* output, float beta, const float* input, c
   a.out_w_fd = FastDiv((uint32_t)sh.out_w);
   a.taps_fd = FastDiv((uint32_t)(d.kernel_width * d.kernel_height));
   a.kw_fd = FastDiv((uint32_t)d.kernel_width);
-  // the positions and the tiles of a launch are counted in 31 bits
-  const int64_t step = images_per_launch(sh.n_rows * (a.m / 4096 + 1));
+  const int64_t step = std::max<int64_t>(1, conv_product_positions(a.m) / sh.n_rows);
   for (int64_t b0 = 0; b0 < sh.batch; b0 += step) {
     const int64_t nb = std::min(step, sh.batch - b0);
     a.input = forward ? input + b0 * sh.in_image : nullptr;

@@ -477,6 +477,13 @@ int64_t conv_product_units(int64_t m, int64_t n) {
   return (m + bm - 1) / bm * ((n + bn - 1) / bn);
 }
 
+int64_t conv_product_positions(int64_t m) {
+  constexpr int64_t kMostTiles = int64_t(1) << 23;
+  static_assert(kMostTiles * kBlock < int64_t(1) << 32, "a launch of 2^32 lanes or more is refused");
+  const int bm = tile_rows(m);
+  return kMostTiles / ((m + bm - 1) / bm) * (bm == 128 ? 64 : 128);
+}
+
 void conv_product(hipStream_t s, ConvProductArgs a, bool forward) {
   const int bm = tile_rows(a.m);
   a.units = (uint32_t)conv_product_units(a.m, a.n);
