@@ -369,6 +369,29 @@ bool matrix_core_product(const ct_conv_desc& d, const ConvShape& sh, int64_t m, 
          (k <= kShortChain || conv_product_units(m, sh.batch * sh.n_rows) >= kFullChip);
 }
 
+// Backward-data, of m cells over k out channels: the library needs one launch here too, and its times
+// depend on more than the sizes (20 to 110 TFLOP/s for products of one size).  The lines below are
+// drawn through 310 shapes; its time is the second.
+//  - Few tiles: k up to 112 ([9, 10, 15, 15] under 102 of 3 x 3 10.0 and 7.2 us, calls 13.7 and
+//    16.1; k 128, [1, 128, 28, 28], 12.4 and 6.9, calls 16.9 and 15.4).
+//  - k up to 64: results of up to 2 M cells, where the host decides; images of more than 3500
+//    positions ([69, 6, 71, 71] under 38 34 and 130, [3, 64, 112, 112] under 64 41 and 56); and from
+//    1750 tiles on ([64, 64, 56, 56] under 64 212 and 236; below, [16, 64, 28, 28] under 64, 882
+//    tiles, 22 and 17).
+//  - k above: from 768 tiles on ([38, 53, 21, 21] under 155 of 5 x 5 90 and 196), 400 for up to 96
+//    cells ([60, 9, 28, 28] under 181 32 and 67), 250 for images of up to 128 positions
+//    ([32, 256, 7, 7] under 256 32 and 55).  But not k up to 256 over 192 cells or more in images of
+//    500 to 4096 positions, where the library runs at 80 to 110 TFLOP/s: [64, 128, 28, 28] under 128
+//    177 and 147, [98, 26, 46, 46] under 164 209 and 175.  (Beyond 256 it is either way, 0.7 to 1.6.)
+bool backward_data_product(const ct_conv_desc& d, const ConvShape& sh) {
+  const int64_t m = sh.n_cols, k = d.out_channels, n_rows = sh.n_rows, tiles = conv_product_units(m, sh.batch * n_rows);
+  if (sh.conv_image == 0 || n_rows > conv_product_positions(m)) return false;
+  if (k <= 112 && tiles < 128) return true;
+  if (k <= 64) return m * sh.batch * n_rows <= (int64_t(1) << 21) || n_rows > 3500 || tiles >= 1750 || (n_rows <= 128 && tiles >= 250);
+  if (k <= 256 && m >= 192 && n_rows >= 500 && n_rows <= 4096) return false;
+  return tiles >= (m <= 96 ? 400 : 768) || (n_rows <= 128 && tiles >= 250);
+}
+
 void run_product(hipStream_t s, float* output, float beta, const float* input, const float* weights, float* workspace,
                  const ct_conv_desc& d, const ConvShape& sh, bool forward) {
   ConvProductArgs a{};
@@ -588,7 +611,7 @@ int backward_data_t(void* stream, T* input_gradient, const T* output_gradient, c
   hipStream_t s = static_cast<hipStream_t>(stream);
   // unrolled[b] [n_cols, n_rows] = weights^T [n_cols, out_channels] x output_gradient[b] [out_channels, n_rows]
   if constexpr (std::is_same<T, float>::value) {
-    if (sh.conv_image > 0 && matrix_core_product(d, sh, sh.n_cols, d.out_channels)) {
+    if (backward_data_product(d, sh)) {
       run_product(s, const_cast<float*>(output_gradient), 0.f, nullptr, weights, workspace, d, sh, false);
       roll_back(s, workspace, input_gradient, d, sh);
       note_kernel("conv_product+conv_roll");
