@@ -356,17 +356,27 @@ void roll_back(hipStream_t s, const T* workspace, T* input_gradient, const ct_co
   }
 }
 
-// Whether a float product goes to the matrix-core kernels: where they have the tiles to fill the
-// chip, or a k so short that the chain over it is over before the library's second launch is.
-// A tile of 16 k takes about 0.9 us when a block has the unit to itself, whatever the number of
-// blocks, and the library's two launches 15 to 20 us: forward over [1, 64, 56, 56] and 64 windows
-// of 3 x 3 (k 576, 25 tiles) 43 us here, 19 there; over [3, 15, 109, 109] (k 135, 279 tiles) 28 and
-// 36; over [134, 94, 15, 15] and 145 windows (k 846, 707 tiles) 147 both; over [34, 30, 57, 57] and
-// 106 of 5 x 5 (k 750, 1493 tiles) 250 and 347.
-bool matrix_core_product(const ct_conv_desc& d, const ConvShape& sh, int64_t m, int64_t k) {
-  constexpr int64_t kFullChip = 768, kShortChain = 192;
-  return sh.in_image > 0 && d.kernel_width * d.kernel_height <= kConvMaskTaps && sh.n_rows <= conv_product_positions(m) &&
-         (k <= kShortChain || conv_product_units(m, sh.batch * sh.n_rows) >= kFullChip);
+// Whether a float product goes to the matrix-core kernels: not where the library is faster.  Times are
+// those of the kernels, the unrolling in front of the library's forward product counted; where a
+// product is over in some ten microseconds the host's part decides, and the library's is longer, by
+// 3 us and by 5 us for forward, which has a launch more there.
+//
+// Forward: k up to 160 cells, the chain of a block being over before the library's second launch
+// is (a tile of 16 k takes about 0.9 us when a block has the unit to itself, whatever the number of
+// blocks): [1, 13, 10, 10] under 8 windows of 3 x 3 (k 117) 8.9 and 7.0 us, but a call takes 10.4
+// and 14.8; [38, 7, 10, 10] under 39 of 5 x 5 at stride 2 (k 175, 3 tiles) 17 and 7, calls 17.9 and
+// 15.0.  Above, the tiles to fill the chip: [1, 64, 56, 56] under 64 of 3 x 3 (k 576, 25 tiles) 43
+// and 19; [64, 64, 56, 56] under 64 235 and 263, [34, 30, 57, 57] under 106 of 5 x 5 (k 750) 237 and
+// 338.  From 128 out channels and 576 cells on the library's larger tiles win again:
+// [16, 64, 56, 56] under 128 (k 576) 114 and 91, [16, 128, 28, 28] under 512 223 and 164.
+bool forward_product(const ct_conv_desc& d, const ConvShape& sh) {
+  constexpr int64_t kFullChip = 768, kShortChain = 160, kMidChain = 192, kMidTiles = 128, kLongChain = 576, kManyRows = 128;
+  const int64_t m = d.out_channels, k = sh.n_cols, tiles = conv_product_units(m, sh.batch * sh.n_rows);
+  if (sh.in_image == 0 || k < 4 || d.kernel_width * d.kernel_height > kConvMaskTaps ||
+      sh.n_rows > conv_product_positions(m))
+    return false;
+  if (k <= kShortChain || (k <= kMidChain && tiles >= kMidTiles)) return true;
+  return tiles >= kFullChip && (k < kLongChain || m < kManyRows);
 }
 
 // Backward-data, of m cells over k out channels: the library needs one launch here too, and its times
@@ -432,7 +442,7 @@ int forward_t(void* stream, T* output, double output_alpha, const T* input, cons
   if constexpr (std::is_same<T, float>::value) {
     // The kernel gathers the input while other blocks store the output: a call in place, or on buffers that
     // share some of their bytes, unrolls the whole input first.
-    if (sh.n_cols >= 4 && matrix_core_product(d, sh, d.out_channels, sh.n_cols) &&
+    if (forward_product(d, sh) &&
         !overlap(output, sh.batch * sh.out_image, input, sh.batch * sh.in_image)) {
       run_product(s, output, (float)output_alpha, input, weights, workspace, d, sh, true);
       note_kernel("conv_product");

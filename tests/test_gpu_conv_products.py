@@ -41,7 +41,7 @@ def test_weight_gradient_over_many_images(P, code, batch):
 
 # (batch, in channels, out channels, height, width, kernel width, kernel height, pad, stride): the edges of the tiles
 # (32, 64 and 128 rows, 128 and 64 columns, 16 k, 64 positions of a piece), of a run of sums (128 k), of the mask of taps
-# (32), of the rows (4 positions, 4 cells) and of the routes (k 192, 768 tiles)
+# (32), of the rows (4 positions, 4 cells) and of the routes
 PRODUCT_CASES = [
     (1, 1, 1, 2, 2, 1, 1, 0, 1),        # 4 positions, 1 cell: the product is the library's
     (1, 1, 3, 1, 3, 1, 1, 0, 1),        # 3 positions
@@ -53,8 +53,10 @@ PRODUCT_CASES = [
     (5, 3, 65, 11, 10, 3, 3, 1, 2),     # 65 rows, strided, 30 positions
     (2, 14, 130, 9, 8, 3, 3, 1, 1),     # 126 cells: one run; 130 rows in tiles of 64
     (2, 15, 128, 9, 15, 3, 3, 0, 1),    # 135 cells: two runs; tiles of 128 rows
-    (1, 21, 9, 6, 6, 3, 3, 1, 1),       # 189 cells: the last short chain
-    (1, 22, 9, 6, 6, 3, 3, 1, 1),       # 198 cells, few tiles: the library
+    (1, 17, 9, 6, 6, 3, 3, 1, 1),       # 153 cells: the last short chain
+    (1, 18, 9, 6, 6, 3, 3, 1, 1),       # 162 cells, few tiles: the library
+    (1, 21, 9, 6, 6, 3, 3, 1, 1),       # 189 cells
+    (1, 22, 9, 6, 6, 3, 3, 1, 1),       # 198 cells
     (2, 3, 200, 5, 5, 3, 3, 1, 1),      # the same for backward-data, over 200 out channels
     (1, 2, 4, 27, 19, 5, 5, 2, 1),      # 25 taps, 513 positions: two pieces
     (1, 2, 4, 13, 12, 6, 6, 2, 1),      # 36 taps: no mask
@@ -82,6 +84,13 @@ def weight_route(batch, m, n, n_rows):
 def tiles_of(m, n):
     rows = 32 if m <= 32 else 64 if -(-m // 64) % 2 else 128
     return -(-m // rows) * -(-n // (64 if rows == 128 else 128))
+
+
+def forward_route(batch, m, k, n_rows, taps):
+    """The kernels of an output of m channels over k cells."""
+    tiles = tiles_of(m, batch * n_rows)
+    ours = k <= 160 or (k <= 192 and tiles >= 128) or (tiles >= 768 and (k < 576 or m < 128))
+    return "conv_product" if ours and k >= 4 and taps <= 32 else "conv_unroll+gemm"
 
 
 def data_route(batch, m, k, n_rows):
@@ -116,6 +125,15 @@ WEIGHT_CASES = [
     (7, 160, 128, 11, 9, 3, 3, 1, 1),   # seven partial products of 46 tiles
 ]
 
+# The same for the output's routes
+FORWARD_CASES = [
+    (20, 20, 6, 28, 28, 3, 3, 1, 1),    # 180 cells, 123 tiles: the library
+    (21, 20, 6, 28, 28, 3, 3, 1, 1),    # 129 tiles
+    (62, 64, 6, 40, 40, 3, 3, 1, 1),    # 576 cells over 775 tiles, few out channels
+    (32, 63, 128, 39, 40, 3, 3, 1, 1),  # 567 cells over 780 tiles
+    (32, 64, 128, 39, 40, 3, 3, 1, 1),  # 576 cells: the library
+]
+
 # The same for the input gradient's routes
 DATA_CASES = [
     (2, 3, 112, 5, 5, 3, 3, 1, 1),      # one tile over 112 out channels
@@ -132,7 +150,7 @@ DATA_CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", PRODUCT_CASES + WEIGHT_CASES + DATA_CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("case", PRODUCT_CASES + WEIGHT_CASES + FORWARD_CASES + DATA_CASES, ids=lambda c: "x".join(map(str, c)))
 def test_products_at_the_edges_of_their_tiles(P, case):
     """Whole numbers whose sums stay below 2^24: exact in any order, so everything agrees to the bit."""
     batch, cin, cout, h, w, kw, kh, pad, stride = case
@@ -153,14 +171,9 @@ def test_products_at_the_edges_of_their_tiles(P, case):
                            work.host[:n].reshape(batch, n_rows, n_cols), what)
         assert np.all(got[n:] == 7.0), what
 
-    def route(m, k):
-        rows = 32 if m <= 32 else 64 if -(-m // 64) % 2 else 128
-        tiles = -(-m // rows) * -(-batch * n_rows // (64 if rows == 128 else 128))
-        return kw * kh <= 32 and (k <= 192 or tiles >= 768)
-
     for alpha in (0.0, 2.0):
         kernel = P.run(H.convolution, "forward", vec(out), alpha, vec(inp), vec(weights), vec(work), *geometry)
-        assert (kernel == "conv_product") == (n_cols >= 4 and route(cout, n_cols)), kernel
+        assert kernel == forward_route(batch, cout, n_cols, n_rows, kw * kh), kernel
         H.assert_bit_exact(out.download(), out.host, f"convolution-forward, alpha {alpha}")
         unrolled("unrolled input")
     for alpha in (0.0, 2.0):
