@@ -36,5 +36,27 @@ def test_max_gradient(P, code, k, px, py):
             og, ig = (P.buf(rng.standard_normal(n).astype(NP[code])) for n in (n_out, n_in))
             geometry = (H.pool_desc(k, k, px, py, 2, 2, "max"), 1, planes, h, w, oh, ow)
             P.run(H.pooling_forward, View(out, [n_out]), View(inp, [n_in]), *geometry)
-            P.run(H.pooling_backward, View(ig, [n_in]), View(inp, [n_in]), View(out, [n_out]), View(og, [n_out]), *geometry)
+            kernel = P.run(H.pooling_backward, View(ig, [n_in]), View(inp, [n_in]), View(out, [n_out]), View(og, [n_out]),
+                           *geometry)
+            tiles2 = k == 2 and px == py == 0 and (h, w) == (2 * oh, 2 * ow) and w % 4 == 0
+            general = code == capi.F64 and k == 2 and w % 2 == 1
+            assert kernel == ("pool_backward_tile2" if tiles2 else
+                              "pool_backward_band" if general else "pool_backward_stride2"), (kernel, h, w)
             H.assert_bit_exact(ig.download(), ig.host, f"{planes} planes of {h} x {w}, ceil {up}")
+
+
+def test_wide_planes_of_odd_width_in_double(P):
+    """Planes of an odd width whose rows are off the 16-byte grid every other time: the general form from 2^24 elements on
+    under 3 x 3 windows, and under 2 x 2 always."""
+    k, side = 3, 511
+    out_side = (side - k) // 2 + 1
+    rng = np.random.default_rng(1)
+    for planes, name in ((64, "pool_backward_stride2"), (65, "pool_backward_band")):
+        n_in, n_out = planes * side * side, planes * out_side * out_side
+        inp, out = P.buf(rng.integers(-3, 4, n_in).astype(np.float64)), P.buf(np.zeros(n_out))
+        og, ig = P.buf(rng.integers(-3, 4, n_out).astype(np.float64)), P.buf(rng.integers(-3, 4, n_in).astype(np.float64))
+        geometry = (H.pool_desc(k, k, 0, 0, 2, 2, "max"), 1, planes, side, side, out_side, out_side)
+        P.run(H.pooling_forward, View(out, [n_out]), View(inp, [n_in]), *geometry)
+        kernel = P.run(H.pooling_backward, View(ig, [n_in]), View(inp, [n_in]), View(out, [n_out]), View(og, [n_out]), *geometry)
+        assert kernel == name, (kernel, planes)
+        H.assert_bit_exact(ig.download(), ig.host, f"{planes} planes of {side} x {side}")
