@@ -16,6 +16,10 @@ tables; a training step of a digit network, of which the GPU is busy for 85 us:
 int the results are functions of those values alone and are kept, by value, in
 bounded ``lru_cache`` tables; index tensors and other number types are worked
 out each time.  Callers get fresh lists: nothing that is kept is handed out.
+Shapes that change all the time gain nothing from the tables and pay for their
+entries, so the packed tensors among them are worked out without the general
+algebra (seven functions of a shape never seen: 38 us without tables, 45 with
+tables in front of the general algebra, 15 now; of a shape seen before 7).
 """
 from __future__ import annotations
 
@@ -93,15 +97,24 @@ def extend_strides(shape, strides) -> List[int]:
     return list(reversed(out))
 
 
-@lru_cache(maxsize=_CACHE_LIMIT)
-def _packed_strides(shape: tuple) -> tuple:
-    return tuple(_dimensions(shape, None, None)["strides"])
+def _packed_strides(shape) -> Optional[List[int]]:
+    """Row-major strides of a shape of plain ints of at least 1 (which ``dimensions`` always accepts), else None."""
+    strides, step = [], 1
+    for v in reversed(shape):
+        if type(v) is not int or v < 1:
+            return None
+        strides.append(step)
+        step *= v
+    strides.reverse()
+    return strides
 
 
 def dimensions(shape, names=None, strides=None) -> dict:
     """``dimensions`` (:95-118)."""
-    if strides is None and _plain(shape):
-        return {"shape": list(shape), "strides": list(_packed_strides(tuple(shape))), "names": names}
+    if strides is None:
+        packed = _packed_strides(shape)
+        if packed:
+            return {"shape": list(shape), "strides": packed, "names": names}
     return _dimensions(shape, names, strides)
 
 
@@ -180,7 +193,22 @@ def _dense_of(shp, strides) -> bool:
     return pairs[0][1] == rest
 
 
-_dense_direct = lru_cache(maxsize=_CACHE_LIMIT)(_dense_of)
+def _dense_plain(shp, strides) -> bool:
+    """``_dense_of`` for plain ints: the first of the largest strides steps over all the other elements."""
+    if len(shp) == 1:
+        return strides[0] == 1
+    count, largest, extent = 1, None, 1
+    for s, st in zip(shp, strides):
+        if s != 1:
+            count *= s
+            if largest is None or st > largest:
+                largest, extent = st, s
+    if count == 0:
+        return _dense_of(shp, strides)
+    return largest is not None and largest * extent == count
+
+
+_dense_direct = lru_cache(maxsize=_CACHE_LIMIT)(_dense_plain)
 
 
 def direct(dims) -> bool:
@@ -232,8 +260,23 @@ def max_extend_strides(shp, strides, max_count: int) -> List[int]:
 
 @lru_cache(maxsize=_CACHE_LIMIT)
 def _max_shape_direct(key: tuple) -> tuple:
-    info = _dimension_seq_to_max_shape([{"shape": s, "strides": st} for s, st in key])
-    return tuple(info["max-shape"]), tuple((tuple(d["shape"]), tuple(d["strides"])) for d in info["dimensions"])
+    max_count = 0
+    for shp, strides in key:
+        if len(shp) != len(strides) or not shp:
+            _dimension_seq_to_max_shape([{"shape": list(s), "strides": list(st)} for s, st in key])   # says what is wrong
+        max_count = max(max_count, len(shp))
+    max_shape, extended = [0] * max_count, []
+    for shp, strides in key:
+        pad = max_count - len(shp)
+        if pad:
+            mi = strides.index(max(strides))
+            strides = (strides[mi] * shp[mi],) * pad + strides
+            shp = (1,) * pad + shp
+        for i, v in enumerate(shp):
+            if v > max_shape[i]:
+                max_shape[i] = v
+        extended.append((shp, strides))
+    return tuple(max_shape), tuple(extended)
 
 
 @lru_cache(maxsize=_CACHE_LIMIT)
@@ -281,10 +324,28 @@ def minimize(dims) -> dict:
     return {"shape": [s for s, _ in out], "strides": [st for _, st in out]}
 
 
-@lru_cache(maxsize=_CACHE_LIMIT)
-def _reshaped_strides(key: tuple, new_shape: tuple) -> tuple:
+def _reshape_plain(key: tuple, new_shape: tuple) -> tuple:
     (shp, strides), = key
+    packed = _packed_strides(new_shape)
+    if packed and shp and len(shp) == len(strides):
+        # most tensors are packed, and their reshape is the packed one
+        old = new = 1
+        for s in shp:
+            old *= s
+        for s in new_shape:
+            new *= s
+        last = strides[0]
+        for st in strides:
+            if st > last:
+                break
+            last = st
+        else:
+            if new <= old and _dense_plain(shp, strides):
+                return tuple(packed)
     return tuple(_in_place_reshape({"shape": list(shp), "strides": list(strides)}, list(new_shape))["strides"])
+
+
+_reshaped_strides = lru_cache(maxsize=_CACHE_LIMIT)(_reshape_plain)
 
 
 def in_place_reshape(existing_dims, new_shape: Sequence[int]) -> dict:
@@ -343,9 +404,8 @@ def _in_place_reshape(existing_dims, new_shape: List[int]) -> dict:
 @lru_cache(maxsize=_CACHE_LIMIT)
 def _matrix_direct(key: tuple, to_shape) -> tuple:
     (shp, strides), = key
-    d = {"shape": list(shp), "strides": list(strides)}
-    d = _in_place_reshape(d, to_shape(d))
-    return tuple(d["shape"]), tuple(d["strides"])
+    new_shape = tuple(to_shape({"shape": list(shp), "strides": list(strides)}))
+    return new_shape, _reshape_plain(key, new_shape)
 
 
 def as_matrix(dims, to_shape) -> dict:

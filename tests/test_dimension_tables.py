@@ -75,3 +75,24 @@ def test_results_belong_to_the_caller():
 
 def test_truth_values_are_not_taken_for_the_ints_they_equal():
     assert dims.direct_key({"shape": [True, 2], "strides": [2, 1]}) is None
+
+
+def test_shapes_never_seen_are_worked_out_directly(monkeypatch):
+    """A program whose shapes change all the time pays for the tables' keys and entries; the general algebra on top of
+    that made it slower than no tables.  Packed tensors of plain ints have to do without it, the first time too."""
+    def general(*_):
+        raise AssertionError("the general path")
+
+    for name in ("_dimensions", "_dense_of", "_dimension_seq_to_max_shape", "_in_place_reshape"):
+        monkeypatch.setattr(dims, name, general)
+    rng = random.Random(99)
+    for _ in range(50):
+        n, c = rng.randint(2, 10 ** 7), rng.randint(2, 10 ** 6)
+        d = dims.dimensions([n, 1, c])
+        assert d["strides"] == [c, c, 1]
+        assert dims.dense(d) and dims.access_increasing(d) and dims.ecount(d) == n * c
+        assert dims.in_place_reshape(d, [n * c])["strides"] == [1]
+        assert dims.as_matrix(d, dims.to_batch_shape) == {"shape": [n, c], "strides": [c, 1]}
+        info = dims.dimension_seq_to_max_shape(d, dims.dimensions([c]))
+        assert info == {"max-shape": [n, 1, c], "dimensions": [{"shape": [n, 1, c], "strides": [c, c, 1]},
+                                                               {"shape": [1, 1, c], "strides": [c, c, 1]}]}
