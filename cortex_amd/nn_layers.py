@@ -233,6 +233,14 @@ class Dropout:
         self.rand_buffer = (self.mult_buffer if self.mult_buffer.get_datatype() == "float"
                             else ct.new_tensor([batch_size, n_items], datatype="float"))
 
+    def _one_launch(self) -> bool:
+        """Whether the launch that stores the multipliers can take the buffers: whole ones of one count, float draws,
+        float or double multipliers.  Others take the chain of tensor calls, which converts and checks."""
+        mult, draws = self.mult_buffer, self.rand_buffer
+        return (mult.get_datatype() in ("float", "double") and draws.get_datatype() == "float" and
+                mult.device is draws.device and mult.ecount() == draws.ecount() and
+                all(ct.dense(t) and t.buffer.ecount() == t.ecount() for t in (mult, draws)))
+
     def prepare_forward(self, parameter_buffers=None, input_buffers=None, output_buffers=None):
         kind = self.layer["distribution"]
         if kind not in ("bernoulli", "gaussian"):
@@ -242,8 +250,7 @@ class Dropout:
             # A driver may have the chain below as one launch that stores the same values (the mask of a digit
             # network's 128 x 128 units: two launches of 2.4 us on the GPU, some 20 us of host time, against one).
             fused = getattr(ct.check_stream(), "dropout_bernoulli_mask", None)
-            whole = all(ct.dense(t) and t.buffer.ecount() == t.ecount() for t in (self.mult_buffer, self.rand_buffer))
-            if fused is not None and whole and 0.0 < maximum <= 1.0:
+            if fused is not None and self._one_launch() and 0.0 < maximum <= 1.0:
                 fused(self.mult_buffer.buffer, self.rand_buffer.buffer, self.layer["probability"])
                 return
             distribution = ct.flat_distribution(minimum=maximum - 1.0, maximum=maximum)
