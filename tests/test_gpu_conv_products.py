@@ -152,13 +152,31 @@ DATA_CASES = [
 
 @pytest.mark.parametrize("case", PRODUCT_CASES + WEIGHT_CASES + FORWARD_CASES + DATA_CASES, ids=lambda c: "x".join(map(str, c)))
 def test_products_at_the_edges_of_their_tiles(P, case):
-    """Whole numbers whose sums stay below 2^24: exact in any order, so everything agrees to the bit."""
     batch, cin, cout, h, w, kw, kh, pad, stride = case
-    oh, ow = (h + 2 * pad - kh) // stride + 1, (w + 2 * pad - kw) // stride + 1
+    check_products(P, batch, cin, cout, h, w, kw, kh, pad, pad, stride, stride)
+
+
+# (batch, in channels, out channels, height, width, kernel width, kernel height, pad x and y, stride x and y): windows,
+# paddings and strides that differ between the directions, decoded from one number of a cell
+@pytest.mark.parametrize("case", [
+    (3, 5, 20, 9, 14, 3, 2, 1, 0, 2, 1),
+    (3, 5, 20, 14, 9, 2, 5, 0, 2, 1, 3),
+    (2, 3, 40, 17, 11, 7, 4, 3, 1, 2, 3),
+    (2, 2, 70, 8, 21, 8, 4, 0, 3, 3, 1),    # 32 taps
+    (2, 2, 70, 21, 8, 3, 11, 2, 5, 1, 2),   # 33: no mask
+    (4, 9, 33, 13, 7, 1, 5, 0, 4, 1, 1),
+], ids=lambda c: "x".join(map(str, c)))
+def test_products_under_rectangular_windows(P, case):
+    check_products(P, *case)
+
+
+def check_products(P, batch, cin, cout, h, w, kw, kh, px, py, sx, sy):
+    """Whole numbers whose sums stay below 2^24: exact in any order, so everything agrees to the bit."""
+    oh, ow = (h + 2 * py - kh) // sy + 1, (w + 2 * px - kw) // sx + 1
     n_rows, n_cols = oh * ow, cin * kw * kh
-    desc = H.conv_desc(cin, cout, kw, kh, pad, pad, stride, stride)
+    desc = H.conv_desc(cin, cout, kw, kh, px, py, sx, sy)
     geometry = (desc, batch, h, w, oh, ow)
-    rng = np.random.default_rng(sum(case))
+    rng = np.random.default_rng(batch + cin + cout + h + w + kw + kh + px + sx)
     ints = lambda n: rng.integers(-2, 3, n).astype(np.float32)
     inp, weights, og = P.buf(ints(batch * cin * h * w)), P.buf(ints(cout * n_cols)), P.buf(ints(batch * cout * n_rows))
     out, wg, ig = P.buf(ints(batch * cout * n_rows)), P.buf(ints(cout * n_cols)), P.buf(ints(batch * cin * h * w))
