@@ -808,20 +808,29 @@ void launch_band(hipStream_t s, bool forward, dim3 grid, size_t lds, const BandA
   else hipLaunchKernelGGL((pool_backward_band_kernel<T, OP, KW, KH>), grid, dim3(kBlock), lds, s, a);
 }
 
-// Whether the gradient of the maximum takes the kernel for stride 2.  Measured over 14 shapes (sides of 7
-// to 224, 64 to 16384 planes) for each of 2 x 2 and 3 x 3 windows, with and without padding: float 1.02 to
-// 2.2 times as fast as the general form, whatever the width; double 1.0 to 1.5 times where the
-// width is even.  In double an odd width puts every other row off the 16-byte grid of its pieces,
-// which the general form walks across the rows: 2 x 2 0.89 to 1.0 (16384 planes of 13 x 13 14.2
-// and 15.9 us), 3 x 3 0.98 to 1.25 but 0.97 for what exceeds the caches (2048 planes of 113 x 113
-// 145 and 150 us).
+// Whether the gradient of the maximum takes the kernel for stride 2.  Rows that are whole 16-byte pieces:
+// 1.0 to 2.2 times as fast as the general form, but 0.96 to 1.0 for double under 2 x 2 beyond
+// 100 MiB.  Other rows put its pieces off the 16-byte grid,
+// which the general form walks across the rows; that costs it the more, the less of the
+// tensors the last-level cache holds.  Measured behind a fill of the gradient, 36 shapes of 4 to
+// 33 M elements for each datatype (times the general form's speed):
+//   float, 3 x 3   1.05 to 1.6 up to 24 M elements; beyond, odd widths 1.1 to 1.3 and widths from 90 on
+//                  1.0 to 1.2, but even ones of 46 to 74 0.83 to 0.92 (33 M of 62 x 62: 89 and 104 us)
+//   float, 2 x 2   1.0 to 1.2 up to 10 M; even widths of 46 to 78 0.94 to 0.99 at 16 M and 0.75 to 0.82 at
+//                  33 M, where others are between 0.87 and 1.1
+//   double, 3 x 3  1.02 to 1.1 at 4 M, 0.93 to 1.04 at 10 M, 0.85 to 0.92 at 16 M
+//   double, 2 x 2  0.89 to 1.0 throughout
 template <class T>
 bool max_gradient_at_stride2(const ct_pool_desc& d, const PoolShape& sh) {
   if (d.pool_op != CT_POOL_MAX || d.stride_x != 2 || d.stride_y != 2 || d.kernel_width != d.kernel_height ||
       (d.kernel_width != 2 && d.kernel_width != 3))
     return false;
-  const bool in_caches = sh.planes * sh.in_h * sh.in_w <= int64_t(1) << 24;
-  return sizeof(T) == 4 || sh.in_w % 2 == 0 || (d.kernel_width == 3 && in_caches);
+  const int64_t mib = (sh.planes * sh.in_h * sh.in_w * (int64_t)sizeof(T)) >> 20;
+  const bool three = d.kernel_width == 3, short_even = sh.in_w % 2 == 0 && sh.in_w < 80;
+  if (sh.in_w * (int64_t)sizeof(T) % 16 == 0) return sizeof(T) == 4 || three || mib < 100;
+  if (sizeof(T) == 8) return three && mib < 64;
+  if (three) return !short_even || mib < 100;
+  return mib < (short_even ? 48 : 100);
 }
 
 template <class T, int OP>

@@ -45,18 +45,22 @@ def test_max_gradient(P, code, k, px, py):
             H.assert_bit_exact(ig.download(), ig.host, f"{planes} planes of {h} x {w}, ceil {up}")
 
 
-def test_wide_planes_of_odd_width_in_double(P):
-    """Planes of an odd width whose rows are off the 16-byte grid every other time: the general form from 2^24 elements on
-    under 3 x 3 windows, and under 2 x 2 always."""
-    k, side = 3, 511
+@pytest.mark.parametrize("code,k,side,planes", [
+    (capi.F64, 3, 511, 32), (capi.F64, 3, 511, 33), (capi.F32, 3, 78, 4308), (capi.F32, 3, 78, 4309),
+    (capi.F32, 2, 62, 3273), (capi.F32, 2, 62, 3274), (capi.F32, 2, 511, 100), (capi.F32, 2, 511, 101),
+    (capi.F64, 2, 510, 50), (capi.F64, 2, 510, 51),
+], ids=lambda v: str(v))
+def test_rows_off_the_16_byte_grid(P, code, k, side, planes):
+    """Both sides of the sizes from which such rows take the general form: 64, 100, 48 and 100 MiB of gradient; and 100 for
+    rows on the grid in double under 2 x 2 windows."""
     out_side = (side - k) // 2 + 1
-    rng = np.random.default_rng(1)
-    for planes, name in ((64, "pool_backward_stride2"), (65, "pool_backward_band")):
-        n_in, n_out = planes * side * side, planes * out_side * out_side
-        inp, out = P.buf(rng.integers(-3, 4, n_in).astype(np.float64)), P.buf(np.zeros(n_out))
-        og, ig = P.buf(rng.integers(-3, 4, n_out).astype(np.float64)), P.buf(rng.integers(-3, 4, n_in).astype(np.float64))
-        geometry = (H.pool_desc(k, k, 0, 0, 2, 2, "max"), 1, planes, side, side, out_side, out_side)
-        P.run(H.pooling_forward, View(out, [n_out]), View(inp, [n_in]), *geometry)
-        kernel = P.run(H.pooling_backward, View(ig, [n_in]), View(inp, [n_in]), View(out, [n_out]), View(og, [n_out]), *geometry)
-        assert kernel == name, (kernel, planes)
-        H.assert_bit_exact(ig.download(), ig.host, f"{planes} planes of {side} x {side}")
+    rng = np.random.default_rng(planes)
+    n_in, n_out = planes * side * side, planes * out_side * out_side
+    ints = lambda n: rng.integers(-3, 4, n).astype(NP[code])
+    inp, out, og, ig = P.buf(ints(n_in)), P.buf(np.zeros(n_out, NP[code])), P.buf(ints(n_out)), P.buf(ints(n_in))
+    geometry = (H.pool_desc(k, k, 0, 0, 2, 2, "max"), 1, planes, side, side, out_side, out_side)
+    P.run(H.pooling_forward, View(out, [n_out]), View(inp, [n_in]), *geometry)
+    kernel = P.run(H.pooling_backward, View(ig, [n_in]), View(inp, [n_in]), View(out, [n_out]), View(og, [n_out]), *geometry)
+    limit = 64 if code == capi.F64 and k == 3 else 48 if (k, side) == (2, 62) else 100
+    assert kernel == ("pool_backward_stride2" if n_in * NP[code]().itemsize >> 20 < limit else "pool_backward_band"), kernel
+    H.assert_bit_exact(ig.download(), ig.host, f"{planes} planes of {side} x {side}")
