@@ -357,38 +357,36 @@ void roll_back(hipStream_t s, const T* workspace, T* input_gradient, const ct_co
 }
 
 // Whether a float product goes to the matrix-core kernels: not where the library is faster.  Times are
-// those of the kernels, the unrolling in front of the library's forward product counted; where a
-// product is over in some ten microseconds the host's part decides, and the library's is longer, by
-// 3 us and by 5 us for forward, which has a launch more there.
+// those of the kernels, the unrolling in front of the library's forward product counted.  Where a
+// product is over in some twenty microseconds a layer is bound by the host, and a call of the library
+// costs that 5 to 9 us more.
 //
-// Forward: k up to 160 cells, the chain of a block being over before the library's second launch
+// Forward: k up to 192 cells, the chain of a block being over before the library's second launch
 // is (a tile of 16 k takes about 0.9 us when a block has the unit to itself, whatever the number of
 // blocks): [1, 13, 10, 10] under 8 windows of 3 x 3 (k 117) 8.9 and 7.0 us, but a call takes 10.4
-// and 14.8; [38, 7, 10, 10] under 39 of 5 x 5 at stride 2 (k 175, 3 tiles) 17 and 7, calls 17.9 and
-// 15.0.  Above, the tiles to fill the chip: [1, 64, 56, 56] under 64 of 3 x 3 (k 576, 25 tiles) 43
-// and 19; [64, 64, 56, 56] under 64 235 and 263, [34, 30, 57, 57] under 106 of 5 x 5 (k 750) 237 and
-// 338.  From 128 out channels and 576 cells on the library's larger tiles win again:
+// and 14.8; [38, 7, 10, 10] under 39 of 5 x 5 at stride 2 (k 175, 3 tiles) 17 and 7, the layer's three
+// calls 83 and 90.  Above, the tiles to fill the chip: [1, 64, 56, 56] under 64 of 3 x 3 (k 576, 25
+// tiles) 43 and 19; [64, 64, 56, 56] under 64 235 and 263, [34, 30, 57, 57] under 106 of 5 x 5 (k 750)
+// 237 and 338.  From 128 out channels and 576 cells on the library's larger tiles win again:
 // [16, 64, 56, 56] under 128 (k 576) 114 and 91, [16, 128, 28, 28] under 512 223 and 164.
 bool forward_product(const ct_conv_desc& d, const ConvShape& sh) {
-  constexpr int64_t kFullChip = 768, kShortChain = 160, kMidChain = 192, kMidTiles = 128, kLongChain = 576, kManyRows = 128;
+  constexpr int64_t kFullChip = 768, kShortChain = 192, kLongChain = 576, kManyRows = 128;
   const int64_t m = d.out_channels, k = sh.n_cols, tiles = conv_product_units(m, sh.batch * sh.n_rows);
   if (sh.in_image == 0 || k < 4 || d.kernel_width * d.kernel_height > kConvMaskTaps ||
       sh.n_rows > conv_product_positions(m))
     return false;
-  if (k <= kShortChain || (k <= kMidChain && tiles >= kMidTiles)) return true;
-  return tiles >= kFullChip && (k < kLongChain || m < kManyRows);
+  return k <= kShortChain || (tiles >= kFullChip && (k < kLongChain || m < kManyRows));
 }
 
 // Backward-data, of m cells over k out channels: the library needs one launch here too, and its times
 // depend on more than the sizes (20 to 110 TFLOP/s for products of one size).  The lines below are
 // drawn through 310 shapes; its time is the second.
-//  - Few tiles: k up to 112 ([9, 10, 15, 15] under 102 of 3 x 3 10.0 and 7.2 us, calls 13.7 and
-//    16.1; k 128, [1, 128, 28, 28], 12.4 and 6.9, calls 16.9 and 15.4).
-//  - k up to 64: results of up to 2 M cells, where the host decides; images of more than 3500
-//    positions ([69, 6, 71, 71] under 38 34 and 130, [3, 64, 112, 112] under 64 41 and 56); and from
-//    1750 tiles on ([64, 64, 56, 56] under 64 212 and 236; below, [16, 64, 28, 28] under 64, 882
-//    tiles, 22 and 17).
-//  - k above: from 768 tiles on ([38, 53, 21, 21] under 155 of 5 x 5 90 and 196), 400 for up to 96
+//  - k up to 64: from 0.76 to 5.4 times the library's speed, below 0.9 only where the product takes
+//    20 us or less ([16, 64, 28, 28] under 64 of 3 x 3 22 and 17, [69, 6, 71, 71] under 38 34 and 130,
+//    [64, 64, 56, 56] under 64 212 and 236).
+//  - Few tiles: k up to 160 ([9, 10, 15, 15] under 102 10.0 and 7.2 us, calls 13.7 and 16.1; k 256,
+//    [1, 128, 28, 28] under 256 of 1 x 1, 17.8 and 4.1, calls 20.4 and 15.7).
+//  - Otherwise from 768 tiles on ([38, 53, 21, 21] under 155 of 5 x 5 90 and 196), 400 for up to 96
 //    cells ([60, 9, 28, 28] under 181 32 and 67), 250 for images of up to 128 positions
 //    ([32, 256, 7, 7] under 256 32 and 55).  But not k up to 256 over 192 cells or more in images of
 //    500 to 4096 positions, where the library runs at 80 to 110 TFLOP/s: [64, 128, 28, 28] under 128
@@ -396,8 +394,7 @@ bool forward_product(const ct_conv_desc& d, const ConvShape& sh) {
 bool backward_data_product(const ct_conv_desc& d, const ConvShape& sh) {
   const int64_t m = sh.n_cols, k = d.out_channels, n_rows = sh.n_rows, tiles = conv_product_units(m, sh.batch * n_rows);
   if (sh.conv_image == 0 || n_rows > conv_product_positions(m)) return false;
-  if (k <= 112 && tiles < 128) return true;
-  if (k <= 64) return m * sh.batch * n_rows <= (int64_t(1) << 21) || n_rows > 3500 || tiles >= 1750 || (n_rows <= 128 && tiles >= 250);
+  if (k <= 64 || (k <= 160 && tiles < 256)) return true;
   if (k <= 256 && m >= 192 && n_rows >= 500 && n_rows <= 4096) return false;
   return tiles >= (m <= 96 ? 400 : 768) || (n_rows <= 128 && tiles >= 250);
 }
@@ -525,7 +522,8 @@ void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t 
 //    piece, the library 7 to 10 ns for a position of an image: [16, 64, 56, 56] under 256 of 1 x 1
 //    (64 blocks of 49 pieces) 83 and 28 us, [16, 64, 28, 28] under 64 of 3 x 3 (144 of 13) 30 and
 //    27; but [1, 64, 56, 56] under 64 (63 of 7) 19 and 24, [3, 15, 109, 109] under 84 (138 of 25)
-//    48 and 96.  Results of up to 32 rows or columns, whose blocks have half the waves, fill
+//    48 and 96.  Runs of up to four pieces are over before the host has called the library.
+//    Results of up to 32 rows or columns, whose blocks have half the waves, fill
 //    it for images of up to 2048 positions only: [71, 42, 77, 77] under 11 185 and 137 us,
 //    [40, 63, 60, 60] under 4 of 5 x 5 185 and 144; [34, 89, 37, 37] under 5 83 and 121.
 // Rows shorter than a 16-byte load are the library's too.
@@ -549,7 +547,7 @@ bool weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t fit, ConvWe
   const bool narrow = a.m <= 32 || a.n <= 32;
   if (sh.n_rows > 2 * kConvPiece && run > 1 && (narrow ? tiles / 2 : tiles) > kManyTiles) return false;
   const bool full = tiles * *splits * conv_weight_waves(a.m, a.n) >= kFewWaves && !(narrow && sh.n_rows > kNarrowImage);
-  return full || sh.n_rows <= kShortImage || run <= std::max<int64_t>(2, sh.n_rows / kPositionsPerPiece);
+  return full || sh.n_rows <= kShortImage || run <= std::max<int64_t>(4, sh.n_rows / kPositionsPerPiece);
 }
 
 template <class T>

@@ -53,10 +53,8 @@ PRODUCT_CASES = [
     (5, 3, 65, 11, 10, 3, 3, 1, 2),     # 65 rows, strided, 30 positions
     (2, 14, 130, 9, 8, 3, 3, 1, 1),     # 126 cells: one run; 130 rows in tiles of 64
     (2, 15, 128, 9, 15, 3, 3, 0, 1),    # 135 cells: two runs; tiles of 128 rows
-    (1, 17, 9, 6, 6, 3, 3, 1, 1),       # 153 cells: the last short chain
-    (1, 18, 9, 6, 6, 3, 3, 1, 1),       # 162 cells, few tiles: the library
-    (1, 21, 9, 6, 6, 3, 3, 1, 1),       # 189 cells
-    (1, 22, 9, 6, 6, 3, 3, 1, 1),       # 198 cells
+    (1, 21, 9, 6, 6, 3, 3, 1, 1),       # 189 cells: the last short chain
+    (1, 22, 9, 6, 6, 3, 3, 1, 1),       # 198 cells, few tiles: the library
     (2, 3, 200, 5, 5, 3, 3, 1, 1),      # the same for backward-data, over 200 out channels
     (1, 2, 4, 27, 19, 5, 5, 2, 1),      # 25 taps, 513 positions: two pieces
     (1, 2, 4, 13, 12, 6, 6, 2, 1),      # 36 taps: no mask
@@ -76,7 +74,7 @@ def weight_route(batch, m, n, n_rows):
     narrow = m <= 32 or n <= 32
     if n_rows < 4 or (n_rows > 128 and run > 1 and tiles // (2 if narrow else 1) > 64):
         return "gemm+conv_sum_partials"
-    if n_rows > 400 and (waves < 1400 or narrow and n_rows > 2048) and run > max(2, n_rows // 200):
+    if n_rows > 400 and (waves < 1400 or narrow and n_rows > 2048) and run > max(4, n_rows // 200):
         return "gemm+conv_sum_partials"
     return "conv_weight_gradient" + ("+conv_sum_partials" if splits > 1 else "")
 
@@ -89,7 +87,7 @@ def tiles_of(m, n):
 def forward_route(batch, m, k, n_rows, taps):
     """The kernels of an output of m channels over k cells."""
     tiles = tiles_of(m, batch * n_rows)
-    ours = k <= 160 or (k <= 192 and tiles >= 128) or (tiles >= 768 and (k < 576 or m < 128))
+    ours = k <= 192 or (tiles >= 768 and (k < 576 or m < 128))
     return "conv_product" if ours and k >= 4 and taps <= 32 else "conv_unroll+gemm"
 
 
@@ -97,10 +95,8 @@ def data_route(batch, m, k, n_rows):
     """The kernels of the input gradient of m cells over k out channels."""
     n = batch * n_rows
     tiles = tiles_of(m, n)
-    if k <= 112 and tiles < 128:
+    if k <= 64 or (k <= 160 and tiles < 256):
         ours = True
-    elif k <= 64:
-        ours = m * n <= 1 << 21 or n_rows > 3500 or tiles >= 1750 or (n_rows <= 128 and tiles >= 250)
     elif k <= 256 and m >= 192 and 500 <= n_rows <= 4096:
         ours = False
     else:
@@ -120,6 +116,7 @@ WEIGHT_CASES = [
     (3, 64, 64, 40, 40, 3, 3, 1, 1),    # seven splits of eleven pieces: the library
     (2, 60, 3, 48, 48, 3, 3, 1, 1),     # 36 splits of two pieces of images of 2304 positions, few rows
     (5, 200, 3, 48, 48, 3, 3, 1, 1),    # the same with fourteen: the library
+    (4, 16, 10, 60, 60, 3, 3, 1, 1),    # four of 3600
     (1, 64, 64, 56, 56, 3, 3, 1, 1),    # seven splits of seven pieces of one image
     (6, 200, 128, 11, 9, 1, 1, 0, 1),   # six splits of two pieces, an image each
     (7, 160, 128, 11, 9, 3, 3, 1, 1),   # seven partial products of 46 tiles
@@ -127,8 +124,6 @@ WEIGHT_CASES = [
 
 # The same for the output's routes
 FORWARD_CASES = [
-    (20, 20, 6, 28, 28, 3, 3, 1, 1),    # 180 cells, 123 tiles: the library
-    (21, 20, 6, 28, 28, 3, 3, 1, 1),    # 129 tiles
     (62, 64, 6, 40, 40, 3, 3, 1, 1),    # 576 cells over 775 tiles, few out channels
     (32, 63, 128, 39, 40, 3, 3, 1, 1),  # 567 cells over 780 tiles
     (32, 64, 128, 39, 40, 3, 3, 1, 1),  # 576 cells: the library
@@ -136,16 +131,17 @@ FORWARD_CASES = [
 
 # The same for the input gradient's routes
 DATA_CASES = [
-    (2, 3, 112, 5, 5, 3, 3, 1, 1),      # one tile over 112 out channels
-    (2, 3, 113, 5, 5, 3, 3, 1, 1),      # over 113: the library
+    (2, 3, 160, 5, 5, 3, 3, 1, 1),      # one tile over 160 out channels
+    (2, 3, 161, 5, 5, 3, 3, 1, 1),      # over 161: the library
     (1, 2, 5, 12, 11, 8, 5, 2, 1),      # 40 taps
-    (70, 3, 20, 26, 26, 3, 3, 1, 1),    # 370 tiles, 1.3 M cells
-    (70, 6, 20, 26, 26, 3, 3, 1, 1),    # 2.6 M: the library
-    (3, 24, 20, 62, 62, 3, 3, 1, 1),    # 3844 positions, 364 tiles
+    (70, 6, 64, 26, 26, 3, 3, 1, 1),    # 370 tiles over 64 out channels
+    (70, 6, 65, 26, 26, 3, 3, 1, 1),    # over 65: the library
+    (48, 11, 65, 26, 26, 3, 3, 1, 1),   # 507 tiles of 99 cells: the library
     (40, 9, 65, 36, 36, 3, 3, 1, 1),    # 810 tiles over 65 out channels
     (41, 5, 65, 35, 36, 3, 3, 1, 1),    # 404 tiles of 45 cells
-    (30, 112, 70, 8, 8, 3, 3, 1, 1),    # 240 tiles of images of 64 positions: the library
-    (32, 112, 70, 8, 8, 3, 3, 1, 1),    # 256
+    (31, 112, 70, 8, 8, 3, 3, 1, 1),    # 248 tiles over 70 out channels
+    (32, 112, 70, 8, 8, 3, 3, 1, 1),    # 256, images of 64 positions
+    (32, 112, 70, 12, 11, 3, 3, 1, 1),  # 528, of 132: the library
     (17, 25, 65, 25, 24, 3, 3, 1, 1),   # 225 cells, 600 positions: the library
 ]
 
