@@ -403,7 +403,6 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
           asm volatile("" : "+v"(to));   // added here, not after the next tile's stores
         }
       }
-      keep_order();
     }
   };
   for (; piece < piece_end; ++piece) {
