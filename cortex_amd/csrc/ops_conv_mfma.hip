@@ -22,11 +22,11 @@
 // loads every tile waited for memory twice (at the branches' joins) before its MFMAs.
 //
 // Rounding.  The matrix cores round after every product, so the error of a sum grows with the length
-// of the chain.  Products are summed in chains of eight (weight gradient: sixteen, then in double), and
-// these are added up.  Against 64 bits, over 90 shapes: outputs 0.40 to 1.03 times the error of the
-// library's products, input gradients 0.31 to 1.04, weight gradients 0.07 to 1.08.  The additions are
-// vector instructions that run while the next products do: chains of 128 took the same time.
+// of the chain.  Products are summed in chains of eight (input gradient over more than 48 channels:
+// sixteen, eight in the last tile; weight gradient: sixteen, then in double), and these are added up.  The additions are vector
+// instructions that run while the next products do: chains of 128 took the same time.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "conv_products.h"
@@ -62,11 +62,12 @@ __device__ __forceinline__ f32x4 fix4(f32x4 v, uint32_t i, uint32_t n) {
 }
 
 // Adds the sixteen products of a tile whose left and right elements four lanes hold, four each, to
-// two sums, eight to each.
-__device__ __forceinline__ void product16(f32x4 left, f32x4 right, f32x4 (&sums)[2]) {
+// one sum, or to two sums, eight to each.
+template <int kSums>
+__device__ __forceinline__ void product16(f32x4 left, f32x4 right, f32x4 (&sums)[kSums]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    sums[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(left[i], right[i], sums[i % 2], 0, 0, 0);
+    sums[i % kSums] = __builtin_amdgcn_mfma_f32_16x16x4f32(left[i], right[i], sums[i % kSums], 0, 0, 0);
 }
 // Matrix and vector instructions stay on their side; scalar ones and memory's may pass.
 __device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80); }
@@ -91,7 +92,8 @@ __device__ __forceinline__ uint32_t unit_of_block(uint32_t b, uint32_t units) {
 //     of up to kConvMaskTaps cells).  The k of a tile are decoded side by side, one to a lane, and
 //     handed round with v_readlane: decoded one after the other on the scalar unit they took
 //     as long as the tile's MFMAs.
-template <int BM, bool kForward>
+// kChains: the sums that take turns with the sixteen products of a tile.
+template <int BM, bool kForward, int kChains>
 __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProductArgs a) {
   constexpr int WM = BM / 128 + 1, WN = 4 / WM, BN = 32 * WN, BK = 16, LD = BK + 4;   // waves: WM x WN
   constexpr int MT = BM / WM / 16, kCols = kBlock / BN, kStep = BK / kCols;   // lanes to a column of `right`, k of each
@@ -229,7 +231,8 @@ __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProdu
   __syncthreads();
   const uint32_t row = lane & 15, group = lane >> 4;
   const uint32_t wave_m = wave / WN * (MT * 16), wave_n = wave % WN * 32;
-  auto multiply = [&](int buffer) {
+  auto multiply = [&](int buffer, auto chains) {
+    constexpr int kSums = decltype(chains)::value;
     f32x4 l4[MT], r4[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
@@ -238,24 +241,25 @@ __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProdu
     for (int t = 0; t < MT; ++t)
       l4[t] = *reinterpret_cast<const f32x4*>(&left_lds[buffer][(wave_m + t * 16 + row) * LD + 4 * group]);
     // the sums of a row of tiles are added up while the next row's products run
-    f32x4 sums[MT][2][2];
+    f32x4 sums[MT][2][kSums];
 #pragma unroll
     for (int t = 0; t <= MT; ++t) {
       if (t < MT) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          sums[t][u][0] = sums[t][u][1] = zero4();
+          sums[t][u][0] = sums[t][u][kSums - 1] = zero4();
           product16(l4[t], r4[u], sums[t][u]);
         }
       }
       if (t > 0) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          total[t - 1][u] += sums[t - 1][u][0] + sums[t - 1][u][1];
+          const auto& sum = sums[t - 1][u];
+          total[t - 1][u] += kSums == 2 ? sum[0] + sum[kSums - 1] : sum[0];
           asm volatile("" : "+v"(total[t - 1][u]));   // added here, not after the next tile's stores
         }
       }
-      if constexpr (kForward) keep_order();
+      if constexpr (kForward || BM == 128) keep_order();
     }
   };
   // The last tile is multiplied after the loop: with its loads under a condition every tile
@@ -264,12 +268,12 @@ __global__ void __launch_bounds__(kBlock, 4) conv_product_kernel(const ConvProdu
   const uint32_t k_last = (a.k - 1) / BK * BK;
   for (uint32_t k0 = 0; k0 < k_last; k0 += BK) {
     load_tile(k0 + BK);
-    multiply(buffer);
+    multiply(buffer, std::integral_constant<int, kChains>());
     store_tile(k0 + BK, buffer ^ 1);
     __syncthreads();
     buffer ^= 1;
   }
-  multiply(buffer);
+  multiply(buffer, std::integral_constant<int, 2>());
 
   auto store_columns = [&](int u, bool whole) {
     const uint32_t out_j = n_tile * BN + wave_n + u * 16 + row;
@@ -457,11 +461,11 @@ __global__ void __launch_bounds__(128 * WM * WN, 2) conv_weight_gradient_kernel(
   }
 }
 
-template <bool kForward>
+template <bool kForward, int kChains>
 void launch_product(hipStream_t s, const ConvProductArgs& a, int bm, dim3 grid) {
-  if (bm == 32) hipLaunchKernelGGL((conv_product_kernel<32, kForward>), grid, dim3(kBlock), 0, s, a);
-  else if (bm == 64) hipLaunchKernelGGL((conv_product_kernel<64, kForward>), grid, dim3(kBlock), 0, s, a);
-  else hipLaunchKernelGGL((conv_product_kernel<128, kForward>), grid, dim3(kBlock), 0, s, a);
+  if (bm == 32) hipLaunchKernelGGL((conv_product_kernel<32, kForward, kChains>), grid, dim3(kBlock), 0, s, a);
+  else if (bm == 64) hipLaunchKernelGGL((conv_product_kernel<64, kForward, kChains>), grid, dim3(kBlock), 0, s, a);
+  else hipLaunchKernelGGL((conv_product_kernel<128, kForward, kChains>), grid, dim3(kBlock), 0, s, a);
 }
 
 // Rows of a tile: as few idle rows as possible, 128 before 64 where both leave the same.
@@ -488,8 +492,12 @@ void conv_product(hipStream_t s, ConvProductArgs a, bool forward) {
   a.units = (uint32_t)conv_product_units(a.m, a.n);
   a.m_tiles_fd = FastDiv((a.m + bm - 1) / bm);
   const dim3 grid((a.units + kXcds - 1) / kXcds * kXcds);
-  if (forward) launch_product<true>(s, a, bm, grid);
-  else launch_product<false>(s, a, bm, grid);
+  // Two chains of eight a tile cost the input gradient's product 4 to 6 % where it has many tiles
+  // ([64, 64, 56, 56] under 64 windows of 3 x 3 206 and 195 us); a sum of few tiles needs them.
+  constexpr uint32_t kFewTerms = 48;
+  if (forward) launch_product<true, 2>(s, a, bm, grid);
+  else if (a.k <= kFewTerms) launch_product<false, 2>(s, a, bm, grid);
+  else launch_product<false, 1>(s, a, bm, grid);
 }
 
 int64_t conv_weight_tiles(int64_t m, int64_t n) {
