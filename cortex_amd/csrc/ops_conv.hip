@@ -522,14 +522,17 @@ void sum_partials(hipStream_t s, T* weight_gradient, const T* partials, int64_t 
 //    piece, the library 7 to 10 ns for a position of an image: [16, 64, 56, 56] under 256 of 1 x 1
 //    (64 blocks of 49 pieces) 83 and 28 us, [16, 64, 28, 28] under 64 of 3 x 3 (144 of 13) 30 and
 //    27; but [1, 64, 56, 56] under 64 (63 of 7) 19 and 24, [3, 15, 109, 109] under 84 (138 of 25)
-//    48 and 96.  Runs of up to four pieces are over before the host has called the library.
-//    Results of up to 32 rows or columns, whose blocks have half the waves, fill
-//    it for images of up to 2048 positions only: [71, 42, 77, 77] under 11 185 and 137 us,
-//    [40, 63, 60, 60] under 4 of 5 x 5 185 and 144; [34, 89, 37, 37] under 5 83 and 121.
+//    48 and 96.  Runs of up to four pieces are over before the host has called the library;
+//  - over long runs of images of more than 2048 positions, where its products are at their best, for
+//    results of up to 32 rows or columns, whose blocks have half the waves ([71, 42, 77, 77] under 11
+//    185 and 137 us, [40, 63, 60, 60] under 4 of 5 x 5 185 and 144; [34, 89, 37, 37] under 5 83 and
+//    121), and for rows off the 16-byte grid, whose loads are split ([34, 30, 57, 57] under 106 of
+//    5 x 5 242 and 220, [113, 32, 49, 49] under 79 284 and 248; [83, 20, 33, 33] under 130, 841
+//    positions, 173 and 248).
 // Rows shorter than a 16-byte load are the library's too.
 bool weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t fit, ConvWeightArgs* args, int64_t* splits) {
   constexpr int64_t kWeightBlocks = 512, kTogether = 3, kManyTiles = 64, kFewWaves = 1400, kPositionsPerPiece = 200,
-                    kShortImage = 400, kNarrowImage = 2048;
+                    kShortImage = 400, kLongImage = 2048;
   ConvWeightArgs a{};
   a.out_image = sh.out_image; a.conv_image = sh.conv_image;
   a.m = (uint32_t)d.out_channels; a.n = (uint32_t)sh.n_cols; a.n_rows = (uint32_t)sh.n_rows;
@@ -546,7 +549,8 @@ bool weight_args(const ct_conv_desc& d, const ConvShape& sh, int64_t fit, ConvWe
   if (sh.n_rows < 4) return false;
   const bool narrow = a.m <= 32 || a.n <= 32;
   if (sh.n_rows > 2 * kConvPiece && run > 1 && (narrow ? tiles / 2 : tiles) > kManyTiles) return false;
-  const bool full = tiles * *splits * conv_weight_waves(a.m, a.n) >= kFewWaves && !(narrow && sh.n_rows > kNarrowImage);
+  const bool full = tiles * *splits * conv_weight_waves(a.m, a.n) >= kFewWaves &&
+                    !((narrow || sh.n_rows % 4 != 0) && sh.n_rows > kLongImage);
   return full || sh.n_rows <= kShortImage || run <= std::max<int64_t>(4, sh.n_rows / kPositionsPerPiece);
 }
 

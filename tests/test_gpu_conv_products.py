@@ -74,7 +74,7 @@ def weight_route(batch, m, n, n_rows):
     narrow = m <= 32 or n <= 32
     if n_rows < 4 or (n_rows > 128 and run > 1 and tiles // (2 if narrow else 1) > 64):
         return "gemm+conv_sum_partials"
-    if n_rows > 400 and (waves < 1400 or narrow and n_rows > 2048) and run > max(4, n_rows // 200):
+    if n_rows > 400 and (waves < 1400 or (narrow or n_rows % 4) and n_rows > 2048) and run > max(4, n_rows // 200):
         return "gemm+conv_sum_partials"
     return "conv_weight_gradient" + ("+conv_sum_partials" if splits > 1 else "")
 
@@ -117,6 +117,8 @@ WEIGHT_CASES = [
     (2, 60, 3, 48, 48, 3, 3, 1, 1),     # 36 splits of two pieces of images of 2304 positions, few rows
     (5, 200, 3, 48, 48, 3, 3, 1, 1),    # the same with fourteen: the library
     (4, 16, 10, 60, 60, 3, 3, 1, 1),    # four of 3600
+    (200, 5, 40, 46, 46, 3, 3, 1, 1),   # 200 splits of 34 pieces of images of 2116 positions
+    (200, 5, 40, 47, 47, 3, 3, 1, 1),   # of 2209, off the 16-byte grid: the library
     (1, 64, 64, 56, 56, 3, 3, 1, 1),    # seven splits of seven pieces of one image
     (6, 200, 128, 11, 9, 1, 1, 0, 1),   # six splits of two pieces, an image each
     (7, 160, 128, 11, 9, 3, 3, 1, 1),   # seven partial products of 46 tiles
