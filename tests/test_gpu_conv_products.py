@@ -97,7 +97,7 @@ def data_route(batch, m, k, n_rows):
     tiles = tiles_of(m, n)
     if k <= 64 or (k <= 160 and tiles < 256):
         ours = True
-    elif k <= 256 and m >= 192 and 500 <= n_rows <= 4096:
+    elif m >= 192 and (500 if k <= 256 else 1000) <= n_rows <= 4096:
         ours = False
     else:
         ours = tiles >= (400 if m <= 96 else 768) or (n_rows <= 128 and tiles >= 250)
@@ -145,6 +145,8 @@ DATA_CASES = [
     (32, 112, 70, 8, 8, 3, 3, 1, 1),    # 256, images of 64 positions
     (32, 112, 70, 12, 11, 3, 3, 1, 1),  # 528, of 132: the library
     (17, 25, 65, 25, 24, 3, 3, 1, 1),   # 225 cells, 600 positions: the library
+    (26, 22, 260, 27, 37, 3, 3, 1, 1),  # 782 tiles of 198 cells over 260 out channels, 999 positions
+    (26, 22, 260, 25, 40, 3, 3, 1, 1),  # of 1000: the library
 ]
 
 
