@@ -382,7 +382,7 @@ bool forward_product(const ct_conv_desc& d, const ConvShape& sh) {
 // depend on more than the sizes (20 to 110 TFLOP/s for products of one size).  The lines below are
 // drawn through 310 shapes; its time is the second.
 //  - k up to 64: from 0.7 to 5 times the library's speed ([69, 6, 71, 71] under 38 34 and 130,
-//    [64, 64, 56, 56] under 64 195 and 230; the worst are [16, 64, 28, 28] under 64 of 3 x 3 22 and 17,
+//    [64, 64, 56, 56] under 64 207 and 225; the worst are [16, 64, 28, 28] under 64 of 3 x 3 22 and 17,
 //    [37, 58, 56, 56] under 24 77 and 53, [64, 256, 56, 56] under 64 of 1 x 1 101 and 88).
 //  - Few tiles: k up to 160 ([9, 10, 15, 15] under 102 10.0 and 7.2 us, calls 13.7 and 16.1; k 256,
 //    [1, 128, 28, 28] under 256 of 1 x 1, 17.8 and 4.1, calls 20.4 and 15.7).
@@ -392,14 +392,15 @@ bool forward_product(const ct_conv_desc& d, const ConvShape& sh) {
 //    positions, where the library runs at 80 to 110 TFLOP/s: [64, 128, 28, 28] under 128 177 and 147,
 //    [98, 26, 46, 46] under 164 209 and 175.  Beyond 256 channels that holds from 1000 positions on
 //    (117 shapes of 1600 and 3136, 2 to 64 images, 300 to 512 channels, roll back included: 0.86 to
-//    1.32 times the library's time, above 1 in 106; [16, 64, 56, 56] under 512 302 and 257); below,
-//    [16, 64, 28, 28] under 384 takes 72 and 103, [8, 512, 28, 28] under 512 340 and 313 and
-//    [16, 64, 28, 28] under 300 66 and 58.
+//    1.32 times the library's time, above 1 in 106; [16, 64, 56, 56] under 512 302 and 257), and over
+//    3000 cells or more throughout ([32, 512, 28, 28] under 512 1195 and 1067, [8, 384, 28, 28] under
+//    384 201 and 186, [4, 448, 28, 28] under 448 156 and 125); else, [16, 64, 28, 28] under 384 takes
+//    72 and 103, [16, 320, 28, 28] under 320 280 and 430, but [16, 64, 28, 28] under 300 66 and 58.
 bool backward_data_product(const ct_conv_desc& d, const ConvShape& sh) {
   const int64_t m = sh.n_cols, k = d.out_channels, n_rows = sh.n_rows, tiles = conv_product_units(m, sh.batch * n_rows);
   if (sh.conv_image == 0 || n_rows > conv_product_positions(m)) return false;
   if (k <= 64 || (k <= 160 && tiles < 256)) return true;
-  if (m >= 192 && n_rows >= (k <= 256 ? 500 : 1000) && n_rows <= 4096) return false;
+  if (m >= 192 && n_rows >= (k <= 256 || m >= 3000 ? 500 : 1000) && n_rows <= 4096) return false;
   return tiles >= (m <= 96 ? 400 : 768) || (n_rows <= 128 && tiles >= 250);
 }
 

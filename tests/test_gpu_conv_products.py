@@ -97,7 +97,7 @@ def data_route(batch, m, k, n_rows):
     tiles = tiles_of(m, n)
     if k <= 64 or (k <= 160 and tiles < 256):
         ours = True
-    elif m >= 192 and (500 if k <= 256 else 1000) <= n_rows <= 4096:
+    elif m >= 192 and (500 if k <= 256 or m >= 3000 else 1000) <= n_rows <= 4096:
         ours = False
     else:
         ours = tiles >= (400 if m <= 96 else 768) or (n_rows <= 128 and tiles >= 250)
@@ -147,6 +147,8 @@ DATA_CASES = [
     (17, 25, 65, 25, 24, 3, 3, 1, 1),   # 225 cells, 600 positions: the library
     (26, 22, 260, 27, 37, 3, 3, 1, 1),  # 782 tiles of 198 cells over 260 out channels, 999 positions
     (26, 22, 260, 25, 40, 3, 3, 1, 1),  # of 1000: the library
+    (5, 333, 260, 25, 20, 3, 3, 1, 1),  # 940 tiles of 2997 cells, 500 positions
+    (5, 334, 260, 25, 20, 3, 3, 1, 1),  # of 3006: the library
 ]
 
 
