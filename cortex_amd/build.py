@@ -40,6 +40,7 @@ SOURCES = [
     "ops_batchnorm.hip",
     "ops_rand.hip",
     "ops_blas.cpp",
+    "ops_gemm.hip",
     "ops_gemv.hip", "ops_pool.hip", "ops_conv.hip", "ops_conv_mfma.hip", "ops_lrn.hip",
 ]
 

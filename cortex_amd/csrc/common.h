@@ -26,6 +26,9 @@ bool debug_sync();
 // slot; a call that needs two live temporaries uses two slots.
 enum ScratchSlot { kScratchReduce = 0, kScratchAccumA = 1, kScratchAccumB = 2, kScratchSlots = 3 };
 int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot = kScratchReduce);
+// The same where the caller can do without: null, and no error, if the block is too small and cannot grow, for want of memory
+// or because the stream is being captured.
+void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot = kScratchReduce);
 void release_stream_scratch(hipStream_t s);
 
 inline void note_kernel(const char* name) { *last_kernel_slot() = name; }

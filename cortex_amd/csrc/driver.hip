@@ -57,6 +57,36 @@ int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot) {
   return CT_OK;
 }
 
+void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  ScratchBlock& b = g_scratch[ScratchKey{dev, s, slot}];
+  if (b.bytes >= bytes) return b.ptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+  void* grown = nullptr;
+  if (hipMalloc(&grown, want) != hipSuccess) {   // the block stays what it was
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (b.ptr) {
+    // earlier kernels of this stream may still be reading the old block
+    if (hipStreamSynchronize(s) != hipSuccess) {
+      (void)hipFree(grown);
+      return nullptr;   // the error is the stream's and stays with it
+    }
+    (void)hipFree(b.ptr);
+  }
+  b.ptr = grown;
+  b.bytes = want;
+  return grown;
+}
+
 void release_stream_scratch(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return;

@@ -1,9 +1,7 @@
-// ops_blas.cpp -- gemm! (src/cortex/tensor/math.clj:106-114) on rocBLAS.  It is
-// a plain library matrix product (the reference's backends call netlib BLAS and
-// cuBLAS for it, src/cortex/compute/cpu/tensor_math.clj:672-726,
-// src/cortex/compute/cuda/tensor_math.clj:633-660), so the vendor library's MFMA
-// kernels are the right tool; nothing is hand-written here.  gemv!, which is
-// bound by memory rather than by the matrix cores, lives in ops_gemv.hip.
+// ops_blas.cpp -- gemm! (src/cortex/tensor/math.clj:106-114).  Float products go to the kernels of ops_gemm.hip; double
+// ones, and the few shapes of float that are faster here, to rocBLAS (the reference's backends call netlib BLAS and
+// cuBLAS, src/cortex/compute/cpu/tensor_math.clj:672-726, src/cortex/compute/cuda/tensor_math.clj:633-660).  gemv!, which
+// is bound by memory rather than by the matrix cores, lives in ops_gemv.hip.
 //
 // The tensors are row-major and BLAS is column-major: a row-major matrix with
 // row pitch ld is the column-major matrix of its transpose with leading
@@ -22,6 +20,7 @@
 #include <thread>
 
 #include "common.h"
+#include "gemm.h"
 
 using namespace cthip;
 
@@ -179,6 +178,11 @@ int ct_gemm(void* stream, void* c, int64_t c_colstride, int trans_a, int trans_b
   CT_REQUIRE(a_colstride >= (trans_a ? a_row_count : a_col_count), "ct_gemm: A column stride is shorter than its rows");
   CT_REQUIRE(b_colstride >= (trans_b ? a_col_count : b_col_count), "ct_gemm: B column stride is shorter than its rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == CT_F32) {
+    const GemmProduct p{(const float*)a, (const float*)b, (float*)c, a_colstride, b_colstride, c_colstride, 0, 0, 0, a_row_count,
+                        b_col_count, a_col_count, 1, !trans_a, trans_b != 0, (float)alpha, (float)beta};
+    if (gemm_split_takes(p)) return gemm_split(s, p);
+  }
   RocblasApi* api;
   rocblas_handle h;
   if (int rc = blas_handle(s, &api, &h)) return rc;

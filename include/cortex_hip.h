@@ -337,8 +337,13 @@ int ct_softmax_spatial(void* stream, void* output, const ct_dims* output_dims, c
  *   C[a_row_count, b_col_count] = alpha * op(A) * op(B) + beta * C,
  * op(A) is [a_row_count, a_col_count], op(B) is [a_col_count, b_col_count]
  * (the counts are taken after the transposition, src/cortex/tensor.clj:920-951);
- * a column stride is the distance in elements between two stored rows.  Runs on
- * rocBLAS, loaded on first use.  dtype is CT_F32 or CT_F64. */
+ * a column stride is the distance in elements between two stored rows.  Float
+ * products run on the library's own kernels (operands held exactly, sums in float),
+ * double ones and some shapes of float on rocBLAS, loaded on first use.  A float
+ * product of few results over a long sum keeps partial sums in the stream's
+ * scratch memory, up to 256 MiB, where there is room or it can grow (not while the
+ * stream is being captured), and does without otherwise.  dtype is CT_F32 or
+ * CT_F64. */
 int ct_gemm(void* stream, void* c, int64_t c_colstride, int trans_a, int trans_b, double alpha,
             const void* a, int64_t a_row_count, int64_t a_col_count, int64_t a_colstride,
             const void* b, int64_t b_col_count, int64_t b_colstride, double beta, int dtype);

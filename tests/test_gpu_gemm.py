@@ -1,0 +1,118 @@
+"""gemm! of float matrices at the edges of its tiles and of its number range, against the CPU oracle."""
+import numpy as np
+import pytest
+
+import harness as H
+from harness import View
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def P(pair_factory):
+    with pair_factory() as pair:
+        yield pair
+
+
+def run(P, a, b, c, ta, tb, m, n, k, alpha=1.0, beta=0.0):
+    """c [m, ldc] = alpha * op(a) op(b) + beta * c on both sides; the kernels that ran, the result, the oracle's."""
+    ba, bb, bc = P.buf(a), P.buf(b), P.buf(c)
+    va, vb, vc = (View(x, [x.init.size]) for x in (ba, bb, bc))
+    kernel = P.run(H.gemm, vc, c.shape[1], ta, tb, alpha, va, m, k, a.shape[1], vb, n, b.shape[1], beta)
+    return kernel, bc.download().reshape(c.shape), bc.host.reshape(c.shape)
+
+
+def operands(make, m, n, k, ta, tb, pad=0):
+    return (make((k, m + pad) if ta else (m, k + pad)), make((n, k + pad) if tb else (k, n + pad)), make((m, n + pad)))
+
+
+# tiles are 32, 64 or 128 a side and hold 32 k, in pairs; sixteen waves of the small kernel take 512 k between them
+EDGES = [(1, 1, 1), (3, 2, 5), (31, 33, 31), (32, 32, 32), (33, 31, 33), (64, 65, 63), (63, 64, 65), (130, 60, 97), (65, 40, 512),
+         (40, 65, 513), (5, 7, 545), (10, 128, 1100), (700, 520, 40), (513, 700, 33), (770, 1030, 66), (513, 385, 700),
+         (1040, 1025, 129), (1025, 1040, 290), (2050, 1100, 130), (300, 500, 1100), (130, 70, 3000), (1152, 1030, 550)]
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("size", EDGES, ids=str)
+def test_whole_numbers_are_exact(P, size, ta, tb):
+    """Whole numbers whose sums stay below 2^24: every product and sum is exact in any order."""
+    m, n, k = size
+    rng = np.random.default_rng(m + n + k)
+    a, b, c = operands(lambda s: rng.integers(-7, 8, s).astype(np.float32), m, n, k, ta, tb, pad=(m + k) % 3)
+    for alpha, beta in ((1.0, 0.0), (2.0, -1.0)):
+        kernel, got, want = run(P, a, b, c, ta, tb, m, n, k, alpha, beta)
+        assert kernel.startswith("gemm_"), kernel
+        H.assert_bit_exact(got, want, f"{size} ta={ta} tb={tb} alpha={alpha} ({kernel})")
+
+
+KERNELS = {(40, 40, 100): "gemm_small", (10, 20, 3700): "gemm_medium_pair+gemm_sum", (640, 640, 50): "gemm_medium",
+           (900, 900, 400): "gemm_medium_pair", (2048, 2048, 256): "gemm_large", (64, 2048, 4096): "gemm_medium_pair+gemm_sum",
+           (1024, 1536, 2048): "gemm_large+gemm_sum", (2000, 2000, 20): "rocblas_gemm"}
+
+
+@pytest.mark.parametrize("size", KERNELS, ids=str)
+def test_error_is_below_a_plain_sum_s(P, size):
+    """The 2-norm of the error against 64 bits stays below that of the plain float sum, rounded after every product; the
+    kernel that ran is the one that the sizes call for.  The plain sum rounds k times at the size of the sum so far; the
+    large products here once for 16 k, the five small ones, 2^-8 of them, as often each, and what is left out is 2^-25 of
+    a product: a sixteenth of the roundings and a quarter of the error, of which half is asked for."""
+    m, n, k = size
+    rng = np.random.default_rng(k)
+    a, b, c = operands(lambda s: rng.standard_normal(s).astype(np.float32), m, n, k, False, True)
+    kernel, got, _ = run(P, a, b, c, False, True, m, n, k)
+    assert kernel == KERNELS[size], kernel
+    some = slice(0, 10)   # of the rows: two hundred sums or more
+    a64, b64 = a[some].astype(np.float64), b.astype(np.float64)
+    exact, plain = a64 @ b64.T, np.zeros((len(a64), n), np.float32)
+    for i in range(k):
+        plain = (plain + a64[:, i, None] * b64[None, :, i]).astype(np.float32)
+    if kernel != "rocblas_gemm":
+        assert np.linalg.norm(got[some] - exact) <= 0.5 * np.linalg.norm(plain - exact)
+
+
+@pytest.mark.parametrize("size", [(40, 50, 100), (640, 640, 50), (900, 900, 400), (2048, 2048, 256), (64, 2048, 4096)], ids=str)
+def test_the_ends_of_the_number_range(P, size):
+    """Infinities, NaN, and floats and results beyond what the pieces hold: the block forms its sums again from the floats.
+    The oracle sums in double and rounds once; bar: 1e-5 of the sum of magnitudes and, where that is
+    denormal, half of the least float for each of the k products, which are rounded to multiples of it; classes alike."""
+    m, n, k = size
+    rng = np.random.default_rng(m)
+    a, b, c = operands(lambda s: rng.standard_normal(s).astype(np.float32), m, n, k, False, True)
+    a[1, 3], a[2, k - 1], a[3, 0], a[4, 5], a[5, :] = np.inf, -np.inf, np.nan, 3e38, 1e-42
+    a[6, :] = 1e-30
+    b[2, :], b[3, 1], b[4, :] = 0.0, 1e37, 1e38
+    a[7, :] *= 1e20
+    b[6, :] *= 1e18
+    kernel, got, want = run(P, a, b, c, False, True, m, n, k)
+    scale = np.abs(np.where(np.isfinite(a), a, 0).astype(np.float64)) @ np.abs(b.astype(np.float64)).T
+    sure = scale <= 1e38   # sums of finite products that come near the largest float may pass it on the way
+    special = ~np.isfinite(want)
+    assert np.array_equal(np.isnan(got)[sure], np.isnan(want)[sure]), kernel
+    assert np.array_equal(got[sure & special & ~np.isnan(want)], want[sure & special & ~np.isnan(want)]), kernel
+    fine = sure & ~special
+    assert np.all(np.abs(got[fine].astype(np.float64) - want[fine]) <= 1e-5 * scale[fine] + k * 2.0 ** -150), kernel
+
+
+@pytest.mark.parametrize("exponent", [-135, -100, 60])
+def test_scaled_operands_scale_the_result(P, exponent):
+    """Multiplying an operand by a power of two multiplies the result, to the bit, as long as neither leaves the floats:
+    also where the operand's last bits are denormal (whole numbers below 2^8 keep them)."""
+    m, n, k = 70, 50, 90
+    rng = np.random.default_rng(7)
+    a, b, c = operands(lambda s: rng.integers(-120, 121, s).astype(np.float32), m, n, k, False, True)
+    _, want, _ = run(P, a, b, c, False, True, m, n, k)
+    kernel, got, _ = run(P, np.ldexp(a, exponent).astype(np.float32), b, c, False, True, m, n, k)
+    H.assert_bit_exact(got, np.ldexp(want, exponent).astype(np.float32), kernel)
+
+
+def test_a_result_over_its_own_operand_is_the_library_s(P):
+    m = 48
+    rng = np.random.default_rng(8)
+    a = P.buf(rng.integers(-4, 5, m * m).astype(np.float32))
+    b, c = P.buf(rng.integers(-4, 5, m * m).astype(np.float32)), P.buf(np.zeros(2 * m * m, np.float32))
+    v = lambda x: View(x, [x.init.size])
+    assert P.run(H.gemm, v(c), m, False, False, 1.0, v(a), m, m, m, v(b), m, m, 0.0) == "gemm_small"
+    H.gemm(P.hip, v(a), m, False, False, 1.0, v(a), m, m, m, v(b), m, m, 0.0)
+    from cortex_amd import capi
+    assert capi.last_kernel() == "rocblas_gemm"
