@@ -18,17 +18,23 @@ struct ConvProductArgs {
   float* output;
   float* workspace;
   int64_t in_image, out_image, conv_image;
-  uint32_t m, n, k, n_rows;
+  uint32_t m, n, k, n_rows, images;   // n = images * n_rows
   uint32_t in_plane, in_h, in_w, kw, kh;
   int32_t px, py, sx, sy;
   float beta;
-  uint32_t units;
+  uint32_t units, rows_per_block;
   FastDiv m_tiles_fd, rows_fd, out_w_fd, taps_fd, kw_fd;
 };
 void conv_product(hipStream_t s, ConvProductArgs a, bool forward);
 // The tiles that such a product has, and the positions that one launch of it may have.
 int64_t conv_product_units(int64_t m, int64_t n);
 int64_t conv_product_positions(int64_t m);
+
+// The same on the bfloat16 matrix cores, and whether a product is faster there (n positions in all); a launch may have so
+// many positions, and its buffers must stay below 2^31 bytes, the input's with the padding in front of its first image.
+bool conv_product_splits(int64_t m, int64_t n, int64_t k, bool forward);
+int64_t conv_split_positions(int64_t m);
+void conv_product_split(hipStream_t s, ConvProductArgs a, bool forward);
 
 // The positions of a piece, the unit in which the weight gradient's sum is split.
 constexpr int kConvPiece = 64;

@@ -195,7 +195,8 @@ __global__ void __launch_bounds__(kBlock) conv_roll_unit_stride_kernel(const Con
 template <class T, int KW, int KH>
 __global__ void __launch_bounds__(kBlock) conv_roll_unit_stride_pieces_kernel(const ConvArgs a) {
   constexpr int VEC = 16 / sizeof(T);
-  const uint32_t lane = blockIdx.x * kBlock + threadIdx.x;
+  // from the end on: what the product stored last is still in the last-level cache
+  const uint32_t lane = (gridDim.x - 1 - blockIdx.x) * kBlock + threadIdx.x;
   if (lane >= a.total) return;
   const uint32_t e0 = lane * VEC;
   uint32_t image, rest, chan, r, iy, ix;
@@ -404,6 +405,15 @@ bool backward_data_product(const ct_conv_desc& d, const ConvShape& sh) {
   return tiles >= (m <= 96 ? 400 : 768) || (n_rows <= 128 && tiles >= 250);
 }
 
+// Images of one launch of a product on the bfloat16 matrix cores, which indexes its buffers in bytes below 2^31; none if one
+// image by itself is too large.
+int64_t images_of_a_split(const ct_conv_desc& d, const ConvShape& sh, int64_t m) {
+  constexpr int64_t kMostFloats = (int64_t(1) << 29) - 1;
+  const int64_t padding = (int64_t)d.pad_y * sh.in_w + d.pad_x, largest = std::max({sh.in_image, sh.out_image, sh.conv_image});
+  if (largest + padding > kMostFloats) return 0;
+  return std::min((kMostFloats - padding) / largest, conv_split_positions(m) / sh.n_rows);
+}
+
 void run_product(hipStream_t s, float* output, float beta, const float* input, const float* weights, float* workspace,
                  const ct_conv_desc& d, const ConvShape& sh, bool forward) {
   ConvProductArgs a{};
@@ -421,14 +431,18 @@ void run_product(hipStream_t s, float* output, float beta, const float* input, c
   a.out_w_fd = FastDiv((uint32_t)sh.out_w);
   a.taps_fd = FastDiv((uint32_t)(d.kernel_width * d.kernel_height));
   a.kw_fd = FastDiv((uint32_t)d.kernel_width);
-  const int64_t step = std::max<int64_t>(1, conv_product_positions(a.m) / sh.n_rows);
+  int64_t step = std::max<int64_t>(1, conv_product_positions(a.m) / sh.n_rows);
+  const bool split = conv_product_splits(a.m, sh.batch * sh.n_rows, a.k, forward) && images_of_a_split(d, sh, a.m) > 0;
+  if (split) step = std::min(step, images_of_a_split(d, sh, a.m));
   for (int64_t b0 = 0; b0 < sh.batch; b0 += step) {
     const int64_t nb = std::min(step, sh.batch - b0);
     a.input = forward ? input + b0 * sh.in_image : nullptr;
     a.output = output + b0 * sh.out_image;
     a.workspace = workspace + b0 * sh.conv_image;
+    a.images = (uint32_t)nb;
     a.n = (uint32_t)(nb * sh.n_rows);
-    conv_product(s, a, forward);
+    if (split) conv_product_split(s, a, forward);
+    else conv_product(s, a, forward);
   }
 }
 

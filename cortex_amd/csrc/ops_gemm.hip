@@ -28,13 +28,6 @@ namespace {
 // consecutive rows' reads of one chunk cover 128 bytes' worth of banks once.
 __device__ __forceinline__ uint32_t tile_at(uint32_t row, uint32_t chunk) { return row * 32 + ((chunk ^ (row >> 1)) & 3) * 8; }
 
-__device__ __forceinline__ f32x16 zero16() {
-  f32x16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
-}
-
 struct GemmArgs {
   const float* a;
   const float* b;

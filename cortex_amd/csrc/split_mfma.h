@@ -73,6 +73,13 @@ __device__ __forceinline__ void split4(f32x4 x, u32x4 (&pieces)[kSplitPieces], i
   }
 }
 
+__device__ __forceinline__ f32x16 zero16() {
+  f32x16 z;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.f;
+  return z;
+}
+
 __device__ __forceinline__ bool not_finite(float x) { return (__builtin_bit_cast(uint32_t, x) & 0x7f800000u) == 0x7f800000u; }
 
 }  // namespace cthip

@@ -306,3 +306,63 @@ def test_weight_gradient_over_its_own_operand(P):
     gradient = both.init[:cout * n_rows].reshape(cout, n_rows).astype(np.float64)
     unrolled = work.download().reshape(n_cols, n_rows).astype(np.float64)
     H.assert_bit_exact(both.download(), (gradient @ unrolled.T).astype(np.float32).reshape(-1), "convolution-backward-weights")
+
+
+# (batch, in channels, out channels, side, window, stride): the float products that are formed in three pieces to a float: 64
+# cells or more over 288 blocks of 256 positions; 20 to 64 out channels over 128 rows or more; more than 64; runs of six
+# pieces of positions or more.  Remainders of 32 cells, 32 rows, 16 channels and 256 positions.
+SPLIT_CASES = [
+    (46, 8, 33, 40, 3, 1),      # 72 cells, 288 blocks, images of 1600 positions: a block spans two
+    (150, 7, 64, 23, 3, 1),     # 63 cells: the float kernel; 310 blocks of 79350 positions
+    (150, 11, 65, 23, 3, 1),    # 99 cells: the last tile of three; 65 rows: two tiles
+    (30, 4, 31, 50, 5, 1),      # 100 cells of 25 taps, one tile of rows, 294 blocks
+    (41, 15, 20, 40, 3, 1),     # 135 rows over 20 channels and 65600 positions
+    (40, 15, 20, 40, 3, 1),     # 64000 positions: the float kernel
+    (7, 57, 33, 36, 3, 1),      # 513 rows over 33 channels and 9072 positions, in several runs of rows
+    (2, 57, 64, 68, 3, 1),      # 9248 positions, 64 channels
+    (3, 33, 66, 20, 1, 1),      # 33 rows over 66 channels
+    (5, 20, 200, 19, 3, 2),     # 180 rows over 200
+    (6, 15, 129, 33, 3, 1),     # 135 rows over 129 channels, weight gradient over six long runs
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_products_in_pieces_at_the_edges_of_their_tiles(P, case):
+    batch, cin, cout, side, k, stride = case
+    check_products(P, batch, cin, cout, side, side, k, k, k // 2, k // 2, stride, stride)
+
+
+@pytest.mark.parametrize("case", [(46, 8, 33, 40, 3), (41, 15, 20, 40, 3), (5, 20, 200, 19, 3)], ids=lambda c: "x".join(map(str, c)))
+def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
+    """An infinity, a NaN and floats that the pieces do not hold, in the weights and in both gradients' operands: the blocks
+    that meet them form their sums again from the floats.  Where the oracle's sums are finite the bar is 1e-5 of the sums of
+    magnitudes; elsewhere the classes agree."""
+    batch, cin, cout, side, k = case
+    n_rows, n_cols = side * side, cin * k * k
+    desc, geometry = H.conv_desc(cin, cout, k, k, k // 2, k // 2, 1, 1), (batch, side, side, side, side)
+    rng = np.random.default_rng(cin)
+    normal = lambda n: rng.standard_normal(n).astype(np.float32)
+    x, w, g = normal(batch * cin * n_rows), normal(cout * n_cols), normal(batch * cout * n_rows)
+    x[5], x[7 * n_rows + 3], w[3], w[n_cols + 1], g[11], g[2 * n_rows + 1] = np.inf, 1e35, np.nan, -1e36, -np.inf, 3e35
+    inp, weights, og = P.buf(x), P.buf(w), P.buf(g)
+    out, wg, ig = P.buf(normal(batch * cout * n_rows)), P.buf(normal(cout * n_cols)), P.buf(normal(batch * cin * n_rows))
+    work = P.buf(np.zeros(batch * n_rows * n_cols, np.float32))
+    clean = lambda v: np.abs(np.where(np.isfinite(v) & (np.abs(v) < 1e30), v, 0)).max()
+
+    def check(buf, scale, what):
+        got, want = buf.download().astype(np.float64), buf.host.astype(np.float64)
+        plain = np.isfinite(want) & (np.abs(want) < 1e30)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), what
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]), what
+        big = np.isfinite(want) & ~plain
+        assert np.all(np.abs(got[big] - want[big]) <= 1e-5 * np.abs(want[big])), what
+        assert np.all(np.abs(got[plain] - want[plain]) <= 1e-5 * scale), what
+        assert not np.all(np.isnan(want)) and plain.any(), what
+
+    P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    check(out, clean(x) * clean(w) * n_cols, "convolution-forward")
+    P.run(H.convolution, "backward_weights", vec(wg), 0.0, vec(og), vec(inp), vec(work), desc, *geometry)
+    got, want = wg.download(), wg.host
+    assert np.array_equal(np.isnan(got), np.isnan(want)), "convolution-backward-weights"
+    P.run(H.convolution, "backward_data", vec(ig), 0.0, vec(og), vec(weights), vec(work), desc, *geometry)
+    check(ig, clean(g) * clean(w) * cout * k * k, "convolution-backward-data")
