@@ -10,6 +10,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -108,9 +109,30 @@ def _compile(src: str, force: bool) -> Path:
     return obj
 
 
+FRONT = HERE / f"_front{sysconfig.get_config_var('EXT_SUFFIX')}"
+
+
+def _build_front(force: bool) -> None:
+    """The native half of the Python front end (csrc/front.cpp), for the interpreter that runs this."""
+    src, header = CSRC / "front.cpp", HERE.parent / "include" / "cortex_hip.h"
+    if not force and FRONT.exists() and FRONT.stat().st_mtime >= max(src.stat().st_mtime, header.stat().st_mtime):
+        return
+    include = sysconfig.get_paths()["include"]
+    if not (Path(include) / "Python.h").exists():
+        sys.stderr.write(f"{include}/Python.h is missing: the front end stays in Python\n")
+        return
+    fresh = FRONT.with_suffix(".tmp")     # this process may have the old one loaded
+    cmd = ["g++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", f"-I{include}", str(src), "-o", str(fresh)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {src.name}:\n{res.stderr}")
+    fresh.replace(FRONT)
+
+
 def build(force: bool = True, jobs: int | None = None) -> Path:
     """Compiles every source and links the shared library; returns its path."""
     jobs = jobs or min(8, os.cpu_count() or 1)
+    _build_front(force)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(lambda s: _compile(s, force), SOURCES))
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)]

@@ -194,6 +194,12 @@ def load_library(path: Optional[Path] = None) -> C.CDLL:
     return lib
 
 
+try:
+    from . import _front as front
+except ImportError:     # not built: calls go through ctypes
+    front = None
+
+
 _lib: Optional[C.CDLL] = None
 
 
@@ -201,6 +207,9 @@ def lib() -> C.CDLL:
     global _lib
     if _lib is None:
         _lib = load_library()
+        if front is not None:
+            for name in PROTOTYPES:
+                front.bind(name, C.cast(getattr(_lib, name), C.c_void_p).value)
     return _lib
 
 
@@ -210,10 +219,18 @@ def check(status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    """Calls entry point ``name`` and raises on a non-zero status."""
+    """Calls entry point ``name`` and raises on a non-zero status.  A ``ct_dims`` may also be given as its bytes."""
+    if bytes in map(type, args):
+        args = [C.byref(CtDims.from_buffer_copy(a)) if type(a) is bytes else a for a in args]
     status = getattr(_lib or lib(), name)(*args)
     if status != 0:
         check(status)
+
+
+if front is not None:
+    # In native code (csrc/front.cpp) for the entry points that a training step is made of, once the library is loaded;
+    # other calls, and arguments that only ctypes converts, go through the function above.
+    call = front.stand_in(call, check)
 
 
 def last_kernel() -> str:

@@ -20,11 +20,19 @@ Shapes that change all the time gain nothing from the tables and pay for their
 entries, so the packed tensors among them are worked out without the general
 algebra (seven functions of a shape never seen: 38 us without tables, 45 with
 tables in front of the general algebra, 15 now; of a shape seen before 7).
+Where ``csrc/front.cpp`` is built it answers for plain ints in place of the
+tables, which are then reached only by what it hands on; the figures above are
+of the Python functions.
 """
 from __future__ import annotations
 
 from functools import lru_cache
 from typing import List, Optional, Sequence
+
+try:
+    from . import _front as front
+except ImportError:     # not built: everything below works without it
+    front = None
 
 _CACHE_LIMIT = 4096
 
@@ -417,6 +425,20 @@ def as_matrix(dims, to_shape) -> dict:
     return {"shape": list(shp), "strides": list(strides)}
 
 
+def as_2d(dims) -> dict:
+    return as_matrix(dims, to_2d_shape)
+
+
+def as_batch(dims) -> dict:
+    return as_matrix(dims, to_batch_shape)
+
+
+def commensurate_dims(*args) -> bool:
+    """Whether the dimensions are plain ints and every one divides the largest: what is not is for the general rules."""
+    key = direct_key(*args)
+    return key is not None and commensurate(key)
+
+
 def transpose(dims, reorder_vec: Sequence[int]) -> dict:
     """``transpose`` (:473-484): permutes shape and strides; no data moves."""
     shp, strides = dims["shape"], dims["strides"]
@@ -477,3 +499,12 @@ def select(dims, *args) -> dict:
     new_strides = list(reversed([st for _, st in kept]))
     new_shape = list(reversed([len(a) if isinstance(a, (list, range)) else a for a, _ in kept]))
     return {"dimensions": {"shape": new_shape, "strides": new_strides}, "elem-offset": elem_addr}
+
+
+if front is not None:
+    # The same functions in native code (csrc/front.cpp) where every entry is a plain int; they hand on to the ones above
+    # what is not.  A bias over 128 x 784 from Python: 6.4 us a call, 9.1 without; a digit network's training step: 170, 241.
+    direct_key, ecount, shape, dense, access_increasing, dimension_seq_to_max_shape, commensurate_dims, to_2d_shape, \
+        to_batch_shape, as_2d, as_batch = (front.stand_in(f) for f in (
+            direct_key, ecount, shape, dense, access_increasing, dimension_seq_to_max_shape, commensurate_dims, to_2d_shape,
+            to_batch_shape, as_2d, as_batch))

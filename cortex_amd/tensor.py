@@ -39,17 +39,23 @@ class TensorError(ValueError):
     """Stands in for the ``ex-info`` of ``when-not-error``."""
 
 
-@contextlib.contextmanager
-def tensor_context(stream, datatype: str = "double"):
+class tensor_context(contextlib.ContextDecorator):
     """Binds ``*stream*`` and ``*datatype*`` (``tensor.clj:89-111``;
     ``src/cortex/verify/tensor.clj:11-17``)."""
-    t1 = _stream.set(stream)
-    t2 = _datatype.set(datatype)
-    try:
-        yield stream
-    finally:
-        _stream.reset(t1)
-        _datatype.reset(t2)
+
+    def __init__(self, stream, datatype: str = "double"):
+        self.stream, self.datatype = stream, datatype
+
+    def _recreate_cm(self):
+        return tensor_context(self.stream, self.datatype)
+
+    def __enter__(self):
+        self._tokens = _stream.set(self.stream), _datatype.set(self.datatype)
+        return self.stream
+
+    def __exit__(self, *exc):
+        _stream.reset(self._tokens[0])
+        _datatype.reset(self._tokens[1])
 
 
 def check_stream():
@@ -200,11 +206,11 @@ def to_vector(t: Tensor) -> Tensor:
 
 
 def as_2d_matrix(t: Tensor) -> Tensor:
-    return t._with(dimensions=dims.as_matrix(t.dimensions, dims.to_2d_shape))
+    return Tensor(t.device, dims.as_2d(t.dimensions), t.buffer)
 
 
 def as_batch_matrix(t: Tensor) -> Tensor:
-    return t._with(dimensions=dims.as_matrix(t.dimensions, dims.to_batch_shape))
+    return Tensor(t.device, dims.as_batch(t.dimensions), t.buffer)
 
 
 def transpose(t: Tensor, reorder_vec) -> Tensor:
@@ -274,8 +280,7 @@ def _check_partial_alias(*args) -> None:
 def _ensure_broadcast_rules(*args) -> None:
     """``ensure-broadcast-rules`` (``tensor.clj:592-604``): every operand
     dimension must divide the max dimension."""
-    key = dims.direct_key(*[a.dimensions for a in args])
-    if key is not None and dims.commensurate(key):
+    if dims.commensurate_dims(*[a.dimensions for a in args]):
         return
     info = dims.dimension_seq_to_max_shape(*[a.dimensions for a in args])
     max_shape = info["max-shape"]
