@@ -32,13 +32,15 @@
 // the remaining axes) applies that destination element's updates in increasing
 // position, which is increasing e: accum_grouped_kernel.  Bit-identical to the
 // serial loop for every op.  Up to 8192 index entries are ranked by one small
-// kernel; longer index tensors go through the vendor sort (rocPRIM's
-// radix_sort_pairs, stable, the positions fed from a counting iterator).  Shapes outside that pattern (reduced axes next to an
+// kernel, 16385 to 262144 sorted by the kernels of index_sort.h, the rest by the
+// vendor sort (rocPRIM's radix_sort_pairs, stable, the positions fed from a
+// counting iterator).  Shapes outside that pattern (reduced axes next to an
 // indexed one, an indexed y) keep the serial kernel.
 #include <algorithm>
 
 #include "elementwise.h"
 #include "functors.h"
+#include "index_sort.h"
 #include "ops.h"
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -488,6 +490,14 @@ int sort_index(hipStream_t s, const int32_t* index, uint32_t n, const int32_t** 
     *skey = k;
     *perm = k + n;
     return CT_OK;
+  }
+  if (n > kSortMinEntries && n <= kSortMaxEntries) {
+    // two bytes an entry more than the library's sort; where a captured stream has only those, that one it is
+    block = stream_scratch_if_any(s, index_sort_bytes(n), kScratchAccumA);
+    if (block) {
+      index_sort(s, index, n, block, skey, perm);
+      return CT_OK;
+    }
   }
   // the positions come from a counting iterator, so no array of them has to be written first
   size_t temp_bytes = 0;

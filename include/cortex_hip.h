@@ -168,7 +168,8 @@ int ct_stream_destroy(void* stream);
  * passes and batch-normalization statistics (reductions never need more than 16 MiB),
  * accumulate_bytes for each of the two blocks that accumulations into a broadcast or indexed
  * destination stage their temporaries through (at most the destination's size times the updates'
- * outermost extent; 12 bytes per index entry plus the sort's workspace for indexed rows).
+ * outermost extent; for indexed rows 18 bytes per index entry and 8 KiB up to 262144 entries, beyond
+ * that 8 bytes per entry plus the library sort's workspace, about as much again).
  * Zero leaves a block as it is. */
 int ct_stream_reserve_scratch(void* stream, size_t partial_bytes, size_t accumulate_bytes);
 

@@ -130,6 +130,31 @@ def test_accumulate_into_indexed_rows(P, code, rows, classes, width, kernel):
         centers.reset()
 
 
+SORTED = [
+    # entries, values below (the digits of a pass are 11 bits: one, two or three passes)
+    (16384, 2048),       # the library's sort still
+    (16385, 2048), (16385, 2049), (18432, 1 << 22),   # a tile of one entry; whole tiles only
+    (20001, (1 << 22) + 1), (33333, 2),               # two values: whole waves of one digit
+    (65537, 40000), (100000, 9000000), (131073, 5000),  # tiles in both words that a lane looks at
+    (262144, 1 << 17), (262145, 1 << 17),             # the largest, and the library's again
+]
+
+
+@pytest.mark.parametrize("entries,below", SORTED)
+def test_order_of_long_index_tensors(P, entries, below):
+    """Every update in its own turn: float sums whose rounding shows the order, and a last value that wins outright."""
+    rng = np.random.default_rng(entries + below)
+    labels = rng.integers(0, below, entries).astype(np.int32)
+    labels[rng.integers(0, entries, 3)] = below - 1
+    idx = P.buf(labels)
+    table = P.buf(values(rng, capi.F32, below))
+    y = P.buf(values(rng, capi.F32, entries, -9, 9))
+    for dest_alpha in (1.0, 0.0):
+        P.run(H.binary_accum, View(table, [entries, 1], [1, 1], index=[idx, None]), dest_alpha, View(y, [entries, 1]), 1.0, "+",
+              requires_cas=True)
+        exact(table, f"{entries} entries below {below}, destination times {dest_alpha}")
+
+
 @pytest.mark.parametrize("code", [capi.F32, capi.I32])
 def test_accumulate_indexed_layouts(P, code):
     rng = np.random.default_rng(34)
