@@ -358,7 +358,8 @@ void roll_back(hipStream_t s, const T* workspace, T* input_gradient, const ct_co
 }
 
 // Whether a float product goes to the matrix-core kernels: not where the library is faster.  Times are
-// those of the kernels, the unrolling in front of the library's forward product counted.  Where a
+// those of the float ones among them, the unrolling in front of the library's forward product counted
+// (which of them runs is decided in ops_conv_mfma.hip, where the split ones are the faster).  Where a
 // product is over in some twenty microseconds a layer is bound by the host, and a call of the library
 // costs that 5 to 9 us more.
 //
