@@ -155,6 +155,22 @@ def test_order_of_long_index_tensors(P, entries, below):
         exact(table, f"{entries} entries below {below}, destination times {dest_alpha}")
 
 
+@pytest.mark.parametrize("code", [capi.F32, capi.F64, capi.I8])
+@pytest.mark.parametrize("vectors", [255, 256, 257, 383, 384, 385, 1000])
+def test_accumulate_into_wide_indexed_rows(P, code, vectors):
+    """Rows around the first width of two vectors to a lane and around whole waves of lanes."""
+    rng = np.random.default_rng(vectors)
+    rows, classes, width = 50, 7, vectors * (16 // NP[code]().itemsize)
+    centers = P.buf(values(rng, code, classes * width))
+    idx = P.buf(rng.integers(0, classes, rows).astype(np.int32))
+    dest = View(centers, [rows, width], [width, 1], index=[idx, None])
+    y = View(P.buf(values(rng, code, rows * width, -9, 9)), [rows, width])
+    for op, reverse in (("+", False), ("-", True)):
+        k = P.run(H.binary_accum, dest, 1.0, y, 1.0, op, reverse=reverse, requires_cas=True)
+        assert k == "accum_grouped_vec", k
+        exact(centers, f"accumulate {op} rows of {vectors} vectors")
+
+
 @pytest.mark.parametrize("code", [capi.F32, capi.I32])
 def test_accumulate_indexed_layouts(P, code):
     rng = np.random.default_rng(34)
