@@ -44,12 +44,15 @@ class tensor_context(contextlib.ContextDecorator):
     ``src/cortex/verify/tensor.clj:11-17``)."""
 
     def __init__(self, stream, datatype: str = "double"):
-        self.stream, self.datatype = stream, datatype
+        self.stream, self.datatype, self._tokens = stream, datatype, None
 
     def _recreate_cm(self):
         return tensor_context(self.stream, self.datatype)
 
     def __enter__(self):
+        # an object binds once: a second entry would lose the tokens that the first exit needs
+        if self._tokens is not None:
+            raise RuntimeError("tensor_context: entered before; every `with` takes a new one")
         self._tokens = _stream.set(self.stream), _datatype.set(self.datatype)
         return self.stream
 
