@@ -8,6 +8,7 @@ without building.
 from __future__ import annotations
 
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -118,8 +119,11 @@ def _build_front(force: bool) -> None:
     if not force and FRONT.exists() and FRONT.stat().st_mtime >= max(src.stat().st_mtime, header.stat().st_mtime):
         return
     include = sysconfig.get_paths()["include"]
-    if not (Path(include) / "Python.h").exists():
-        sys.stderr.write(f"{include}/Python.h is missing: the front end stays in Python\n")
+    missing = ("g++" if shutil.which("g++") is None else
+               f"{include}/Python.h" if not (Path(include) / "Python.h").exists() else None)
+    if missing:
+        FRONT.unlink(missing_ok=True)     # of other sources than the library's
+        sys.stderr.write(f"{missing} is missing: the front end stays in Python\n")
         return
     fresh = FRONT.with_suffix(".tmp")     # this process may have the old one loaded
     cmd = ["g++", "-O2", "-std=c++17", "-Wall", "-shared", "-fPIC", f"-I{include}", str(src), "-o", str(fresh)]

@@ -126,3 +126,15 @@ def test_calls_report_what_the_library_reports():
             capi.call("ct_assign_constant", *args)
     with pytest.raises(AttributeError):
         capi.call("ct_no_such_entry")
+
+
+@pytest.mark.parametrize("stale", [False, True])
+def test_a_build_without_a_host_compiler_leaves_the_front_end_in_python(tmp_path, monkeypatch, capsys, stale):
+    from cortex_amd import build
+
+    monkeypatch.setattr(build, "FRONT", tmp_path / build.FRONT.name)
+    if stale:
+        build.FRONT.touch()
+    monkeypatch.setenv("PATH", str(tmp_path))
+    build._build_front(force=True)
+    assert "g++ is missing" in capsys.readouterr().err and list(tmp_path.iterdir()) == []
