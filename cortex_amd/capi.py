@@ -209,7 +209,7 @@ def lib() -> C.CDLL:
         _lib = load_library()
         if front is not None:
             for name in PROTOTYPES:
-                front.bind(name, C.cast(getattr(_lib, name), C.c_void_p).value)
+                front.bind(_lib, name, C.cast(getattr(_lib, name), C.c_void_p).value)
     return _lib
 
 

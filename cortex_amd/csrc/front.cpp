@@ -22,7 +22,7 @@ namespace {
 
 constexpr Py_ssize_t kMost = 8;   // dimensions
 
-PyObject *s_shape, *s_strides, *s_max_shape, *s_dimensions;
+PyObject *s_shape, *s_strides, *s_max_shape, *s_dimensions, *s_lib;
 
 struct Plain {
   Py_ssize_t n;
@@ -369,13 +369,20 @@ Entry g_entries[] = {
     CT_ENTRY(ct_batch_normalize_gradients_spatial), CT_ENTRY(ct_gemm), CT_ENTRY(ct_gemv), CT_ENTRY(ct_rand),
     CT_ENTRY(ct_dropout_bernoulli_mask), CT_ENTRY(ct_adam_step), CT_ENTRY(ct_adadelta_step), CT_ENTRY(ct_lrn_forward),
     CT_ENTRY(ct_lrn_backward)};
-PyObject* g_index;   // name -> index of an entry whose address is known
+PyObject* g_index;     // name -> index of an entry whose address is known
+PyObject* g_library;   // the library that the addresses are of
+
+// Whether capi's library is the one whose addresses are known: a program may put another in its place.
+bool bound_library() {
+  PyObject* python = g_python[kCall];
+  return g_library && PyFunction_Check(python) && PyDict_GetItem(PyFunction_GET_GLOBALS(python), s_lib) == g_library;
+}
 
 // capi.call; `check` is called with a status that is not zero, and raises.
 PyObject* g_check;
 PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
   PyObject* at = n > 0 && PyUnicode_CheckExact(args[0]) ? PyDict_GetItem(g_index, args[0]) : nullptr;
-  if (at) {
+  if (at && bound_library()) {
     const Entry& e = g_entries[PyLong_AsLong(at)];
     int status = 0;
     if (e.invoke(e.address, args + 1, n - 1, &status)) {
@@ -386,15 +393,21 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return hand_on(kCall, args, n);
 }
 
-// bind(name, address): whether the entry point is one that `call` knows.
+// bind(library, name, address): whether the entry point is one that `call` knows.  The addresses of one library are known at a
+// time.
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 2 || !PyUnicode_Check(args[0])) return PyErr_SetString(PyExc_TypeError, "bind(name, address)"), nullptr;
+  if (n != 3 || !PyUnicode_Check(args[1])) return PyErr_SetString(PyExc_TypeError, "bind(library, name, address)"), nullptr;
+  if (args[0] != g_library) {
+    PyDict_Clear(g_index);
+    Py_INCREF(args[0]);
+    Py_XSETREF(g_library, args[0]);
+  }
   for (size_t i = 0; i < sizeof(g_entries) / sizeof(g_entries[0]); ++i)
-    if (PyUnicode_CompareWithASCIIString(args[0], g_entries[i].name) == 0) {
-      g_entries[i].address = PyLong_AsVoidPtr(args[1]);
+    if (PyUnicode_CompareWithASCIIString(args[1], g_entries[i].name) == 0) {
+      g_entries[i].address = PyLong_AsVoidPtr(args[2]);
       if (PyErr_Occurred()) return nullptr;
       PyObject* at = PyLong_FromSize_t(i);
-      const int rc = at ? PyDict_SetItem(g_index, args[0], at) : -1;
+      const int rc = at ? PyDict_SetItem(g_index, args[1], at) : -1;
       Py_XDECREF(at);
       if (rc) return nullptr;
       Py_RETURN_TRUE;
@@ -462,6 +475,7 @@ PyMODINIT_FUNC PyInit__front() {
   s_strides = PyUnicode_InternFromString("strides");
   s_max_shape = PyUnicode_InternFromString("max-shape");
   s_dimensions = PyUnicode_InternFromString("dimensions");
+  s_lib = PyUnicode_InternFromString("_lib");
   g_index = PyDict_New();
-  return s_shape && s_strides && s_max_shape && s_dimensions && g_index ? PyModule_Create(&g_module) : nullptr;
+  return s_shape && s_strides && s_max_shape && s_dimensions && s_lib && g_index ? PyModule_Create(&g_module) : nullptr;
 }

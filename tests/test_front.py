@@ -128,6 +128,29 @@ def test_calls_report_what_the_library_reports():
         capi.call("ct_no_such_entry")
 
 
+def test_calls_go_to_the_library_that_is_set(monkeypatch):
+    """A library put in the place of the one that was loaded gets every call, those that the native half makes among them."""
+    if not capi.LIB_PATH.exists():
+        pytest.skip("the library is not built")
+    capi.lib()
+    refused = ("ct_memset", None, None, capi.F32, 0.0, -1)
+    with pytest.raises(capi.CortexHipError):
+        capi.call(*refused)
+
+    class Library:
+        def ct_memset(self, *args):
+            calls.append(args)
+            return 0
+
+    calls = []
+    with monkeypatch.context() as m:
+        m.setattr(capi, "_lib", Library())
+        assert capi.call(*refused) is None and calls == [refused[1:]]
+    with pytest.raises(capi.CortexHipError):
+        capi.call(*refused)
+    assert len(calls) == 1
+
+
 @pytest.mark.parametrize("stale", [False, True])
 def test_a_build_without_a_host_compiler_leaves_the_front_end_in_python(tmp_path, monkeypatch, capsys, stale):
     from cortex_amd import build
