@@ -41,6 +41,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "conv_gather.h"
 #include "conv_products.h"
 #include "split_mfma.h"
 
@@ -429,10 +430,10 @@ __global__ void __launch_bounds__(kPositions, 2) conv_forward_kernel(const ConvP
     for (uint32_t kx = 0; kx < a.kw; ++kx, bit <<= 1)
       taps_outside |= (((uint32_t)iy0 + ky < a.in_h) & ((uint32_t)ix0 + kx < a.in_w)) ? 0u : bit;
   // bytes, from the first row and column of the padding on, so that no window begins below the base
-  const uint32_t pad = (uint32_t)a.py * a.in_w + (uint32_t)a.px;
-  const __amdgpu_buffer_rsrc_t source = buffer_of(a.input - pad, (a.images * (uint32_t)a.in_image + pad) * 4);
+  const uint32_t padding = gather_padding(a.in_w, a.px, a.py), length = gather_length(a.images, (uint32_t)a.in_image, padding);
+  const __amdgpu_buffer_rsrc_t source = buffer_of(a.input - padding, length * 4);
   const __amdgpu_buffer_rsrc_t cells = buffer_of(a.workspace, a.images * (uint32_t)a.conv_image * 4);
-  const uint32_t from = (image * (uint32_t)a.in_image + pad + (uint32_t)iy0 * a.in_w + (uint32_t)ix0) * 4;
+  const uint32_t from = gather_window(image, (uint32_t)a.in_image, a.in_w, padding, iy0, ix0) * 4;
   const uint32_t to = m_tile == 0 && j < a.n ? (image * (uint32_t)a.conv_image + pos) * 4 : kOutside;
 
   // kCount k from k0 on, decoded by the lanes and loaded
@@ -442,7 +443,7 @@ __global__ void __launch_bounds__(kPositions, 2) conv_forward_kernel(const ConvP
     uint32_t channel, tap, ky, kx;
     a.taps_fd.divmod(my_k, channel, tap);
     a.kw_fd.divmod(tap, ky, kx);
-    const uint32_t my_cell = (channel * a.in_plane + ky * a.in_w + kx) * 4, my_shift = 31 - tap;
+    const uint32_t my_cell = gather_tap(channel, ky, kx, a.in_plane, a.in_w, length) * 4, my_shift = 31 - tap;
 #pragma unroll
     for (int e = 0; e < kCount; ++e) {
       const uint32_t at = from | ((taps_outside << __builtin_amdgcn_readlane(my_shift, e)) & kOutside);

@@ -332,6 +332,18 @@ def test_products_in_pieces_at_the_edges_of_their_tiles(P, case):
     check_products(P, batch, cin, cout, side, side, k, k, k // 2, k // 2, stride, stride)
 
 
+# The output formed in pieces over a single image of one or two rows: the window reaches below it (test_conv_gather.py has the
+# arithmetic).  Those cells are zero, also in the unrolled input.
+@pytest.mark.parametrize("case", [
+    (1, 8, 5, 1, 80000, 3, 3, 1, 1, 1, 1),
+    (1, 4, 5, 2, 40000, 5, 5, 2, 2, 1, 1),
+    (1, 16, 5, 1, 80000, 1, 5, 0, 2, 1, 1),
+    (2, 8, 5, 1, 40000, 3, 3, 1, 1, 1, 1),
+], ids=lambda c: "x".join(map(str, c)))
+def test_products_in_pieces_over_low_images(P, case):
+    check_products(P, *case)
+
+
 @pytest.mark.parametrize("case", [(46, 8, 33, 40, 3), (41, 15, 20, 40, 3), (5, 20, 200, 19, 3)], ids=lambda c: "x".join(map(str, c)))
 def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
     """An infinity, a NaN and floats that the pieces do not hold, in the weights and in both gradients' operands: the blocks
