@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <type_traits>
 
 #include "../../include/cortex_hip.h"
@@ -29,7 +30,25 @@ int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot = kScratchR
 // The same where the caller can do without: null, and no error, if the block is too small and cannot grow, for want of memory
 // or because the stream is being captured.
 void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot = kScratchReduce);
+// The block as it is, if it is as large: null rather than another.
+void* stream_scratch_held(hipStream_t s, size_t bytes, int slot = kScratchReduce);
 void release_stream_scratch(hipStream_t s);
+
+// Scratch of a stream for the partial sums of a matrix product, and the stream's right to launch what uses it: two threads may
+// form products on one stream, and one's launches must not come between the other's.  A block that has become too small is kept
+// until the stream is destroyed, for a recorded graph may still write to it: blocks double, so that all of them together stay
+// below twice kMostProductScratch.
+constexpr size_t kMostProductScratch = size_t(256) << 20;
+class ProductScratch {
+ public:
+  // Holds nothing if the block is too small and cannot grow, for want of memory or because a stream is being captured.
+  ProductScratch(hipStream_t s, size_t bytes);
+  void* get() const { return ptr_; }
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+  void* ptr_ = nullptr;
+};
 
 inline void note_kernel(const char* name) { *last_kernel_slot() = name; }
 

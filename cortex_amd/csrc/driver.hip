@@ -3,7 +3,9 @@
 // the library's error state.
 #include <atomic>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <vector>
 
 #include "elementwise.h"
 #include "functors.h"
@@ -34,6 +36,14 @@ struct ScratchKey {
 struct ScratchBlock { void* ptr; size_t bytes; };
 std::mutex g_scratch_mutex;
 std::map<ScratchKey, ScratchBlock> g_scratch;
+
+struct ProductBlocks {
+  std::mutex mutex;            // held while a product's launches are made
+  std::vector<void*> blocks;   // the last one is in use
+  size_t bytes = 0;
+};
+constexpr int kProductKey = kScratchSlots;   // in the place of a slot
+std::map<ScratchKey, std::unique_ptr<ProductBlocks>> g_products;
 }  // namespace
 
 int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot) {
@@ -57,23 +67,36 @@ int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot) {
   return CT_OK;
 }
 
+namespace {
+// Memory for a caller that can do without: none while the stream is being captured.
+void* allocate_if_any(hipStream_t s, size_t bytes) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  void* block = nullptr;
+  if (hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
+      hipMalloc(&block, bytes) == hipSuccess)
+    return block;
+  (void)hipGetLastError();
+  return nullptr;
+}
+}  // namespace
+
+void* stream_scratch_held(hipStream_t s, size_t bytes, int slot) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  const auto it = g_scratch.find(ScratchKey{dev, s, slot});
+  return it != g_scratch.end() && it->second.bytes >= bytes ? it->second.ptr : nullptr;
+}
+
 void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   ScratchBlock& b = g_scratch[ScratchKey{dev, s, slot}];
   if (b.bytes >= bytes) return b.ptr;
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
   const size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
-  void* grown = nullptr;
-  if (hipMalloc(&grown, want) != hipSuccess) {   // the block stays what it was
-    (void)hipGetLastError();
-    return nullptr;
-  }
+  void* const grown = allocate_if_any(s, want);
+  if (!grown) return nullptr;   // the block stays what it was
   if (b.ptr) {
     // earlier kernels of this stream may still be reading the old block
     if (hipStreamSynchronize(s) != hipSuccess) {
@@ -87,10 +110,36 @@ void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot) {
   return grown;
 }
 
+ProductScratch::ProductScratch(hipStream_t s, size_t bytes) {
+  int dev = 0;
+  if (bytes > kMostProductScratch || hipGetDevice(&dev) != hipSuccess) return;
+  ProductBlocks* p;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    auto& entry = g_products[ScratchKey{dev, s, kProductKey}];
+    if (!entry) entry = std::make_unique<ProductBlocks>();
+    p = entry.get();
+  }
+  lock_ = std::unique_lock<std::mutex>(p->mutex);
+  if (p->bytes < bytes) {
+    size_t want = std::max(size_t(1) << 20, 2 * p->bytes);
+    while (want < bytes) want *= 2;
+    void* const grown = allocate_if_any(s, want);
+    if (!grown) return;
+    p->blocks.push_back(grown);
+    p->bytes = want;
+  }
+  ptr_ = p->blocks.back();
+}
+
 void release_stream_scratch(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  if (auto it = g_products.find(ScratchKey{dev, s, kProductKey}); it != g_products.end()) {
+    for (void* block : it->second->blocks) (void)hipFree(block);
+    g_products.erase(it);
+  }
   for (int slot = 0; slot < kScratchSlots; ++slot) {
     auto it = g_scratch.find(ScratchKey{dev, s, slot});
     if (it == g_scratch.end()) continue;
@@ -245,8 +294,10 @@ int ct_stream_destroy(void* stream) {
 
 int ct_stream_reserve_scratch(void* stream, size_t partial_bytes, size_t accumulate_bytes) {
   void* unused = nullptr;
-  if (partial_bytes)
+  if (partial_bytes) {
     if (int rc = stream_scratch((hipStream_t)stream, partial_bytes, &unused, kScratchReduce)) return rc;
+    (void)ProductScratch((hipStream_t)stream, std::min(partial_bytes, kMostProductScratch));   // products can do without
+  }
   if (accumulate_bytes) {
     if (int rc = stream_scratch((hipStream_t)stream, accumulate_bytes, &unused, kScratchAccumA)) return rc;
     if (int rc = stream_scratch((hipStream_t)stream, accumulate_bytes, &unused, kScratchAccumB)) return rc;

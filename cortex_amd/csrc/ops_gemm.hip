@@ -15,6 +15,7 @@
 //
 // Tiles and their choice: below, at expected_time.
 #include <algorithm>
+#include <optional>
 
 #include "common.h"
 #include "gemm.h"
@@ -502,8 +503,6 @@ double expected_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
   return us;
 }
 
-constexpr int64_t kMostScratch = int64_t(256) << 20;
-
 Plan best_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
   struct Candidate {
     Tile tile;
@@ -516,7 +515,7 @@ Plan best_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
   for (const Candidate& c : kCandidates) {
     const Plan p = plan_of(c.tile, c.splits, k);
     if (p.splits != c.splits || (p.tile != kSmall && k < 32)) continue;
-    if (p.splits > 1 && (!may_split || batch > 1 || p.splits * m * n * (int64_t)sizeof(float) > kMostScratch)) continue;
+    if (p.splits > 1 && (!may_split || batch > 1 || p.splits * m * n * (int64_t)sizeof(float) > (int64_t)kMostProductScratch)) continue;
     const double us = expected_time(p, m, n, batch);
     if (best_us < 0.0 || us < best_us) {
       best = p;
@@ -554,10 +553,12 @@ bool gemm_split_takes(const GemmProduct& p) {
 
 int gemm_split(hipStream_t s, const GemmProduct& p) {
   Plan plan = best_plan(p.m, p.n, p.k, p.batch, true);
+  std::optional<ProductScratch> scratch;   // until both launches are made
   float* partial = nullptr;
   if (plan.splits > 1) {
     // no room, or none to be had while the stream is being captured: one launch
-    partial = static_cast<float*>(stream_scratch_if_any(s, (size_t)(plan.splits * p.m * p.n) * sizeof(float)));
+    scratch.emplace(s, (size_t)(plan.splits * p.m * p.n) * sizeof(float));
+    partial = static_cast<float*>(scratch->get());
     if (!partial) plan = best_plan(p.m, p.n, p.k, p.batch, false);
   }
   GemmArgs a{};

@@ -165,7 +165,9 @@ int ct_stream_destroy(void* stream);
  * allocates a new one.  A caller that wants no allocation and no synchronisation inside later
  * calls (a latency-critical loop, a stream about to be captured into a graph) reserves once:
  * partial_bytes for the partial results of split reductions, matrix-vector products, convolution
- * passes and batch-normalization statistics (reductions never need more than 16 MiB),
+ * passes and batch-normalization statistics (reductions never need more than 16 MiB), and as much
+ * again, up to 256 MiB, for those of float matrix products (ct_gemm), which have blocks of their own:
+ * those grow without synchronising, and the smaller ones stay until the stream is destroyed;
  * accumulate_bytes for each of the two blocks that accumulations into a broadcast or indexed
  * destination stage their temporaries through (at most the destination's size times the updates'
  * outermost extent; for indexed rows 18 bytes per index entry and 8 KiB up to 262144 entries, beyond
@@ -341,10 +343,10 @@ int ct_softmax_spatial(void* stream, void* output, const ct_dims* output_dims, c
  * a column stride is the distance in elements between two stored rows.  Float
  * products run on the library's own kernels (operands held exactly, sums in float),
  * double ones and some shapes of float on rocBLAS, loaded on first use.  A float
- * product of few results over a long sum keeps partial sums in the stream's
- * scratch memory, up to 256 MiB, where there is room or it can grow (not while the
- * stream is being captured), and does without otherwise.  dtype is CT_F32 or
- * CT_F64. */
+ * product of few results over a long sum keeps partial sums in scratch memory of
+ * the stream, up to 256 MiB, where there is room or it can grow (not while the
+ * stream is being captured), and does without otherwise: the sum is then taken in
+ * another order and may differ in its last bits.  dtype is CT_F32 or CT_F64. */
 int ct_gemm(void* stream, void* c, int64_t c_colstride, int trans_a, int trans_b, double alpha,
             const void* a, int64_t a_row_count, int64_t a_col_count, int64_t a_colstride,
             const void* b, int64_t b_col_count, int64_t b_colstride, double beta, int dtype);

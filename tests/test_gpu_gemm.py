@@ -1,4 +1,7 @@
 """gemm! of float matrices at the edges of its tiles and of its number range, against the CPU oracle."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -116,3 +119,48 @@ def test_a_result_over_its_own_operand_is_the_library_s(P):
     H.gemm(P.hip, v(a), m, False, False, 1.0, v(a), m, m, m, v(b), m, m, 0.0)
     from cortex_amd import capi
     assert capi.last_kernel() == "rocblas_gemm"
+
+
+def test_two_threads_on_one_stream():
+    """Products with partial sums, of two sizes, from two threads on one stream: the launches of one call stay together."""
+    from cortex_amd import capi
+    stream = C.c_void_p()
+    capi.call("ct_set_device", 0)
+    capi.call("ct_set_debug_sync", 0)
+    capi.call("ct_stream_create", C.byref(stream))
+    errors, calls = [], 300
+    start = threading.Barrier(2)
+
+    def work(m, n, k):
+        try:
+            capi.call("ct_set_device", 0)
+            rng = np.random.default_rng(m)
+            host = [rng.integers(-3, 4, s).astype(np.float32) for s in ((m, k), (n, k), (m, n))]
+            a, b, c = (H.Buf(h, gpu=True) for h in host)
+            others = [H.Buf(np.zeros((m, n), np.float32), gpu=True) for _ in range(9)]
+            start.wait()
+            for i in range(calls):
+                to = c if i % 10 == 0 else others[i % 10 - 1]
+                capi.call("ct_gemm", stream, to.dev, n, 0, 1, 1.0, a.dev, m, k, k, b.dev, n, k, 0.0, capi.F32)
+                assert capi.last_kernel().endswith("+gemm_sum")
+            capi.call("ct_stream_sync", stream)
+            want = host[0] @ host[1].T
+            for x in [c] + others:
+                assert np.array_equal(x.download().reshape(m, n), want)
+                x.free()
+            a.free()
+            b.free()
+        except BaseException as e:     # the other thread is not left at the barrier
+            start.abort()
+            errors.append(e)
+
+    try:
+        threads = [threading.Thread(target=work, args=size) for size in ((10, 20, 3700), (64, 2048, 4096))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+    finally:
+        capi.call("ct_stream_destroy", stream)
+        capi.call("ct_set_debug_sync", 1)

@@ -164,3 +164,112 @@ def test_a_recorded_step_replays_to_the_eager_results():
             t.free()
         capi.call("ct_stream_destroy", stream)
         capi.call("ct_set_debug_sync", 1)
+
+
+class Recorded:
+    """What `step` puts on `stream`, as a graph that can be launched again and again."""
+
+    def __init__(self, rt, stream, step):
+        self.rt, self.stream, self.graph, self.exec = rt, stream, C.c_void_p(), C.c_void_p()
+        assert rt.hipStreamBeginCapture(stream, HIP_STREAM_CAPTURE_MODE_THREAD_LOCAL) == 0
+        try:
+            step()
+        finally:
+            ended = rt.hipStreamEndCapture(stream, C.byref(self.graph))
+        assert ended == 0 and self.graph.value, f"the capture did not end cleanly (hipError {ended})"
+        assert rt.hipGraphInstantiate(C.byref(self.exec), self.graph, None, None, 0) == 0
+
+    def replay(self):
+        assert self.rt.hipGraphLaunch(self.exec, self.stream) == 0
+        capi.call("ct_stream_sync", self.stream)
+
+    def destroy(self):
+        capi.call("ct_stream_sync", self.stream)
+        assert self.rt.hipGraphExecDestroy(self.exec) == 0 and self.rt.hipGraphDestroy(self.graph) == 0
+
+
+@pytest.fixture()
+def fresh():
+    """A stream without scratch, debug-sync mode off, and a list of tensors that are given back."""
+    capi.call("ct_set_device", 0)
+    capi.call("ct_set_debug_sync", 0)
+    stream, tensors = C.c_void_p(), []
+    capi.call("ct_stream_create", C.byref(stream))
+
+    def tensor(host):
+        tensors.append(Dev(host))
+        return tensors[-1]
+
+    yield stream, tensor
+    capi.call("ct_stream_sync", stream)
+    for t in tensors:
+        t.free()
+    capi.call("ct_stream_destroy", stream)
+    capi.call("ct_set_debug_sync", 1)
+
+
+def product(stream, c, a, b, m, n, k):
+    """c [m, n] = a [m, k] b [n, k]^T; the kernels that were launched."""
+    capi.call("ct_gemm", stream, c.ptr, n, 0, 1, 1.0, a.ptr, m, k, k, b.ptr, n, k, 0.0, capi.F32)
+    return capi.last_kernel()
+
+
+def whole(rng, *shape):
+    return rng.integers(-3, 4, shape).astype(np.float32)
+
+
+def test_recorded_products_and_reductions_outlive_a_larger_eager_product(fresh):
+    """A product with partial sums and a split reduction, recorded with the scratch that a first eager call left; then eager
+    products that need many times the scratch, between the replays.  Whole numbers: every sum is exact."""
+    stream, tensor = fresh
+    capi.call("ct_stream_reserve_scratch", stream, 1 << 20, 0)
+    rng = np.random.default_rng(3)
+    m, n, k, rows, cols = 10, 20, 3700, 4096, 2048
+    a, b, c = tensor(whole(rng, m, k)), tensor(whole(rng, n, k)), tensor(whole(rng, m, n))
+    x, total = tensor(whole(rng, rows, cols)), tensor(whole(rng, cols))
+    sizes = [(768, 1024, 4096), (2048, 3072, 4096)]
+    large = [(tensor(whole(rng, q, s)), tensor(whole(rng, p, s)), tensor(np.zeros((q, p), np.float32)), (q, p, s)) for q, p, s in sizes]
+
+    def step():
+        assert product(stream, c, a, b, m, n, k).endswith("+gemm_sum")
+        capi.call("ct_unary_reduce", stream, total.ptr, C.byref(dims([cols, 1])), 1.0, x.ptr, C.byref(dims([cols, rows], [1, cols])),
+                  capi.REDUCE_OPS["sum"], capi.F32)
+
+    step()      # the kernels are loaded
+    capi.call("ct_stream_sync", stream)
+    recorded = Recorded(hip_runtime(), stream, step)
+    for replay in range(5):
+        host_a, host_x = whole(rng, m, k), whole(rng, rows, cols)
+        a.upload(host_a, stream)
+        x.upload(host_x, stream)
+        if replay:
+            p, q, r, size = large[replay % 2]
+            assert product(stream, r, p, q, *size).endswith("+gemm_sum")
+        recorded.replay()
+        assert np.array_equal(c.download(stream).reshape(m, n), host_a @ b.host.reshape(n, k).T), replay
+        assert np.array_equal(total.download(stream), host_x.sum(axis=0)), replay
+        if replay:
+            rows_of = slice(0, 7)
+            want = p.host.reshape(size[0], size[2])[rows_of] @ q.host.reshape(size[1], size[2]).T
+            assert np.array_equal(r.download(stream).reshape(size[:2])[rows_of], want), replay
+    recorded.destroy()
+
+
+def test_a_product_recorded_without_scratch_does_without(fresh):
+    """The same product keeps no partial sums where a capture finds no scratch, and its result is as exact."""
+    stream, tensor = fresh
+    rng = np.random.default_rng(4)
+    m, n, k = 10, 20, 3700
+    a, b, c = tensor(whole(rng, m, k)), tensor(whole(rng, n, k)), tensor(whole(rng, m, n))
+    kernels = []
+    product(stream, c, a, b, m, n, 30)      # the library is loaded; no scratch needed
+    recorded = Recorded(hip_runtime(), stream, lambda: kernels.append(product(stream, c, a, b, m, n, k)))
+    assert kernels[0].startswith("gemm_") and not kernels[0].endswith("+gemm_sum"), kernels
+    for replay in range(3):
+        host = whole(rng, m, k)
+        a.upload(host, stream)
+        recorded.replay()
+        assert np.array_equal(c.download(stream).reshape(m, n), host @ b.host.reshape(n, k).T), replay
+        assert product(stream, c, a, b, m, n, k).endswith("+gemm_sum")
+        assert np.array_equal(c.download(stream).reshape(m, n), host @ b.host.reshape(n, k).T), replay
+    recorded.destroy()
