@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) gemm_small_kernel(const Gemm
       r[e] = r_next[e];
     }
   }
-  bool found = false;
+  bool found = a.k == 1;   // a product by itself: the floats' is rounded once, and what the pieces leave out is not made up for
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const float sum = sums[0][e] + sums[1][e];

@@ -97,6 +97,25 @@ def test_the_ends_of_the_number_range(P, size):
     assert np.all(np.abs(got[fine].astype(np.float64) - want[fine]) <= 1e-5 * scale[fine] + k * 2.0 ** -150), kernel
 
 
+@pytest.mark.parametrize("size", [(1, 1), (5, 1435), (100, 39), (500, 500)], ids=str)
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_outer_products_are_the_floats_products(P, size, ta, tb):
+    """One product to a result: rounded once, as float multiplication rounds it, also where it is denormal or overflows."""
+    m, n = size
+    rng = np.random.default_rng(m)
+    a, b, c = operands(lambda s: rng.standard_normal(s).astype(np.float32), m, n, 1, ta, tb)
+    a.reshape(-1)[::7] *= 1e-25
+    a.reshape(-1)[3::11] *= 1e25
+    b.reshape(-1)[::5] *= 1e-18
+    b.reshape(-1)[2::13] *= 1e18
+    kernel, got, _ = run(P, a, b, c, ta, tb, m, n, 1)
+    assert kernel == "gemm_small", kernel
+    with np.errstate(over="ignore"):
+        want = a.reshape(m, 1) * b.reshape(1, n) + np.float32(0)   # a sum begins at +0
+    H.assert_bit_exact(got, want, kernel)
+
+
 @pytest.mark.parametrize("exponent", [-135, -100, 60])
 def test_scaled_operands_scale_the_result(P, exponent):
     """Multiplying an operand by a power of two multiplies the result, to the bit, as long as neither leaves the floats:
