@@ -6,12 +6,14 @@
 // clock gives way: at these rates it stands at 1.8 to 2.0 of 2.4 GHz, and more instructions a cycle lower it further
 // (matrix instructions alone, on normal operands: 1770 of 2500 TFLOP/s, 295 in floats).
 //
-// Times of products, in us, the library's second: [1024, 4096] over 4096 k, b stored [n][k] 223 and 273, stored [k][n] 209
-// and 267; [4096, 4096] over 1024, both stored [k][.] 225 and 275; 4096 cubed 741 and 1121; 2048 cubed 96 and 133;
-// [64, 4096] over 4096 26 and 114; [128, 784] over 128 5.2 and 7.9; [128, 128] over 784 8.3 and 7.3, but a call costs the
-// host 3 and 5.  Over 420 products of layers of 1 to 4096 a side: 1.36 times the library's speed in the geometric mean, 0.8
-// at the least (few k, or a chain of blocks that just misses a round), 5.6 at the most; errors against 64 bits 0.1 to 1.0
-// of the library's.
+// Times of products, in us, the library's second: [1024, 4096] over 4096 k, b stored [n][k] 197 and 271, stored [k][n] 203
+// and 261; [4096, 4096] over 1024, both stored [k][.] 214 and 274; 4096 cubed 725 and 1121; 2048 cubed 94 and 133;
+// [64, 4096] over 4096 24 and 114; [128, 784] over 128 4.5 and 7.2; [128, 128] over 784 5.5 and 6.9.  Over 900 products of
+// layers of 1 to 4096 a side, whole calls one after the other: 1.47 times the library's speed in the geometric mean, 0.86 to
+// 4.3 in 98 % of them, 0.72 at the least.  Where it is below 0.9 they are of three kinds: a and b stored with their k side by
+// side, 500 to 1500 of them, over 70 to 700 tiles of 32 x 32 ([457, 132] over 1056 10.2 and 7.2); 65 to 275 k over 1 to 2
+// million results ([1682, 1039] over 93 9.9 and 7.5); and a chain of blocks that just misses a round.
+// Errors against 64 bits, of the library's: 0.05 to 1.0, 0.34 in the median.
 //
 // Tiles and their choice: below, at expected_time.
 #include <algorithm>
@@ -334,36 +336,65 @@ __device__ __forceinline__ void load8_at(const float* p, int64_t ld, f32x4 (&to)
   }
 }
 
-// The same for results too small to fill the chip with tiles, in one launch: a block owns 32 x 32, its sixteen waves take
-// every sixteenth run of 32 k each, straight from memory into the fragments, and their sums are added in LDS in their order.
-constexpr int kSmallWaves = 16;
+// The same for results too small to fill the chip with tiles, in one launch: a block owns S x S, its W waves take every W-th
+// run of 32 k each, straight from memory into the fragments, and their sums are added in LDS in their order.  In tiles of
+// 16 x 16 the sums of four runs are added up there too: through 3000 k and more the error was up to 1.3 times that of shorter
+// sums.  (In tiles of 32 x 32 it cost up to a fifth of the time; those have sixteen waves where a wave would take more.)
+constexpr uint32_t kRunsToASum = 4;
 
-template <bool kA, bool kB>
-__global__ void __launch_bounds__(64 * kSmallWaves) gemm_small_kernel(const GemmArgs a) {
-  constexpr int BK = 32;
-  __shared__ float partial[kSmallWaves][1024];
+template <int S>
+struct SmallTile;
+template <>
+struct SmallTile<32> {
+  static constexpr int kParts = 2;   // products to a run of 32 k
+  using Cells = f32x16;
+  static __device__ __forceinline__ Cells product(bf16x8 l, bf16x8 r, Cells sum) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, r, sum, 0, 0, 0);
+  }
+  static __device__ __forceinline__ Cells product_in_float(float l, float r, Cells sum) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(l, r, sum, 0, 0, 0);
+  }
+};
+template <>
+struct SmallTile<16> {
+  static constexpr int kParts = 1;
+  using Cells = f32x4;
+  static __device__ __forceinline__ Cells product(bf16x8 l, bf16x8 r, Cells sum) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, r, sum, 0, 0, 0);
+  }
+  static __device__ __forceinline__ Cells product_in_float(float l, float r, Cells sum) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(l, r, sum, 0, 0, 0);
+  }
+};
+
+template <int S, int W, bool kA, bool kB>
+__global__ void __launch_bounds__(64 * W, 4) gemm_small_kernel(const GemmArgs a) {
+  using Tile = SmallTile<S>;
+  using Cells = typename Tile::Cells;
+  constexpr int BK = 32, kParts = Tile::kParts, kCells = S * S / 64, E = kParts * 8;   // floats of a run to a lane
+  __shared__ float partial[W][S * S];
   const uint32_t unit = unit_of_block(blockIdx.x, a.units);
   if (unit >= a.units) return;
   const Place place = place_of(a, unit);
-  const uint32_t lane = threadIdx.x & 63, row = lane & 31, half = lane >> 5;
+  const uint32_t lane = threadIdx.x & 63, row = lane % S, group = lane / S;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t k_first = place.split * a.tiles_per_group * BK, k_end = min(a.k, k_first + a.tiles_per_group * BK);
-  const uint32_t m = min(place.m_tile * 32 + row, a.m - 1), n = min(place.n_tile * 32 + row, a.n - 1);
+  const uint32_t m = min(place.m_tile * S + row, a.m - 1), n = min(place.n_tile * S + row, a.n - 1);
   const float* left = a.a + (int64_t)place.batch * a.a_batch + (kA ? (int64_t)m * a.lda : m);
   const float* right = a.b + (int64_t)place.batch * a.b_batch + (kB ? (int64_t)n * a.ldb : n);
-  // a lane's sixteen k of a run: 8 * half + 0 .. 7 and 16 + 8 * half + 0 .. 7
-  auto load = [&](uint32_t k0, f32x4 (&l)[4], f32x4 (&r)[4]) {
+  // a lane's k of a run: 8 * group + 0 .. 7 and, in two parts, 16 more
+  auto load = [&](uint32_t k0, f32x4 (&l)[E / 4], f32x4 (&r)[E / 4]) {
     if (k0 + BK <= k_end) {
 #pragma unroll
-      for (uint32_t part = 0; part < 2; ++part) {
-        const int64_t k = k0 + part * 16 + half * 8;
+      for (uint32_t part = 0; part < kParts; ++part) {
+        const int64_t k = k0 + part * 16 + group * 8;
         load8_at<kA>(left + (kA ? k : k * a.lda), a.lda, reinterpret_cast<f32x4(&)[2]>(l[part * 2]));
         load8_at<kB>(right + (kB ? k : k * a.ldb), a.ldb, reinterpret_cast<f32x4(&)[2]>(r[part * 2]));
       }
     } else {
 #pragma unroll
-      for (uint32_t e = 0; e < 16; ++e) {
-        const uint32_t at = k0 + e / 8 * 16 + half * 8 + e % 8;
+      for (uint32_t e = 0; e < E; ++e) {
+        const uint32_t at = k0 + e / 8 * 16 + group * 8 + e % 8;
         const int64_t k = min(at, k_end - 1);
         const float x = left[kA ? k : k * a.lda], y = right[kB ? k : k * a.ldb];
         l[e / 4][e % 4] = at < k_end ? x : 0.f;
@@ -371,16 +402,27 @@ __global__ void __launch_bounds__(64 * kSmallWaves) gemm_small_kernel(const Gemm
       }
     }
   };
-  f32x16 sums[2] = {zero16(), zero16()};
+  Cells sums[2] = {};   // the products of the leading pieces; all others
   const SplitWeights weights;
-  f32x4 l[4], r[4], l_next[4], r_next[4];
+  f32x4 l[E / 4], r[E / 4], l_next[E / 4], r_next[E / 4];
   const uint32_t k_mine = k_first + wave * BK;
+  bool found = a.k == 1;   // a product by itself: the floats' is rounded once, and what the pieces leave out is not made up for
+  auto add_up = [&](bool first) {
+#pragma unroll
+    for (int e = 0; e < kCells; ++e) {
+      const float sum = sums[0][e] + sums[1][e];
+      found |= not_finite(sum);
+      float& cell = partial[wave][e * 64 + lane];
+      cell = first ? sum * kSplitUnscale : cell + sum * kSplitUnscale;
+    }
+  };
   if (k_mine < k_end) load(k_mine, l, r);
-  for (uint32_t k0 = k_mine; k0 < k_end; k0 += kSmallWaves * BK) {
-    const uint32_t next = k0 + kSmallWaves * BK;
+  uint32_t run = 0;
+  for (uint32_t k0 = k_mine; k0 < k_end; k0 += W * BK, ++run) {
+    const uint32_t next = k0 + W * BK;
     if (next < k_end) load(next, l_next, r_next);
 #pragma unroll
-    for (int part = 0; part < 2; ++part) {
+    for (int part = 0; part < kParts; ++part) {
       u32x4 lp[kSplitPieces], rp[kSplitPieces];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -389,45 +431,44 @@ __global__ void __launch_bounds__(64 * kSmallWaves) gemm_small_kernel(const Gemm
       }
 #pragma unroll
       for (int i = 0; i < kSplitProducts; ++i) {
-        f32x16& to = sums[i + 1 < kSplitProducts];
-        to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lp[kSplitLeft[i]]),
-                                                     __builtin_bit_cast(bf16x8, rp[kSplitRight[i]]), to, 0, 0, 0);
+        Cells& to = sums[i + 1 < kSplitProducts];
+        to = Tile::product(__builtin_bit_cast(bf16x8, lp[kSplitLeft[i]]), __builtin_bit_cast(bf16x8, rp[kSplitRight[i]]), to);
+      }
+    }
+    if constexpr (S == 16) {
+      if (run % kRunsToASum == kRunsToASum - 1) {   // behind the loads of the next run
+        add_up(run < kRunsToASum);
+        sums[0] = sums[1] = Cells{};
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E / 4; ++e) {
       l[e] = l_next[e];
       r[e] = r_next[e];
     }
   }
-  bool found = a.k == 1;   // a product by itself: the floats' is rounded once, and what the pieces leave out is not made up for
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const float sum = sums[0][e] + sums[1][e];
-    found |= not_finite(sum);
-    partial[wave][e * 64 + lane] = sum * kSplitUnscale;
-  }
+  if (S == 32 || run % kRunsToASum > 0 || run == 0) add_up(S == 32 || run < kRunsToASum);
   if (__syncthreads_or(found)) {
-    f32x16 total = zero16();
-    for (uint32_t k0 = k_mine; k0 < k_end; k0 += kSmallWaves * BK) {
+    Cells total = {};
+    for (uint32_t k0 = k_mine; k0 < k_end; k0 += W * BK) {
       load(k0, l, r);
-      f32x16 sum = zero16();
+      Cells sum = {};
 #pragma unroll
-      for (int e = 0; e < 16; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(l[e / 4][e % 4], r[e / 4][e % 4], sum, 0, 0, 0);
+      for (int e = 0; e < E; ++e) sum = Tile::product_in_float(l[e / 4][e % 4], r[e / 4][e % 4], sum);
       total += sum;
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) partial[wave][e * 64 + lane] = total[e];
+    for (int e = 0; e < kCells; ++e) partial[wave][e * 64 + lane] = total[e];
     __syncthreads();
   }
   float* c = a.c + (int64_t)place.split * a.c_split + (int64_t)place.batch * a.c_batch;
 #pragma unroll
-  for (uint32_t i = threadIdx.x; i < 1024; i += 64 * kSmallWaves) {
+  for (uint32_t i = threadIdx.x; i < S * S; i += 64 * W) {
     const uint32_t e = i / 64, at_lane = i % 64;
-    const uint32_t cm = place.m_tile * 32 + 8 * (e / 4) + 4 * (at_lane / 32) + e % 4, cn = place.n_tile * 32 + at_lane % 32;
+    const uint32_t cm = place.m_tile * S + 8 * (e / 4) + 4 * (at_lane / S) + e % 4, cn = place.n_tile * S + at_lane % S;
     float sum = partial[0][i];
 #pragma unroll
-    for (int w = 1; w < kSmallWaves; ++w) sum += partial[w][i];
+    for (int w = 1; w < W; ++w) sum += partial[w][i];
     if (cm >= a.m || cn >= a.n) continue;
     float& cell = c[(int64_t)cm * a.ldc + cn];
     const float value = a.alpha * sum;
@@ -448,17 +489,21 @@ __global__ void __launch_bounds__(256) gemm_sum_kernel(const float* partial, flo
   cell = (float)(beta == 0.f ? alpha * sum : alpha * sum + (double)(beta * cell));
 }
 
-enum Tile { kSmall, kMedium, kMediumPair, kLarge };
+enum Tile { kFine, kSmallHalf, kSmall, kMedium, kMediumPair, kLarge };
 struct TileShape {
   int rows, columns, groups, group_threads;
 };
-constexpr TileShape kTiles[] = {{32, 32, 1, 64 * kSmallWaves}, {64, 64, 1, 256}, {64, 64, 2, 256}, {128, 128, 1, 512}};
+constexpr TileShape kTiles[] = {{16, 16, 1, 64 * 8}, {32, 32, 1, 64 * 8}, {32, 32, 1, 64 * 16}, {64, 64, 1, 256}, {64, 64, 2, 256},
+                                {128, 128, 1, 512}};
+constexpr bool is_small(Tile tile) { return tile < kMedium; }
 
 template <bool kA, bool kB>
 void launch(hipStream_t s, const GemmArgs& a, Tile tile) {
   const dim3 grid((a.units + kXcds - 1) / kXcds * kXcds), block(kTiles[tile].groups * kTiles[tile].group_threads);
   switch (tile) {
-    case kSmall: hipLaunchKernelGGL((gemm_small_kernel<kA, kB>), grid, block, 0, s, a); break;
+    case kFine: hipLaunchKernelGGL((gemm_small_kernel<16, 8, kA, kB>), grid, block, 0, s, a); break;
+    case kSmallHalf: hipLaunchKernelGGL((gemm_small_kernel<32, 8, kA, kB>), grid, block, 0, s, a); break;
+    case kSmall: hipLaunchKernelGGL((gemm_small_kernel<32, 16, kA, kB>), grid, block, 0, s, a); break;
     case kMedium: hipLaunchKernelGGL((gemm_kernel<64, 64, 2, 2, 1, kA, kB>), grid, block, 0, s, a); break;
     case kMediumPair: hipLaunchKernelGGL((gemm_kernel<64, 64, 2, 2, 2, kA, kB>), grid, block, 0, s, a); break;
     case kLarge: hipLaunchKernelGGL((gemm_kernel<128, 128, 2, 4, 1, kA, kB>), grid, block, 0, s, a); break;
@@ -476,16 +521,24 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 Plan plan_of(Tile tile, int64_t splits, int64_t k) {
   const TileShape& t = kTiles[tile];
-  const int64_t k_tiles = ceil_div(k, 32), unit = tile == kSmall ? 1 : 2 * t.groups;   // a group's tiles come in pairs
+  const int64_t k_tiles = ceil_div(k, 32), unit = is_small(tile) ? 1 : 2 * t.groups;   // a group's tiles come in pairs
   const int64_t per_split = ceil_div(ceil_div(k_tiles, splits), unit) * unit;
   return {tile, ceil_div(k_tiles, per_split), per_split / t.groups};
+}
+
+constexpr int64_t kUnits = 256;
+
+// The launch of a sum, and its bytes at 3.3 TB/s.
+double sum_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
+  return p.splits > 1 ? 2.5 + 1.2e-6 * (double)((p.splits + 1) * m * n * batch) : 0.0;
 }
 
 // What a plan is expected to take, in microseconds: lines through the times of 420 products of 1 to 4096 a side in all
 // four layouts, 95 % of which lie within 0.8 to 1.2 of them.  A unit holds one block (three of kMedium, whose steps then
 // take longer); blocks beyond the chip's units wait for a round of their own.
+// The line of the small kernel is that of a block of sixteen waves to 32 x 32, which was timed with the others.  The plans
+// that run in its place are faster (best_small_plan); the lines to the other kernels lie where that one left them.
 double expected_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
-  constexpr int64_t kUnits = 256;
   const TileShape& t = kTiles[p.tile];
   const int64_t blocks = ceil_div(m, t.rows) * ceil_div(n, t.columns) * batch * p.splits;
   double us;
@@ -494,35 +547,69 @@ double expected_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
     us = 3.3 + 1.3 * (double)shared + (double)p.tiles_per_group * (0.31 * (double)(full + (rest > 0)) + 0.33 * (double)shared);
   } else {
     const double rounds = (double)ceil_div(blocks, kUnits);
-    if (p.tile == kSmall) us = 2.0 + rounds * 3.0 * (double)ceil_div(p.tiles_per_group, kSmallWaves);
+    if (p.tile == kSmall) us = 2.0 + rounds * 3.0 * (double)ceil_div(p.tiles_per_group, 16);
     else if (p.tile == kMediumPair) us = 1.2 + rounds * (3.9 + 0.87 * (double)p.tiles_per_group);
     else us = 1.8 + rounds * (3.7 + 1.19 * (double)p.tiles_per_group);
   }
-  // the sum: its launch on the device and on the host, and its bytes at 3.3 TB/s
-  if (p.splits > 1) us += 2.5 + 2.0 + 1.2e-6 * (double)((p.splits + 1) * m * n * batch);
-  return us;
+  constexpr double kHostOfALaunch = 2.0;
+  return us + sum_time(p, m, n, batch) + (p.splits > 1 ? kHostOfALaunch : 0.0);
 }
 
-Plan best_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
-  struct Candidate {
-    Tile tile;
-    int64_t splits;
-  };
-  constexpr Candidate kCandidates[] = {{kSmall, 1}, {kSmall, 2}, {kMedium, 1}, {kMediumPair, 1}, {kMediumPair, 2},
-                                       {kMediumPair, 4}, {kMediumPair, 8}, {kLarge, 1}, {kLarge, 2}, {kLarge, 4}};
+struct Candidate {
+  Tile tile;
+  int64_t splits;
+};
+
+bool may_be(const Plan& p, const Candidate& c, int64_t m, int64_t n, int64_t batch, bool may_split) {
+  if (p.splits != c.splits) return false;
+  return p.splits == 1 || (may_split && batch == 1 && p.splits * m * n * (int64_t)sizeof(float) <= (int64_t)kMostProductScratch);
+}
+
+// The tile of the small kernel, its waves and its splits.  The splitting bounds it (4.5 vector instructions a float): a tile
+// of 16 x 16 splits half the floats that one of 32 x 32 does, for a quarter of the products, and four times the units share the
+// work.  Eight waves to a tile leave room for two and more to a unit.  Blocks that share a unit add their times, long runs of
+// 16 x 16 a little more.  Lines through 8000 times of 2200 products, 96 % of which lie within 0.82 to 1.15 of them.  Us, 16 x 16,
+// 32 x 32 under eight waves and under sixteen (which was all there was): [3, 8] over 1505 6.2, 10.3, 9.8; [1417, 11] over 3308
+// 11.5, 21.4, 19.9; [178, 478] over 1316 10.9, 12.0, 11.6; [2940, 308] over 93 11.4, 8.5, 13.2; [2538, 17] over 3033, with a
+// second launch for the sum of two halves, 14.2 in place of 22.4.
+Plan best_small_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
+  constexpr Candidate kCandidates[] = {{kFine, 1}, {kSmallHalf, 1}, {kSmall, 1}, {kSmall, 2}};
+  constexpr double kShortRuns = 5.0;
   Plan best = plan_of(kSmall, 1, k);
   double best_us = -1.0;
   for (const Candidate& c : kCandidates) {
     const Plan p = plan_of(c.tile, c.splits, k);
-    if (p.splits != c.splits || (p.tile != kSmall && k < 32)) continue;
-    if (p.splits > 1 && (!may_split || batch > 1 || p.splits * m * n * (int64_t)sizeof(float) > (int64_t)kMostProductScratch)) continue;
-    const double us = expected_time(p, m, n, batch);
+    const TileShape& t = kTiles[p.tile];
+    const double runs = (double)p.tiles_per_group / (t.group_threads / 64);
+    if (!may_be(p, c, m, n, batch, may_split) || (p.tile == kSmallHalf && runs > kRunsToASum)) continue;
+    const double shared = (double)ceil_div(ceil_div(m, t.rows) * ceil_div(n, t.columns) * batch * p.splits, kUnits);
+    double us = sum_time(p, m, n, batch);
+    if (p.tile == kSmall) us += 1.3 + shared * (2.5 + 2.3 * runs);
+    else if (p.tile == kSmallHalf) us += 2.7 + shared * (1.06 + 1.24 * runs);
+    else us += 2.7 + shared * (0.41 + 0.57 * runs + (shared > 1.0 ? 0.3 * std::max(0.0, runs - kShortRuns) : 0.0));
     if (best_us < 0.0 || us < best_us) {
       best = p;
       best_us = us;
     }
   }
   return best;
+}
+
+Plan best_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
+  constexpr Candidate kCandidates[] = {{kSmall, 1}, {kSmall, 2}, {kMedium, 1}, {kMediumPair, 1}, {kMediumPair, 2},
+                                       {kMediumPair, 4}, {kMediumPair, 8}, {kLarge, 1}, {kLarge, 2}, {kLarge, 4}};
+  Plan best = plan_of(kSmall, 1, k);
+  double best_us = -1.0;
+  for (const Candidate& c : kCandidates) {
+    const Plan p = plan_of(c.tile, c.splits, k);
+    if (!may_be(p, c, m, n, batch, may_split) || (!is_small(p.tile) && k < 32)) continue;
+    const double us = expected_time(p, m, n, batch);
+    if (best_us < 0.0 || us < best_us) {
+      best = p;
+      best_us = us;
+    }
+  }
+  return is_small(best.tile) ? best_small_plan(m, n, k, batch, may_split) : best;
 }
 
 bool overlap(const float* a, int64_t a_count, const float* b, int64_t b_count) {
@@ -541,7 +628,9 @@ namespace cthip {
 // Not taken: fewer than 32 k over more tiles than one round of the small kernel (the tiles of the others have 32;
 // [1846, 1794] over 23 k 35 us here, 9 there), and what 32-bit indexes do not hold.
 bool gemm_split_takes(const GemmProduct& p) {
-  constexpr int64_t kMostLd = int64_t(1) << 22, kMostTiles = int64_t(1) << 22, kMostCells = (int64_t(1) << 31) - 1;
+  constexpr int64_t kMostLd = int64_t(1) << 22, kMostTiles = int64_t(1) << 21, kMostCells = (int64_t(1) << 31) - 1;
+  // a single row of tiles has two of 16 x 16 to each; where there are more rows and so many tiles, 32 x 32 is taken
+  static_assert(kMostTiles * 2 * 64 * 8 < int64_t(1) << 32, "a launch of 2^32 lanes or more is refused");
   if (p.m < 1 || p.n < 1 || p.k < 1 || p.batch < 1 || p.alpha == 0.f) return false;
   if (p.lda > kMostLd || p.ldb > kMostLd || p.m * p.n > kMostCells) return false;
   const int64_t small_tiles = ceil_div(p.m, 32) * ceil_div(p.n, 32) * p.batch;
@@ -590,9 +679,9 @@ int gemm_split(hipStream_t s, const GemmProduct& p) {
     hipLaunchKernelGGL(gemm_sum_kernel, dim3((cells + 255) / 256), dim3(256), 0, s, partial, p.c, (uint32_t)p.n, p.ldc, cells,
                        (uint32_t)plan.splits, p.alpha, p.beta, FastDiv((uint32_t)p.n));
   }
-  static const char* const kNames[] = {"gemm_small", "gemm_medium", "gemm_medium_pair", "gemm_large"};
-  static const char* const kSplitNames[] = {"gemm_small+gemm_sum", "gemm_medium+gemm_sum", "gemm_medium_pair+gemm_sum",
-                                            "gemm_large+gemm_sum"};
+  static const char* const kNames[] = {"gemm_small", "gemm_small", "gemm_small", "gemm_medium", "gemm_medium_pair", "gemm_large"};
+  static const char* const kSplitNames[] = {"gemm_small+gemm_sum",  "gemm_small+gemm_sum",       "gemm_small+gemm_sum",
+                                            "gemm_medium+gemm_sum", "gemm_medium_pair+gemm_sum", "gemm_large+gemm_sum"};
   note_kernel(partial ? kSplitNames[plan.tile] : kNames[plan.tile]);
   return after_launch(s);
 }

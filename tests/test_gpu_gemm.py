@@ -35,6 +35,12 @@ EDGES = [(1, 1, 1), (3, 2, 5), (31, 33, 31), (32, 32, 32), (33, 31, 33), (64, 65
          (1040, 1025, 129), (1025, 1040, 290), (2050, 1100, 130), (300, 500, 1100), (130, 70, 3000), (1152, 1030, 550)]
 
 
+# the small kernel: tiles of 16 x 16, whose eight waves take 256 k between them, in one run, in two and a remainder, and with
+# partial sums; of 32 x 32 over more of them
+EDGES += [(16, 16, 256), (15, 17, 255), (17, 15, 257), (33, 16, 511), (1, 49, 513), (47, 1, 288), (10, 30, 2600), (640, 450, 255),
+          (650, 430, 257), (417, 801, 480)]
+
+
 @pytest.mark.parametrize("ta", [False, True])
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("size", EDGES, ids=str)
@@ -51,7 +57,7 @@ def test_whole_numbers_are_exact(P, size, ta, tb):
 
 KERNELS = {(40, 40, 100): "gemm_small", (10, 20, 3700): "gemm_medium_pair+gemm_sum", (640, 640, 50): "gemm_medium",
            (900, 900, 400): "gemm_medium_pair", (2048, 2048, 256): "gemm_large", (64, 2048, 4096): "gemm_medium_pair+gemm_sum",
-           (1024, 1536, 2048): "gemm_large+gemm_sum", (2000, 2000, 20): "rocblas_gemm"}
+           (1024, 1536, 2048): "gemm_large+gemm_sum", (2000, 2000, 20): "rocblas_gemm", (650, 450, 255): "gemm_small"}
 
 
 @pytest.mark.parametrize("size", KERNELS, ids=str)
@@ -74,7 +80,8 @@ def test_error_is_below_a_plain_sum_s(P, size):
         assert np.linalg.norm(got[some] - exact) <= 0.5 * np.linalg.norm(plain - exact)
 
 
-@pytest.mark.parametrize("size", [(40, 50, 100), (640, 640, 50), (900, 900, 400), (2048, 2048, 256), (64, 2048, 4096)], ids=str)
+@pytest.mark.parametrize("size", [(40, 50, 100), (640, 640, 50), (900, 900, 400), (2048, 2048, 256), (64, 2048, 4096), (650, 450, 255)],
+                         ids=str)
 def test_the_ends_of_the_number_range(P, size):
     """Infinities, NaN, and floats and results beyond what the pieces hold: the block forms its sums again from the floats.
     The oracle sums in double and rounds once; bar: 1e-5 of the sum of magnitudes and, where that is
