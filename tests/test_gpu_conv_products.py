@@ -344,7 +344,56 @@ def test_products_in_pieces_over_low_images(P, case):
     check_products(P, *case)
 
 
-@pytest.mark.parametrize("case", [(46, 8, 33, 40, 3), (41, 15, 20, 40, 3), (5, 20, 200, 19, 3)], ids=lambda c: "x".join(map(str, c)))
+def in_pieces(batch, m, k, n_rows, taps):
+    """Whether the output of m channels over k cells, its weight gradient and its input gradient are formed in pieces."""
+    n = batch * n_rows
+    forward = forward_route(batch, m, k, n_rows, taps) == "conv_product" and k >= 64 and -(-m // 64) * -(-n // 256) >= 288
+    pieces, fit = batch * -(-n_rows // 64), max(batch * max(1, min(64, n_rows // 4096)), (1 << 20) // (4 * m * k))
+    want = 1 if pieces <= 3 else max(1, min(512 // (-(-m // 64) * -(-k // 64)), fit, pieces))
+    weights = weight_route(batch, m, k, n_rows).startswith("conv_weight") and min(m, k) > 32 and -(-pieces // want) >= 6
+    data = k > 32 if m > 64 else m >= 20 and k >= 128 and n >= (8192 if k >= 512 else 65536)
+    return forward, weights, data_route(batch, k, m, n_rows) == "conv_product+conv_roll" and data
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_which_products_are_formed_in_pieces(P, case):
+    """Sums of one product of two floats and zeros: the float kernels and the library round it once.  The pieces leave out up to
+    2^-24 of it, and of the thousands of sums here some are rounded the other way."""
+    batch, cin, cout, side, k, stride = case
+    out_side = (side + 2 * (k // 2) - k) // stride + 1
+    n_rows, n_cols = out_side ** 2, cin * k * k
+    desc, geometry = H.conv_desc(cin, cout, k, k, k // 2, k // 2, stride, stride), (batch, side, side, out_side, out_side)
+    rng = np.random.default_rng(cin + cout)
+    normal = lambda *n: rng.standard_normal(n).astype(np.float32)
+    at = lambda n, below: rng.integers(0, below, n)
+    inp, work = P.buf(normal(batch * cin * side * side)), P.buf(normal(batch * n_rows * n_cols))
+    out, wg, ig = P.buf(normal(batch * cout * n_rows)), P.buf(normal(cout * n_cols)), P.buf(normal(batch * cin * side * side))
+
+    cell, one = at(cout, n_cols), normal(cout)
+    w = np.zeros((cout, n_cols), np.float32)
+    w[np.arange(cout), cell] = one
+    H.convolution(P.hip, "forward", vec(out), 0.0, vec(inp), vec(P.buf(w)), vec(work), desc, *geometry)
+    unrolled = work.download().reshape(batch, n_cols, n_rows)
+    got = [np.any(out.download().reshape(batch, cout, n_rows) != unrolled[:, cell] * one[None, :, None])]
+
+    image, position = at(cout, batch), at(cout, n_rows)
+    g = np.zeros((batch, cout, n_rows), np.float32)
+    g[image, np.arange(cout), position] = one
+    H.convolution(P.hip, "backward_weights", vec(wg), 0.0, vec(P.buf(g)), vec(inp), vec(work), desc, *geometry)
+    got.append(np.any(wg.download().reshape(cout, n_cols) != unrolled[image, :, position] * one[:, None]))
+
+    channel, w, ones = at(batch * n_rows, cout).reshape(batch, n_rows), normal(cout, n_cols), normal(batch, n_rows)
+    g = np.zeros((batch, cout, n_rows), np.float32)
+    np.put_along_axis(g, channel[:, None], ones[:, None], axis=1)
+    H.convolution(P.hip, "backward_data", vec(ig), 0.0, vec(P.buf(g)), vec(P.buf(w)), vec(work), desc, *geometry)
+    got.append(np.any(work.download().reshape(batch, n_cols, n_rows) != w.T[:, channel].transpose(1, 0, 2) * ones[:, None]))
+    assert tuple(map(bool, got)) == in_pieces(batch, cout, n_cols, n_rows, k * k)
+
+
+# Each kernel of the products in pieces: the output over 33 and over 31 channels, the weight gradient, the input gradient over
+# 20, 33, 66 and 65 channels (the last two in tiles of 64 and of 128 rows); and one that is formed in floats throughout
+@pytest.mark.parametrize("case", [(46, 8, 33, 40, 3), (30, 4, 31, 50, 5), (41, 15, 20, 40, 3), (7, 57, 33, 36, 3),
+                                  (3, 33, 66, 20, 1), (150, 11, 65, 23, 3), (6, 15, 129, 33, 3), (5, 20, 200, 19, 3)], ids=lambda c: "x".join(map(str, c)))
 def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
     """An infinity, a NaN and floats that the pieces do not hold, in the weights and in both gradients' operands: the blocks
     that meet them form their sums again from the floats.  Where the oracle's sums are finite the bar is 1e-5 of the sums of
@@ -355,11 +404,14 @@ def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
     rng = np.random.default_rng(cin)
     normal = lambda n: rng.standard_normal(n).astype(np.float32)
     x, w, g = normal(batch * cin * n_rows), normal(cout * n_cols), normal(batch * cout * n_rows)
-    x[5], x[7 * n_rows + 3], w[3], w[n_cols + 1], g[11], g[2 * n_rows + 1] = np.inf, 1e35, np.nan, -1e36, -np.inf, 3e35
+    x[5], x[3 * n_rows + 3], w[3], w[n_cols + 1], g[11], g[2 * n_rows + 1] = np.inf, 1e35, np.nan, -1e36, -np.inf, 3e35
     inp, weights, og = P.buf(x), P.buf(w), P.buf(g)
     out, wg, ig = P.buf(normal(batch * cout * n_rows)), P.buf(normal(cout * n_cols)), P.buf(normal(batch * cin * n_rows))
     work = P.buf(np.zeros(batch * n_rows * n_cols, np.float32))
-    clean = lambda v: np.abs(np.where(np.isfinite(v) & (np.abs(v) < 1e30), v, 0)).max()
+    ordinary = lambda v: np.where(np.isfinite(v) & (np.abs(v) < 1e30), v, 0).astype(np.float64)
+    largest = lambda v: np.abs(ordinary(v)).max()
+    # of the sums over the positions: by Cauchy and Schwarz, of the channels' norms
+    norm = lambda v, channels: np.sqrt((ordinary(v).reshape(batch, channels, n_rows) ** 2).sum(axis=(0, 2))).max()
 
     def check(buf, scale, what):
         got, want = buf.download().astype(np.float64), buf.host.astype(np.float64)
@@ -372,9 +424,27 @@ def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
         assert not np.all(np.isnan(want)) and plain.any(), what
 
     P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
-    check(out, clean(x) * clean(w) * n_cols, "convolution-forward")
+    check(out, largest(x) * largest(w) * n_cols, "convolution-forward")
     P.run(H.convolution, "backward_weights", vec(wg), 0.0, vec(og), vec(inp), vec(work), desc, *geometry)
-    got, want = wg.download(), wg.host
-    assert np.array_equal(np.isnan(got), np.isnan(want)), "convolution-backward-weights"
+    check(wg, norm(g, cout) * norm(x, cin), "convolution-backward-weights")
     P.run(H.convolution, "backward_data", vec(ig), 0.0, vec(og), vec(weights), vec(work), desc, *geometry)
-    check(ig, clean(g) * clean(w) * cout * k * k, "convolution-backward-data")
+    check(ig, largest(g) * largest(w) * cout * k * k, "convolution-backward-data")
+
+
+@pytest.mark.parametrize("exponent", [-118, -126, -133, -142])
+def test_products_in_pieces_of_small_operands(P, exponent):
+    """Floats of 24 bits around the least normal one, under weights near 2^100: the remainders that the pieces are cut from are
+    denormal.  The oracle sums in double; bar: 1e-6 of the sum of magnitudes."""
+    batch, cin, cout, side, k = 46, 8, 33, 40, 3
+    n_rows, n_cols = side * side, cin * k * k
+    desc, geometry = H.conv_desc(cin, cout, k, k, 1, 1, 1, 1), (batch, side, side, side, side)
+    rng = np.random.default_rng(-exponent)
+    full = lambda n, e: np.ldexp(rng.choice([-1.0, 1.0], n) * rng.integers(1 << 23, 1 << 24, n), e - 23).astype(np.float32)
+    inp, weights = P.buf(full(batch * cin * n_rows, exponent)), P.buf(full(cout * n_cols, 100))
+    out = P.buf(np.zeros(batch * cout * n_rows, np.float32))
+    work = P.buf(np.zeros(batch * n_rows * n_cols, np.float32))
+    assert in_pieces(batch, cout, n_cols, n_rows, k * k)[0]
+    P.run(H.convolution, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    unrolled = np.abs(work.download().reshape(batch, n_cols, n_rows)).astype(np.float64)
+    scale = np.matmul(np.abs(weights.init.reshape(cout, n_cols)).astype(np.float64), unrolled).reshape(-1)
+    assert np.all(np.abs(out.download().astype(np.float64) - out.host) <= 1e-6 * scale)

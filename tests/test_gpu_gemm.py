@@ -123,6 +123,21 @@ def test_outer_products_are_the_floats_products(P, size, ta, tb):
     H.assert_bit_exact(got, want, kernel)
 
 
+@pytest.mark.parametrize("size", [(40, 50, 100), (640, 640, 64), (650, 450, 255)], ids=str)
+@pytest.mark.parametrize("exponent", [-118, -126, -133, -142])
+def test_small_operands(P, exponent, size):
+    """Floats of 24 bits around the least normal one, by floats near 2^100: the remainders that the pieces are cut from are
+    denormal.  The oracle sums in double; bar: 1e-6 of the sum of magnitudes."""
+    m, n, k = size
+    rng = np.random.default_rng(m)
+    full = lambda s, e: np.ldexp(rng.choice([-1.0, 1.0], s) * rng.integers(1 << 23, 1 << 24, s), e - 23).astype(np.float32)
+    a, b = full((m, k), exponent), full((n, k), 100)
+    kernel, got, want = run(P, a, b, np.zeros((m, n), np.float32), False, True, m, n, k)
+    assert kernel.startswith("gemm_"), kernel
+    scale = np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64)).T
+    assert np.all(np.abs(got.astype(np.float64) - want) <= 1e-6 * scale), kernel
+
+
 @pytest.mark.parametrize("exponent", [-135, -100, 60])
 def test_scaled_operands_scale_the_result(P, exponent):
     """Multiplying an operand by a power of two multiplies the result, to the bit, as long as neither leaves the floats:
