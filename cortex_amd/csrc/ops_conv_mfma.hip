@@ -721,7 +721,7 @@ template <int BM>
 __global__ void __launch_bounds__(BM == 128 ? 512 : 256, 2) conv_data_kernel(const ConvProductArgs a) {
   constexpr int T = BM == 128 ? 512 : 256, BN = 128, BK = 32, WM = BM / 32, WN = T / 64 / WM, NT = BN / WN / 32;
   constexpr int kStep = BK * BN / T, kRuns = kStep / 8;   // k of a column of `right` that a lane stages, in runs of eight
-  constexpr int kLeftChunks = BM * BK / 8;
+  static_assert(BM * BK / 8 == T, "a run of eight k of the left operand to a lane");
   constexpr int kPlane = (BM + BN) * BK, kBuffer = kSplitPieces * kPlane;
   constexpr uint32_t kTilesToASum = 4;
   __shared__ __attribute__((aligned(16))) uint16_t lds[2 * kBuffer];   // [buffer][piece][rows of the left, of the right operand]
@@ -743,12 +743,11 @@ __global__ void __launch_bounds__(BM == 128 ? 512 : 256, 2) conv_data_kernel(con
   const uint32_t from = (image * (uint32_t)a.out_image + pos) * 4;
 
   const uint32_t left_row = tid % BM, left_chunk = tid / BM;
-  const bool stages_left = kLeftChunks >= T || tid < kLeftChunks;
   const float* weights = a.weights + min(m_tile * BM + left_row, a.m - 1);
   f32x4 left_raw[2];
   float right_raw[kStep];
   auto load_left = [&](uint32_t k0) {
-    const uint32_t k = min(k0, (a.k - 1) / BK * BK) + (kLeftChunks >= T ? left_chunk : left_chunk & 3) * 8;
+    const uint32_t k = min(k0, (a.k - 1) / BK * BK) + left_chunk * 8;
     // the weights as stored are [k][m]: consecutive lanes take consecutive m
 #pragma unroll
     for (uint32_t e = 0; e < 8; ++e) left_raw[e / 4][e % 4] = weights[(int64_t)min(k + e, a.k - 1) * a.m];
@@ -790,7 +789,6 @@ __global__ void __launch_bounds__(BM == 128 ? 512 : 256, 2) conv_data_kernel(con
       u32x4 pieces[kSplitPieces];
       split4(left_raw[0], pieces, 0, split_weights);
       split4(left_raw[1], pieces, 4, split_weights);
-      if (!stages_left) return;
 #pragma unroll
       for (int p = 0; p < kSplitPieces; ++p) *reinterpret_cast<u32x4*>(buffer + p * kPlane + stage_left_at) = pieces[p];
     };
@@ -914,10 +912,8 @@ __global__ void __launch_bounds__(BM == 128 ? 512 : 256, 2) conv_data_kernel(con
     for (uint32_t k0 = 0; k0 < a.k; k0 += BK) {
       load_left(k0);
       drop_left(k0);
-      if (stages_left) {
-        *reinterpret_cast<f32x4*>(left_lds + left_row * LD + left_chunk * 8) = left_raw[0];
-        *reinterpret_cast<f32x4*>(left_lds + left_row * LD + left_chunk * 8 + 4) = left_raw[1];
-      }
+      *reinterpret_cast<f32x4*>(left_lds + left_row * LD + left_chunk * 8) = left_raw[0];
+      *reinterpret_cast<f32x4*>(left_lds + left_row * LD + left_chunk * 8 + 4) = left_raw[1];
 #pragma unroll
       for (int run = 0; run < kRuns; ++run) {
         load_right(k0, run);
@@ -1427,10 +1423,9 @@ void conv_product_split(hipStream_t s, ConvProductArgs a, bool forward) {
     else if (past) hipLaunchKernelGGL((conv_data_few_kernel<4, true>), blocks, block, 0, s, a);
     else hipLaunchKernelGGL((conv_data_few_kernel<4, false>), blocks, block, 0, s, a);
   } else {
-    const int bm = tile_rows(a.m);
+    const int bm = tile_rows(a.m);   // more than 32 rows: 64 or 128
     const dim3 blocks = grid((a.m + bm - 1) / bm, 128);
-    if (bm == 32) hipLaunchKernelGGL((conv_data_kernel<32>), blocks, dim3(256), 0, s, a);
-    else if (bm == 64) hipLaunchKernelGGL((conv_data_kernel<64>), blocks, dim3(256), 0, s, a);
+    if (bm == 64) hipLaunchKernelGGL((conv_data_kernel<64>), blocks, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((conv_data_kernel<128>), blocks, dim3(512), 0, s, a);
   }
 }
