@@ -5,13 +5,13 @@
 
 namespace cthip {
 
-// c[i] = alpha * a[i] b[i] + beta * c[i] for i < batch: a [m, k], stored so if row_major_a, else [k, m]; b [k, n], stored
-// [n, k] if row_major_b, else as it is.
+// c = alpha * a b + beta * c: a [m, k], stored so if row_major_a, else [k, m]; b [k, n], stored [n, k] if row_major_b, else
+// as it is.
 struct GemmProduct {
   const float* a;
   const float* b;
   float* c;
-  int64_t lda, ldb, ldc, a_batch, b_batch, c_batch, m, n, k, batch;
+  int64_t lda, ldb, ldc, m, n, k;
   bool row_major_a, row_major_b;
   float alpha, beta;
 };

@@ -179,8 +179,8 @@ int ct_gemm(void* stream, void* c, int64_t c_colstride, int trans_a, int trans_b
   CT_REQUIRE(b_colstride >= (trans_b ? a_col_count : b_col_count), "ct_gemm: B column stride is shorter than its rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == CT_F32) {
-    const GemmProduct p{(const float*)a, (const float*)b, (float*)c, a_colstride, b_colstride, c_colstride, 0, 0, 0, a_row_count,
-                        b_col_count, a_col_count, 1, !trans_a, trans_b != 0, (float)alpha, (float)beta};
+    const GemmProduct p{(const float*)a, (const float*)b, (float*)c, a_colstride, b_colstride, c_colstride, a_row_count,
+                        b_col_count, a_col_count, !trans_a, trans_b != 0, (float)alpha, (float)beta};
     if (gemm_split_takes(p)) return gemm_split(s, p);
   }
   RocblasApi* api;

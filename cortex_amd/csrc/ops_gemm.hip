@@ -34,12 +34,12 @@ __device__ __forceinline__ uint32_t tile_at(uint32_t row, uint32_t chunk) { retu
 struct GemmArgs {
   const float* a;
   const float* b;
-  float* c;              // the result, or partial[split][batch][m][n]
-  int64_t lda, ldb, ldc, a_batch, b_batch, c_batch, c_split;
+  float* c;              // the result, or partial[split][m][n]
+  int64_t lda, ldb, ldc, c_split;
   uint32_t m, n, k, m_tiles, n_tiles, units;
   uint32_t tiles_per_group;   // of k; an even number
   float alpha, beta;
-  FastDiv tiles_fd, group_fd, batch_fd;
+  FastDiv tiles_fd, group_fd;
 };
 
 // Consecutive units of work on one die: neighbouring tiles share operands in its L2.
@@ -53,14 +53,13 @@ __device__ __forceinline__ uint32_t unit_of_block(uint32_t b, uint32_t units) {
 constexpr uint32_t kGroup = 8;
 
 struct Place {
-  uint32_t split, batch, m_tile, n_tile;
+  uint32_t split, m_tile, n_tile;
 };
 
 __device__ __forceinline__ Place place_of(const GemmArgs& a, uint32_t unit) {
   Place p;
   uint32_t rest, tile, group;
-  a.tiles_fd.divmod(unit, rest, tile);
-  a.batch_fd.divmod(rest, p.split, p.batch);
+  a.tiles_fd.divmod(unit, p.split, tile);
   a.group_fd.divmod(tile, group, rest);
   const uint32_t rows = min(kGroup, a.m_tiles - group * kGroup);
   p.n_tile = rest / rows;
@@ -114,8 +113,8 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) gemm_kernel(const GemmAr
                                                        : ((i < UA ? i : i - UA) * T + tid) % (i < UA ? BM : BN); };
   auto chunk_of = [&](int i) { return (i < UA ? kA : kB) ? ((i < UA ? i : i - UA) * T + tid) % kChunks
                                                          : ((i < UA ? i : i - UA) * T + tid) / (i < UA ? BM : BN); };
-  const float* base_a = a.a + (int64_t)place.batch * a.a_batch + (int64_t)(place.m_tile * BM) * (kA ? a.lda : 1);
-  const float* base_b = a.b + (int64_t)place.batch * a.b_batch + (int64_t)(place.n_tile * BN) * (kB ? a.ldb : 1);
+  const float* base_a = a.a + (int64_t)(place.m_tile * BM) * (kA ? a.lda : 1);
+  const float* base_b = a.b + (int64_t)(place.n_tile * BN) * (kB ? a.ldb : 1);
   uint32_t offset[U];
 #pragma unroll
   for (int i = 0; i < U; ++i) {
@@ -307,7 +306,7 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) gemm_kernel(const GemmAr
         result[e / (NT * 16)][e / 16 % NT][e % 16] += reinterpret_cast<const float*>(all_lds[g])[e * T + tid];
   }
 
-  float* c = a.c + (int64_t)place.split * a.c_split + (int64_t)place.batch * a.c_batch;
+  float* c = a.c + (int64_t)place.split * a.c_split;
 #pragma unroll
   for (int u = 0; u < NT; ++u) {
     const uint32_t n = place.n_tile * BN + wave_n + u * 32 + row;
@@ -380,8 +379,8 @@ __global__ void __launch_bounds__(64 * W, 4) gemm_small_kernel(const GemmArgs a)
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t k_first = place.split * a.tiles_per_group * BK, k_end = min(a.k, k_first + a.tiles_per_group * BK);
   const uint32_t m = min(place.m_tile * S + row, a.m - 1), n = min(place.n_tile * S + row, a.n - 1);
-  const float* left = a.a + (int64_t)place.batch * a.a_batch + (kA ? (int64_t)m * a.lda : m);
-  const float* right = a.b + (int64_t)place.batch * a.b_batch + (kB ? (int64_t)n * a.ldb : n);
+  const float* left = a.a + (kA ? (int64_t)m * a.lda : m);
+  const float* right = a.b + (kB ? (int64_t)n * a.ldb : n);
   // a lane's k of a run: 8 * group + 0 .. 7 and, in two parts, 16 more
   auto load = [&](uint32_t k0, f32x4 (&l)[E / 4], f32x4 (&r)[E / 4]) {
     if (k0 + BK <= k_end) {
@@ -461,7 +460,7 @@ __global__ void __launch_bounds__(64 * W, 4) gemm_small_kernel(const GemmArgs a)
     for (int e = 0; e < kCells; ++e) partial[wave][e * 64 + lane] = total[e];
     __syncthreads();
   }
-  float* c = a.c + (int64_t)place.split * a.c_split + (int64_t)place.batch * a.c_batch;
+  float* c = a.c + (int64_t)place.split * a.c_split;
 #pragma unroll
   for (uint32_t i = threadIdx.x; i < S * S; i += 64 * W) {
     const uint32_t e = i / 64, at_lane = i % 64;
@@ -529,8 +528,8 @@ Plan plan_of(Tile tile, int64_t splits, int64_t k) {
 constexpr int64_t kUnits = 256;
 
 // The launch of a sum, and its bytes at 3.3 TB/s.
-double sum_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
-  return p.splits > 1 ? 2.5 + 1.2e-6 * (double)((p.splits + 1) * m * n * batch) : 0.0;
+double sum_time(const Plan& p, int64_t m, int64_t n) {
+  return p.splits > 1 ? 2.5 + 1.2e-6 * (double)((p.splits + 1) * m * n) : 0.0;
 }
 
 // What a plan is expected to take, in microseconds: lines through the times of 420 products of 1 to 4096 a side in all
@@ -538,9 +537,9 @@ double sum_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
 // take longer); blocks beyond the chip's units wait for a round of their own.
 // The line of the small kernel is that of a block of sixteen waves to 32 x 32, which was timed with the others.  The plans
 // that run in its place are faster (best_small_plan); the lines to the other kernels lie where that one left them.
-double expected_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
+double expected_time(const Plan& p, int64_t m, int64_t n) {
   const TileShape& t = kTiles[p.tile];
-  const int64_t blocks = ceil_div(m, t.rows) * ceil_div(n, t.columns) * batch * p.splits;
+  const int64_t blocks = ceil_div(m, t.rows) * ceil_div(n, t.columns) * p.splits;
   double us;
   if (p.tile == kMedium) {
     const int64_t full = blocks / (3 * kUnits), rest = blocks - full * 3 * kUnits, shared = full * 3 + ceil_div(rest, kUnits);
@@ -552,7 +551,7 @@ double expected_time(const Plan& p, int64_t m, int64_t n, int64_t batch) {
     else us = 1.8 + rounds * (3.7 + 1.19 * (double)p.tiles_per_group);
   }
   constexpr double kHostOfALaunch = 2.0;
-  return us + sum_time(p, m, n, batch) + (p.splits > 1 ? kHostOfALaunch : 0.0);
+  return us + sum_time(p, m, n) + (p.splits > 1 ? kHostOfALaunch : 0.0);
 }
 
 struct Candidate {
@@ -560,9 +559,9 @@ struct Candidate {
   int64_t splits;
 };
 
-bool may_be(const Plan& p, const Candidate& c, int64_t m, int64_t n, int64_t batch, bool may_split) {
+bool may_be(const Plan& p, const Candidate& c, int64_t m, int64_t n, bool may_split) {
   if (p.splits != c.splits) return false;
-  return p.splits == 1 || (may_split && batch == 1 && p.splits * m * n * (int64_t)sizeof(float) <= (int64_t)kMostProductScratch);
+  return p.splits == 1 || (may_split && p.splits * m * n * (int64_t)sizeof(float) <= (int64_t)kMostProductScratch);
 }
 
 // The tile of the small kernel, its waves and its splits.  The splitting bounds it (4.5 vector instructions a float): a tile
@@ -572,7 +571,7 @@ bool may_be(const Plan& p, const Candidate& c, int64_t m, int64_t n, int64_t bat
 // 32 x 32 under eight waves and under sixteen (which was all there was): [3, 8] over 1505 6.2, 10.3, 9.8; [1417, 11] over 3308
 // 11.5, 21.4, 19.9; [178, 478] over 1316 10.9, 12.0, 11.6; [2940, 308] over 93 11.4, 8.5, 13.2; [2538, 17] over 3033, with a
 // second launch for the sum of two halves, 14.2 in place of 22.4.
-Plan best_small_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
+Plan best_small_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
   constexpr Candidate kCandidates[] = {{kFine, 1}, {kSmallHalf, 1}, {kSmall, 1}, {kSmall, 2}};
   constexpr double kShortRuns = 5.0;
   Plan best = plan_of(kSmall, 1, k);
@@ -581,9 +580,9 @@ Plan best_small_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_sp
     const Plan p = plan_of(c.tile, c.splits, k);
     const TileShape& t = kTiles[p.tile];
     const double runs = (double)p.tiles_per_group / (t.group_threads / 64);
-    if (!may_be(p, c, m, n, batch, may_split) || (p.tile == kSmallHalf && runs > kRunsToASum)) continue;
-    const double shared = (double)ceil_div(ceil_div(m, t.rows) * ceil_div(n, t.columns) * batch * p.splits, kUnits);
-    double us = sum_time(p, m, n, batch);
+    if (!may_be(p, c, m, n, may_split) || (p.tile == kSmallHalf && runs > kRunsToASum)) continue;
+    const double shared = (double)ceil_div(ceil_div(m, t.rows) * ceil_div(n, t.columns) * p.splits, kUnits);
+    double us = sum_time(p, m, n);
     if (p.tile == kSmall) us += 1.3 + shared * (2.5 + 2.3 * runs);
     else if (p.tile == kSmallHalf) us += 2.7 + shared * (1.06 + 1.24 * runs);
     else us += 2.7 + shared * (0.41 + 0.57 * runs + (shared > 1.0 ? 0.3 * std::max(0.0, runs - kShortRuns) : 0.0));
@@ -595,21 +594,21 @@ Plan best_small_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_sp
   return best;
 }
 
-Plan best_plan(int64_t m, int64_t n, int64_t k, int64_t batch, bool may_split) {
+Plan best_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
   constexpr Candidate kCandidates[] = {{kSmall, 1}, {kSmall, 2}, {kMedium, 1}, {kMediumPair, 1}, {kMediumPair, 2},
                                        {kMediumPair, 4}, {kMediumPair, 8}, {kLarge, 1}, {kLarge, 2}, {kLarge, 4}};
   Plan best = plan_of(kSmall, 1, k);
   double best_us = -1.0;
   for (const Candidate& c : kCandidates) {
     const Plan p = plan_of(c.tile, c.splits, k);
-    if (!may_be(p, c, m, n, batch, may_split) || (!is_small(p.tile) && k < 32)) continue;
-    const double us = expected_time(p, m, n, batch);
+    if (!may_be(p, c, m, n, may_split) || (!is_small(p.tile) && k < 32)) continue;
+    const double us = expected_time(p, m, n);
     if (best_us < 0.0 || us < best_us) {
       best = p;
       best_us = us;
     }
   }
-  return is_small(best.tile) ? best_small_plan(m, n, k, batch, may_split) : best;
+  return is_small(best.tile) ? best_small_plan(m, n, k, may_split) : best;
 }
 
 bool overlap(const float* a, int64_t a_count, const float* b, int64_t b_count) {
@@ -617,9 +616,7 @@ bool overlap(const float* a, int64_t a_count, const float* b, int64_t b_count) {
   return a0 < b0 + (uintptr_t)b_count * sizeof(float) && b0 < a0 + (uintptr_t)a_count * sizeof(float);
 }
 
-int64_t stored(int64_t rows, int64_t cols, int64_t ld, int64_t stride, int64_t batch) {
-  return (batch - 1) * stride + (rows - 1) * ld + cols;
-}
+int64_t stored(int64_t rows, int64_t cols, int64_t ld) { return (rows - 1) * ld + cols; }
 
 }  // namespace
 
@@ -631,29 +628,28 @@ bool gemm_split_takes(const GemmProduct& p) {
   constexpr int64_t kMostLd = int64_t(1) << 22, kMostTiles = int64_t(1) << 21, kMostCells = (int64_t(1) << 31) - 1;
   // a single row of tiles has two of 16 x 16 to each; where there are more rows and so many tiles, 32 x 32 is taken
   static_assert(kMostTiles * 2 * 64 * 8 < int64_t(1) << 32, "a launch of 2^32 lanes or more is refused");
-  if (p.m < 1 || p.n < 1 || p.k < 1 || p.batch < 1 || p.alpha == 0.f) return false;
+  if (p.m < 1 || p.n < 1 || p.k < 1 || p.alpha == 0.f) return false;
   if (p.lda > kMostLd || p.ldb > kMostLd || p.m * p.n > kMostCells) return false;
-  const int64_t small_tiles = ceil_div(p.m, 32) * ceil_div(p.n, 32) * p.batch;
+  const int64_t small_tiles = ceil_div(p.m, 32) * ceil_div(p.n, 32);
   if (small_tiles > kMostTiles || (p.k < 32 && small_tiles > 256)) return false;
-  const int64_t in_c = stored(p.m, p.n, p.ldc, p.c_batch, p.batch);
-  return !overlap(p.c, in_c, p.a, p.row_major_a ? stored(p.m, p.k, p.lda, p.a_batch, p.batch) : stored(p.k, p.m, p.lda, p.a_batch, p.batch)) &&
-         !overlap(p.c, in_c, p.b, p.row_major_b ? stored(p.n, p.k, p.ldb, p.b_batch, p.batch) : stored(p.k, p.n, p.ldb, p.b_batch, p.batch));
+  const int64_t in_c = stored(p.m, p.n, p.ldc);
+  return !overlap(p.c, in_c, p.a, p.row_major_a ? stored(p.m, p.k, p.lda) : stored(p.k, p.m, p.lda)) &&
+         !overlap(p.c, in_c, p.b, p.row_major_b ? stored(p.n, p.k, p.ldb) : stored(p.k, p.n, p.ldb));
 }
 
 int gemm_split(hipStream_t s, const GemmProduct& p) {
-  Plan plan = best_plan(p.m, p.n, p.k, p.batch, true);
+  Plan plan = best_plan(p.m, p.n, p.k, true);
   std::optional<ProductScratch> scratch;   // until both launches are made
   float* partial = nullptr;
   if (plan.splits > 1) {
     // no room, or none to be had while the stream is being captured: one launch
     scratch.emplace(s, (size_t)(plan.splits * p.m * p.n) * sizeof(float));
     partial = static_cast<float*>(scratch->get());
-    if (!partial) plan = best_plan(p.m, p.n, p.k, p.batch, false);
+    if (!partial) plan = best_plan(p.m, p.n, p.k, false);
   }
   GemmArgs a{};
   a.a = p.a; a.b = p.b; a.c = p.c;
   a.lda = p.lda; a.ldb = p.ldb; a.ldc = p.ldc;
-  a.a_batch = p.a_batch; a.b_batch = p.b_batch; a.c_batch = p.c_batch;
   a.m = (uint32_t)p.m; a.n = (uint32_t)p.n; a.k = (uint32_t)p.k;
   a.alpha = p.alpha; a.beta = p.beta;
   a.m_tiles = (uint32_t)ceil_div(p.m, kTiles[plan.tile].rows);
@@ -661,8 +657,7 @@ int gemm_split(hipStream_t s, const GemmProduct& p) {
   a.tiles_per_group = (uint32_t)plan.tiles_per_group;
   a.tiles_fd = FastDiv(a.m_tiles * a.n_tiles);
   a.group_fd = FastDiv(kGroup * a.n_tiles);
-  a.batch_fd = FastDiv((uint32_t)p.batch);
-  a.units = (uint32_t)(a.m_tiles * a.n_tiles * p.batch * plan.splits);
+  a.units = (uint32_t)(a.m_tiles * a.n_tiles * plan.splits);
   if (partial) {
     a.c = partial;
     a.ldc = p.n;
