@@ -494,20 +494,33 @@ int sort_index(hipStream_t s, const int32_t* index, uint32_t n, const int32_t** 
     *perm = k + n;
     return CT_OK;
   }
+  // the positions come from a counting iterator, so no array of them has to be written first
+  const size_t arrays = ((size_t)n * 4 + 255) / 256 * 256;
+  const rocprim::counting_iterator<int32_t> positions(0);
+  size_t temp_bytes = 0;
+  auto library_bytes = [&](size_t* bytes) -> int {
+    CT_HIP(rocprim::radix_sort_pairs(nullptr, temp_bytes, index, (int32_t*)nullptr, positions, (int32_t*)nullptr, n, 0u, 32u, s));
+    *bytes = 2 * arrays + temp_bytes;
+    return CT_OK;
+  };
+  size_t needed = 0;
   if (n > kSortMinEntries && n <= kSortMaxEntries) {
-    // two bytes an entry more than the library's sort; where a captured stream has only those, that one it is
-    block = stream_scratch_if_any(s, index_sort_bytes(n), kScratchAccumA);
+    // two bytes an entry more than the library's sort, for which no block that holds that one is replaced (a recorded graph
+    // may use it), nor where a stream that is being captured has no more
+    block = stream_scratch_held(s, index_sort_bytes(n), kScratchAccumA);
+    if (!block) {
+      if (int rc = library_bytes(&needed)) return rc;
+      if (!stream_scratch_held(s, needed, kScratchAccumA))
+        block = stream_scratch_if_any(s, index_sort_bytes(n), kScratchAccumA);
+    }
     if (block) {
       index_sort(s, index, n, block, skey, perm);
       return CT_OK;
     }
   }
-  // the positions come from a counting iterator, so no array of them has to be written first
-  size_t temp_bytes = 0;
-  const size_t arrays = ((size_t)n * 4 + 255) / 256 * 256;
-  const rocprim::counting_iterator<int32_t> positions(0);
-  CT_HIP(rocprim::radix_sort_pairs(nullptr, temp_bytes, index, (int32_t*)nullptr, positions, (int32_t*)nullptr, n, 0u, 32u, s));
-  if (int rc = stream_scratch(s, 2 * arrays + temp_bytes, &block, kScratchAccumA)) return rc;
+  if (!needed)
+    if (int rc = library_bytes(&needed)) return rc;
+  if (int rc = stream_scratch(s, needed, &block, kScratchAccumA)) return rc;
   char* base = static_cast<char*>(block);
   int32_t* k = reinterpret_cast<int32_t*>(base);
   int32_t* p = reinterpret_cast<int32_t*>(base + arrays);

@@ -273,3 +273,37 @@ def test_a_product_recorded_without_scratch_does_without(fresh):
         assert product(stream, c, a, b, m, n, k).endswith("+gemm_sum")
         assert np.array_equal(c.download(stream).reshape(m, n), host @ b.host.reshape(n, k).T), replay
     recorded.destroy()
+
+
+def test_a_recorded_sort_of_labels_keeps_its_scratch(fresh):
+    """Updates of 262144 rows chosen by labels, recorded on scratch that holds the library's sort of the labels (16 bytes an
+    entry) and not the kernels' own (18): eager calls between the replays take the block as it is.  Whole numbers."""
+    stream, tensor = fresh
+    n, classes = 262144, 5000
+    capi.call("ct_stream_reserve_scratch", stream, 0, 4600 << 10)
+    rng = np.random.default_rng(5)
+    labels, y = tensor(rng.integers(0, classes, n).astype(np.int32)), tensor(whole(rng, n))
+    sums = [tensor(np.zeros(classes, np.float32)) for _ in range(2)]
+    rows = [capi.make_dims([n, 1], [1, 1], [labels.ptr, None]) for _ in sums]
+    plain = dims([n, 1])
+
+    def add(side):
+        capi.call("ct_memset", stream, sums[side].ptr, capi.F32, 0.0, classes)
+        capi.call("ct_binary_accum", stream, sums[side].ptr, C.byref(rows[side]), 1.0, y.ptr, C.byref(plain), 1.0, n,
+                  capi.BINARY_OPS["+"], 0, 1, capi.F32)
+
+    add(0)
+    capi.call("ct_stream_sync", stream)
+    recorded = Recorded(hip_runtime(), stream, lambda: add(0))
+    for replay in range(4):
+        host_labels, host = rng.integers(0, classes, n).astype(np.int32), whole(rng, n)
+        labels.upload(host_labels, stream)
+        y.upload(host, stream)
+        if replay:
+            add(1)
+        recorded.replay()
+        want = np.bincount(host_labels, weights=host, minlength=classes).astype(np.float32)
+        assert np.array_equal(sums[0].download(stream), want), replay
+        if replay:
+            assert np.array_equal(sums[1].download(stream), want), replay
+    recorded.destroy()
