@@ -326,10 +326,13 @@ constexpr uint32_t kOutside = 0x80000000u;
 // A workspace that the last-level cache does not hold goes past the caches: a wave's loads wait for the stores in front of
 // them, and those for room in the caches ([64, 64, 56, 56] under 64 windows of 3 x 3, 462 MB, us: forward 207 -> 193, input
 // gradient with the roll back 248 -> 234; but [50, 248, 23, 23] under 21, 236 MB, which the roll back then reads from
-// memory, 98 -> 186).  At a stride the roll back skips about in the workspace and needs the caches ([109, 41, 80, 80] under 60
+// memory, 98 -> 186).  Only where the rows of the workspace begin on whole sectors of 64 bytes: others are written to memory in
+// parts, each read first ([132, 125, 41, 41] under 22 of 3 x 3, 1521 positions a row: input gradient 510 us, past the caches
+// 862; [65, 27, 63, 63] under 17 of 5 x 5, 3481: forward 238 and 278).  At a stride the roll back skips about in the workspace and needs the caches ([109, 41, 80, 80] under 60
 // of 5 x 5 at stride 2: input gradient 486 us, past the caches 641).
 constexpr int kStreaming = 2;
 constexpr int64_t kLastLevelCache = int64_t(256) << 20;
+constexpr uint32_t kWholeSectors = 16;
 template <bool kPast>
 __device__ __forceinline__ void store_cell(float x, __amdgpu_buffer_rsrc_t cells, uint32_t at, uint32_t row) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), cells, at, row, kPast ? kStreaming : 0);
@@ -1402,7 +1405,9 @@ void conv_product_split(hipStream_t s, ConvProductArgs a, bool forward) {
     return dim3((a.units + kXcds - 1) / kXcds * kXcds);
   };
   const dim3 block(kPositions);
-  const bool past = (int64_t)a.images * a.conv_image * (int64_t)sizeof(float) > kLastLevelCache && (forward || (a.sx == 1 && a.sy == 1));
+  const bool past = (int64_t)a.images * a.conv_image * (int64_t)sizeof(float) > kLastLevelCache &&
+                    a.n_rows % kWholeSectors == 0 && reinterpret_cast<uintptr_t>(a.workspace) % (kWholeSectors * sizeof(float)) == 0 &&
+                    (forward || (a.sx == 1 && a.sy == 1));
   if (forward) {
     const uint32_t bm = a.m <= 32 ? 32 : 64;
     const dim3 blocks = grid((a.m + bm - 1) / bm, kPositions);
