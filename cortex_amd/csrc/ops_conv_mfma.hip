@@ -1374,22 +1374,32 @@ void conv_product(hipStream_t s, ConvProductArgs a, bool forward) {
 // Forward (k cells): [98, 26, 46, 46] under 164 of 3 x 3 (k 234) 235 us with the float kernel, 179 here, [34, 30, 57, 57]
 // under 106 of 5 x 5 (750) 247 and 186, [60, 9, 28, 28] under 181 (81) 29 and 24; a tile has 32 k, which fewer than 64 do not
 // fill ([104, 1, 80, 80] under 54, 9 cells, 36 and 61), and blocks of 256 positions need to be enough to fill the chip
-// ([20, 17, 17, 17] under 31, 23 blocks, 13 and 16).
+// ([20, 17, 17, 17] under 31, 23 blocks, 13 and 16): the more the shorter the sums ([67, 8, 71, 71] under 19 at stride 2, k
+// 72, 321 blocks, 15.2 and 17.5; from 384 on 0.84 to 1.0 of the float kernel's time).  Of more than 32 rows two blocks share a
+// unit, and short sums are over before a last round of few blocks is ([115, 73, 26, 26] under 104 of 1 x 1, k 73, 602 blocks,
+// 25 and 29; 12 of 14 such shapes of 513 to 640 blocks and up to 112 cells 0.96 to 1.14).
 // Input gradient (k out channels): with many of them the general split kernel throughout ([32, 256, 14, 14] under 256 103
-// and 85, [134, 94, 15, 15] under 145 122 and 107, the least 0.98 times the float one's speed); with up to 64 the kernel
-// that keeps them in registers where the rows pay for that and the positions fill the chip ([64, 64, 56, 56] under 64, 576
-// rows, 214 and 124, without the roll back; [40, 8, 103, 103] under 33 of 1 x 1, 8 rows, 32 and 43; [1, 64, 56, 56] under
-// 64 15 and 17; [174, 172, 26, 26] under 36 of 1 x 1 at stride 2, 29406 positions, 63 and 68).
+// and 85, [134, 94, 15, 15] under 145 122 and 107; of 65 to 80, a third tile mostly idle, 0.96 to 1.08 of the float kernel's
+// time); with up to 64 the kernel that keeps them in registers where the rows pay for that and the positions fill the chip
+// ([64, 64, 56, 56] under 64, 576 rows, 214 and 124, without the roll back; [40, 8, 103, 103] under 33 of 1 x 1, 8 rows, 32
+// and 43; [174, 172, 26, 26] under 36 of 1 x 1 at stride 2, 29406 positions, 63 and 68).  Beyond 32 channels it holds 64, and
+// takes more than the float kernel over small workspaces (with the roll back: k 41 to 64, 20 to 33 MB 1.07 to 1.2 times as long
+// in 13 shapes of 14, 43 MB and more 0.82 to 1.05; k 33 to 40, up to 70 MB 0.98 to 1.15, mostly above 1, 73 MB and more
+// 0.91 to 1.02).
 bool conv_product_splits(int64_t m, int64_t n, int64_t k, bool forward) {
   if (forward) {
-    constexpr int64_t kFewCells = 64, kFewBlocks = 288;
+    constexpr int64_t kFewCells = 64, kShortSums = 96, kShortRounds = 112, kFewBlocks = 288, kFullChip = 384, kFullUnits = 512,
+                      kMostUneven = 640;
     const int64_t blocks = (m + 63) / 64 * ((n + kPositions - 1) / kPositions);
-    return k >= kFewCells && blocks >= kFewBlocks;
+    const bool uneven = m > 32 && blocks > kFullUnits && blocks <= kMostUneven;
+    return k >= kFewCells && blocks >= (k <= kShortSums ? kFullChip : kFewBlocks) && !(k <= kShortRounds && uneven);
   }
   constexpr int64_t kFewRows = 32;   // [104, 1, 50, 50] under 105 of 5 x 5, 25 rows, 37 and 43
   if (k > kFewChannels) return m > kFewRows;
   constexpr int64_t kLeastChannels = 20, kLeastRows = 128, kManyRows = 512, kLeastPositions = 8192, kManyPositions = 65536;
-  return k >= kLeastChannels && m >= kLeastRows && n >= (m >= kManyRows ? kLeastPositions : kManyPositions);
+  if (k < kLeastChannels || m < kLeastRows || n < (m >= kManyRows ? kLeastPositions : kManyPositions)) return false;
+  constexpr int64_t kHalfOfThem = 32, kMostIdle = 40, kLeastCells = int64_t(10) << 20, kManyCells = int64_t(18) << 20;
+  return k <= kHalfOfThem || m * n >= (k <= kMostIdle ? kManyCells : kLeastCells);
 }
 
 int64_t conv_split_positions(int64_t m) {

@@ -308,18 +308,24 @@ def test_weight_gradient_over_its_own_operand(P):
     H.assert_bit_exact(both.download(), (gradient @ unrolled.T).astype(np.float32).reshape(-1), "convolution-backward-weights")
 
 
-# (batch, in channels, out channels, side, window, stride): the float products that are formed in three pieces to a float: 64
-# cells or more over 288 blocks of 256 positions; 20 to 64 out channels over 128 rows or more; more than 64; runs of six
-# pieces of positions or more.  Remainders of 32 cells, 32 rows, 16 channels and 256 positions.
+# (batch, in channels, out channels, side, window, stride): the float products that are formed in three pieces to a float, and
+# others beside the lines: 64 cells or more over 288 blocks of 256 positions, up to 96 cells over 384; 20 to 64 out channels over
+# 128 rows or more, beyond 32 of them in workspaces of 42 MB and more; more than 64; runs of six pieces of positions or more.
+# Remainders of 32 cells, 32 rows, 16 channels and 256 positions.
 SPLIT_CASES = [
-    (46, 8, 33, 40, 3, 1),      # 72 cells, 288 blocks, images of 1600 positions: a block spans two
-    (150, 7, 64, 23, 3, 1),     # 63 cells: the float kernel; 310 blocks of 79350 positions
-    (150, 11, 65, 23, 3, 1),    # 99 cells: the last tile of three; 65 rows: two tiles
+    (46, 8, 33, 40, 3, 1),      # 72 cells, 288 blocks: the float kernel
+    (62, 8, 33, 40, 3, 1),      # 388, images of 1600 positions: a block spans two
+    (190, 7, 64, 23, 3, 1),     # 63 cells: the float kernel; 393 blocks of 100510 positions
+    (150, 7, 64, 23, 3, 1),     # 310 of 79350
+    (150, 11, 65, 23, 3, 1),    # 99 cells: the last tile of three; 65 rows: two tiles; 620 blocks: the float kernel
+    (170, 11, 65, 23, 3, 1),    # 704
     (30, 4, 31, 50, 5, 1),      # 100 cells of 25 taps, one tile of rows, 294 blocks
     (41, 15, 20, 40, 3, 1),     # 135 rows over 20 channels and 65600 positions
     (40, 15, 20, 40, 3, 1),     # 64000 positions: the float kernel
-    (7, 57, 33, 36, 3, 1),      # 513 rows over 33 channels and 9072 positions, in several runs of rows
-    (2, 57, 64, 68, 3, 1),      # 9248 positions, 64 channels
+    (7, 57, 33, 36, 3, 1),      # 513 rows over 33 channels and 9072 positions, 19 MB: the float kernel
+    (36, 57, 33, 36, 3, 1),     # 46656, 96 MB
+    (2, 57, 64, 68, 3, 1),      # 9248 positions, 64 channels, 19 MB: the float kernel
+    (5, 57, 64, 68, 3, 1),      # 23120, 47 MB, in several runs of rows
     (3, 33, 66, 20, 1, 1),      # 33 rows over 66 channels
     (5, 20, 200, 19, 3, 2),     # 180 rows over 200
     (6, 15, 129, 33, 3, 1),     # 135 rows over 129 channels, weight gradient over six long runs
@@ -335,10 +341,10 @@ def test_products_in_pieces_at_the_edges_of_their_tiles(P, case):
 # The output formed in pieces over a single image of one or two rows: the window reaches below it (test_conv_gather.py has the
 # arithmetic).  Those cells are zero, also in the unrolled input.
 @pytest.mark.parametrize("case", [
-    (1, 8, 5, 1, 80000, 3, 3, 1, 1, 1, 1),
+    (1, 8, 5, 1, 100000, 3, 3, 1, 1, 1, 1),
     (1, 4, 5, 2, 40000, 5, 5, 2, 2, 1, 1),
-    (1, 16, 5, 1, 80000, 1, 5, 0, 2, 1, 1),
-    (2, 8, 5, 1, 40000, 3, 3, 1, 1, 1, 1),
+    (1, 16, 5, 1, 100000, 1, 5, 0, 2, 1, 1),
+    (2, 8, 5, 1, 50000, 3, 3, 1, 1, 1, 1),
 ], ids=lambda c: "x".join(map(str, c)))
 def test_products_in_pieces_over_low_images(P, case):
     check_products(P, *case)
@@ -347,11 +353,14 @@ def test_products_in_pieces_over_low_images(P, case):
 def in_pieces(batch, m, k, n_rows, taps):
     """Whether the output of m channels over k cells, its weight gradient and its input gradient are formed in pieces."""
     n = batch * n_rows
-    forward = forward_route(batch, m, k, n_rows, taps) == "conv_product" and k >= 64 and -(-m // 64) * -(-n // 256) >= 288
+    blocks = -(-m // 64) * -(-n // 256)
+    forward = forward_route(batch, m, k, n_rows, taps) == "conv_product" and k >= 64 and blocks >= (384 if k <= 96 else 288)
+    forward = forward and not (k <= 112 and m > 32 and 512 < blocks <= 640)
     pieces, fit = batch * -(-n_rows // 64), max(batch * max(1, min(64, n_rows // 4096)), (1 << 20) // (4 * m * k))
     want = 1 if pieces <= 3 else max(1, min(512 // (-(-m // 64) * -(-k // 64)), fit, pieces))
     weights = weight_route(batch, m, k, n_rows).startswith("conv_weight") and min(m, k) > 32 and -(-pieces // want) >= 6
     data = k > 32 if m > 64 else m >= 20 and k >= 128 and n >= (8192 if k >= 512 else 65536)
+    data = data and (not 32 < m <= 64 or k * n >= (18 if m <= 40 else 10) << 20)
     return forward, weights, data_route(batch, k, m, n_rows) == "conv_product+conv_roll" and data
 
 
@@ -392,7 +401,7 @@ def test_which_products_are_formed_in_pieces(P, case):
 
 # Each kernel of the products in pieces: the output over 33 and over 31 channels, the weight gradient, the input gradient over
 # 20, 33, 66 and 65 channels (the last two in tiles of 64 and of 128 rows); and one that is formed in floats throughout
-@pytest.mark.parametrize("case", [(46, 8, 33, 40, 3), (30, 4, 31, 50, 5), (41, 15, 20, 40, 3), (7, 57, 33, 36, 3),
+@pytest.mark.parametrize("case", [(62, 8, 33, 40, 3), (30, 4, 31, 50, 5), (41, 15, 20, 40, 3), (36, 57, 33, 36, 3),
                                   (3, 33, 66, 20, 1), (150, 11, 65, 23, 3), (6, 15, 129, 33, 3), (5, 20, 200, 19, 3)], ids=lambda c: "x".join(map(str, c)))
 def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
     """An infinity, a NaN and floats that the pieces do not hold, in the weights and in both gradients' operands: the blocks
@@ -435,7 +444,7 @@ def test_products_in_pieces_at_the_ends_of_the_number_range(P, case):
 def test_products_in_pieces_of_small_operands(P, exponent):
     """Floats of 24 bits around the least normal one, under weights near 2^100: the remainders that the pieces are cut from are
     denormal.  The oracle sums in double; bar: 1e-6 of the sum of magnitudes."""
-    batch, cin, cout, side, k = 46, 8, 33, 40, 3
+    batch, cin, cout, side, k = 62, 8, 33, 40, 3
     n_rows, n_cols = side * side, cin * k * k
     desc, geometry = H.conv_desc(cin, cout, k, k, 1, 1, 1, 1), (batch, side, side, side, side)
     rng = np.random.default_rng(-exponent)
