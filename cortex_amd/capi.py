@@ -220,8 +220,9 @@ def check(status: int) -> None:
 
 def call(name: str, *args) -> None:
     """Calls entry point ``name`` and raises on a non-zero status.  A ``ct_dims`` may also be given as its bytes."""
-    if bytes in map(type, args):
-        args = [C.byref(CtDims.from_buffer_copy(a)) if type(a) is bytes else a for a in args]
+    if bytes in map(type, args):    # elsewhere, for instance as the source of a copy, bytes are an address
+        types = (*PROTOTYPES.get(name, ()), *[None] * len(args))
+        args = [C.byref(CtDims.from_buffer_copy(a)) if type(a) is bytes and t is _DP else a for a, t in zip(args, types)]
     status = getattr(_lib or lib(), name)(*args)
     if status != 0:
         check(status)

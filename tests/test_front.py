@@ -151,6 +151,27 @@ def test_calls_go_to_the_library_that_is_set(monkeypatch):
     assert len(calls) == 1
 
 
+def test_bytes_are_dimensions_only_where_the_entry_point_takes_them(monkeypatch):
+    """Bytes in the place of any other pointer are an address, as ctypes has it: the source of a copy, of whatever length."""
+    class Library:
+        def ct_memcpy_async(self, *args):
+            calls.append(args)
+            return 0
+
+        def ct_assign(self, stream, dest, dest_dims, *args):
+            calls.append((dest, dest_dims._obj.ndim, list(dest_dims._obj.shape[:2])))
+            return 0
+
+    calls = []
+    monkeypatch.setattr(capi, "_lib", Library())
+    for source in (b"", bytes(3), bytes(C.sizeof(capi.CtDims)), bytes(5000)):
+        capi.call("ct_memcpy_async", 64, source, len(source), 1, None)
+        assert calls.pop() == (64, source, len(source), 1, None)
+    packed = bytes(capi.make_dims([4, 5], [5, 1]))
+    capi.call("ct_assign", None, 64, packed, 64, packed, capi.F32, 20)
+    assert calls.pop() == (64, 2, [4, 5])
+
+
 @pytest.mark.parametrize("stale", [False, True])
 def test_a_build_without_a_host_compiler_leaves_the_front_end_in_python(tmp_path, monkeypatch, capsys, stale):
     from cortex_amd import build
