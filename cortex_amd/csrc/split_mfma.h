@@ -1,20 +1,24 @@
-// split_mfma.h -- float products on the bfloat16 matrix cores without giving up a bit of the operands.
+// split_mfma.h -- float products on the bfloat16 matrix cores, of operands that are held to the last bit.
 //
 // v_mfma_f32_*_f32 multiplies 157 TFLOP/s, v_mfma_f32_*_bf16 2500.  A float has 24 significant bits, a bfloat16 eight and
 // the same range of exponents: x = hi + mid + lo, each piece the rest of the one before it rounded to nearest, holds every
 // float exactly, so that
-//   a * b = hi hi + (hi mid + mid hi) + (hi lo + mid mid + lo hi) + (mid lo + lo mid + lo lo),
-// whose last bracket is at most 2^-25 of the product and is left out: six products in place of one, each exact in the
-// matrix cores' float sums.  hi hi is summed apart from the rest, in two accumulators that are added at the end: the
-// rounding errors of the five small ones are 2^-8 of the large one's.  Error against 64 bits, relative 2-norm over normal
-// operands (k terms; the library's float product in brackets): k 784 1.6e-7 (2.6e-7), 1024 1.9e-7 (5.7e-7), 4096 4.0e-7
-// (1.15e-6).
+//   a * b = hi hi + (hi mid + mid hi) + (hi lo + mid mid + lo hi) + (mid lo + lo mid + lo lo)
+// (the decomposition of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019).  The last bracket is less than 2^-24 of the product (0.99 of that in the square of
+// 1 + 2^-8 - 2^-17, a sixth on average) and is left out: six products in place of one, each exact in the matrix cores' float
+// sums.  hi hi is summed apart from the rest, in two accumulators that are added at the end: the rounding errors of the five
+// small ones are 2^-8 of the large one's.  A float sum rounds after every product, these once for sixteen: from two terms on
+// that is more than what is left out, and a product by itself is formed from the floats.  Error against 64 bits, relative
+// 2-norm over normal operands (k terms; the library's float product in brackets): k 784 1.6e-7 (2.6e-7), 1024 1.9e-7
+// (5.7e-7), 4096 4.0e-7 (1.15e-6).
 //
 // Range.  The pieces of a small float would be denormal and those of the smallest would not be held at all, so operands
 // are multiplied by 2^16 on the way in (any float, denormals included, is then a multiple of 2^-133, the least bfloat16)
-// and sums by 2^-32 on the way out.  A float of 2^111 or more, an infinity or a NaN becomes an infinity or a NaN in its
-// row's or column's sums (an infinity's rest is NaN), and so does a result of 2^95 or more: a block that finds one in its
-// sums forms them again from the floats themselves, on v_mfma_f32_32x32x2_f32, and stores that.
+// and sums by 2^-32 on the way out.  Pieces below 2^-126 remain, of floats below about 2^-118: neither the conversion nor
+// v_dot2_f32_bf16 nor the matrix cores flush them.  A float of 2^112 or more, an infinity or a NaN becomes an infinity or a
+// NaN in its row's or column's sums (an infinity's rest is NaN), and so does a result of 2^96 or more: a block that finds one
+// in its sums forms them again from the floats themselves, on v_mfma_f32_32x32x2_f32, and stores that.
 #pragma once
 
 #include "common.h"
