@@ -326,13 +326,9 @@ constexpr uint32_t kOutside = 0x80000000u;
 // A workspace that the last-level cache does not hold goes past the caches: a wave's loads wait for the stores in front of
 // them, and those for room in the caches ([64, 64, 56, 56] under 64 windows of 3 x 3, 462 MB, us: forward 207 -> 193, input
 // gradient with the roll back 248 -> 234; but [50, 248, 23, 23] under 21, 236 MB, which the roll back then reads from
-// memory, 98 -> 186).  Only where the rows of the workspace begin on whole sectors of 64 bytes: others are written to memory in
-// parts, each read first ([132, 125, 41, 41] under 22 of 3 x 3, 1521 positions a row: input gradient 510 us, past the caches
-// 862; [65, 27, 63, 63] under 17 of 5 x 5, 3481: forward 238 and 278).  At a stride the roll back skips about in the workspace and needs the caches ([109, 41, 80, 80] under 60
-// of 5 x 5 at stride 2: input gradient 486 us, past the caches 641).
+// memory, 98 -> 186).  Which ones: past_the_caches.
 constexpr int kStreaming = 2;
 constexpr int64_t kLastLevelCache = int64_t(256) << 20;
-constexpr uint32_t kWholeSectors = 16;
 template <bool kPast>
 __device__ __forceinline__ void store_cell(float x, __amdgpu_buffer_rsrc_t cells, uint32_t at, uint32_t row) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), cells, at, row, kPast ? kStreaming : 0);
@@ -1408,6 +1404,27 @@ int64_t conv_split_positions(int64_t m) {
   return kMostTiles / ((m + 31) / 32) * 128;
 }
 
+// Where the rows of the workspace begin on whole sectors of 64 bytes; others are written to memory in parts, each read first.
+// Input gradients then lose ([132, 125, 41, 41] under 22 of 3 x 3, 1521 positions a row, us: 510, past the caches 862), and so
+// they do at a stride, where the roll back skips about in the workspace and needs the caches ([109, 41, 80, 80] under 60 of
+// 5 x 5 at stride 2: 486 and 641).  Forward passes of 32 rows and more have products enough to hide it: 46 shapes 1.01 to
+// 1.41 times as long through the caches ([209, 12, 57, 57] under 51 of 3 x 3, 3249 positions, 116 and 164; [63, 15, 101, 101]
+// under 58 135 and 189), but for windows of one cell, whose stores follow each other as fast as they can ([88, 90, 102, 102]
+// under 43 201 and 185).  Of fewer rows it is 50 shapes of 0.83 to 1.07 ([65, 27, 63, 63] under 17 of 5 x 5, 3481: 278 and
+// 235), but 1.06 to 1.29 in nine where the rows begin on 16 bytes and the gathers take longest, at a stride, or the sums are
+// short ([68, 57, 102, 102] under 25 of 3 x 3 at stride 2, 2500: 143 and 185; [164, 8, 88, 88] under 5 of 3 x 3, 7396: 116 and
+// 134).
+static bool past_the_caches(const ConvProductArgs& a, bool forward) {
+  constexpr uint32_t kSector = 16, kPiece = 4, kFullTile = 32, kShortSums = 192;
+  if ((int64_t)a.images * a.conv_image * (int64_t)sizeof(float) <= kLastLevelCache) return false;
+  const bool whole = a.n_rows % kSector == 0 && reinterpret_cast<uintptr_t>(a.workspace) % (kSector * sizeof(float)) == 0;
+  const bool strided = a.sx != 1 || a.sy != 1;
+  if (!forward) return whole && !strided;
+  if (whole) return true;
+  if (a.kw * a.kh == 1) return false;
+  return a.m >= kFullTile || (a.n_rows % kPiece == 0 && (strided || a.k <= kShortSums));
+}
+
 void conv_product_split(hipStream_t s, ConvProductArgs a, bool forward) {
   const auto grid = [&](uint32_t m_tiles, uint32_t positions) {
     a.units = m_tiles * ((a.n + positions - 1) / positions);
@@ -1415,9 +1432,7 @@ void conv_product_split(hipStream_t s, ConvProductArgs a, bool forward) {
     return dim3((a.units + kXcds - 1) / kXcds * kXcds);
   };
   const dim3 block(kPositions);
-  const bool past = (int64_t)a.images * a.conv_image * (int64_t)sizeof(float) > kLastLevelCache &&
-                    a.n_rows % kWholeSectors == 0 && reinterpret_cast<uintptr_t>(a.workspace) % (kWholeSectors * sizeof(float)) == 0 &&
-                    (forward || (a.sx == 1 && a.sy == 1));
+  const bool past = past_the_caches(a, forward);
   if (forward) {
     const uint32_t bm = a.m <= 32 ? 32 : 64;
     const dim3 blocks = grid((a.m + bm - 1) / bm, kPositions);

@@ -350,6 +350,40 @@ def test_products_in_pieces_over_low_images(P, case):
     check_products(P, *case)
 
 
+@pytest.mark.parametrize("case", [
+    (64, 12, 33, 103, 3, 1),     # rows of 10609 positions
+    (160, 20, 5, 100, 3, 2),     # of 2500, few rows, at a stride
+    (48, 16, 24, 104, 3, 1),     # of 10816, whole sectors: the input gradient too, rolled back from the end
+], ids=lambda c: "x".join(map(str, c)))
+def test_workspaces_beyond_the_last_level_cache(P, case):
+    """Unrolled matrices of more than 256 MiB go past the caches, those of half of the images do not: all of it agrees to the bit
+    (a position's sum does not depend on the images around it)."""
+    batch, cin, cout, side, k, stride = case
+    out_side = (side + 2 * (k // 2) - k) // stride + 1
+    n_rows, n_cols, part = out_side ** 2, cin * k * k, batch // 2
+    cells = n_rows * n_cols
+    assert part * cells * 4 < 256 << 20 < batch * cells * 4 and in_pieces(part, cout, n_cols, n_rows, k * k)[0]
+    desc, geometry = H.conv_desc(cin, cout, k, k, k // 2, k // 2, stride, stride), (side, side, out_side, out_side)
+    rng = np.random.default_rng(cin)
+    normal = lambda n: H.Buf(rng.standard_normal(n).astype(np.float32), gpu=True)
+    x, w, g = normal(batch * cin * side * side), normal(cout * n_cols), normal(batch * cout * n_rows)
+    zeros = lambda n: [H.Buf(np.zeros(n, np.float32), gpu=True) for _ in range(2)]
+    out, ig, work = zeros(batch * cout * n_rows), zeros(batch * cin * side * side), zeros(batch * cells)
+    try:
+        for which, to, per_image, source, source_image in (("forward", out, cout * n_rows, x, cin * side * side),
+                                                           ("backward_data", ig, cin * side * side, g, cout * n_rows)):
+            H.convolution(P.hip, which, vec(to[0]), 0.0, vec(source), vec(w), vec(work[0]), desc, batch, *geometry)
+            for first in (0, part):
+                some = lambda buf, n: View(buf, [part * n], offset=first * n)
+                H.convolution(P.hip, which, some(to[1], per_image), 0.0, some(source, source_image), vec(w), some(work[1], cells), desc,
+                              part, *geometry)
+            H.assert_bit_exact(to[0].download(), to[1].download(), which)
+            H.assert_bit_exact(work[0].download(), work[1].download(), "unrolled, " + which)
+    finally:
+        for buf in (x, w, g, *out, *ig, *work):
+            buf.free()
+
+
 def in_pieces(batch, m, k, n_rows, taps):
     """Whether the output of m channels over k cells, its weight gradient and its input gradient are formed in pieces."""
     n = batch * n_rows
