@@ -9,7 +9,8 @@
 // library's products, with the float kernels and with the split ones: forward 264, 235, 193; weight
 // gradient 220, 178, 150 (its sum over the splits, 5, included); input gradient with the roll back 340, 316, 234;
 // [128, 16, 28, 28] under 32 windows 33, 28, 25; 67, 31, 31 (a float kernel); 36, 36, 35.  Other shapes go
-// either way, and the rules of ops_conv.hip (library or not) and below (which family) draw the lines.
+// either way, and the rules of ops_conv.hip (library or not; drawn through the float kernels' times) and below (which
+// family) draw the lines.
 //   float: what is left is latency: 3.3 to 3.8 waves a SIMD are resident, and the matrix cores of a compute unit are busy
 //     for 51 (forward), 60 (weight gradient) and 54 % (input gradient) of the time that it is.
 //   split: forward and input gradient wait for their loads of single floats behind the stores of the workspace (forward 207
@@ -35,8 +36,8 @@
 // shapes: outputs 0.87 (0.40 to 1.10), input gradients 0.80 (0.33 to 1.04), weight gradients 0.45
 // (0.07 to 1.08); those above 1.04 at errors of 3e-8 to 7e-8.  Chains of 128: up to 1.5, 1.3 and 1.6.
 // The bfloat16 matrix cores round once for sixteen products, the forward sums and those over up to 64 channels run through,
-// others end after 128 products, in the weight gradient after 64 (then in double): over 70 shapes errors of 0.6 to 0.8 of
-// those of the float kernels, 1.0 at the most.
+// others end after 128 products, in the weight gradient after 64 (then in double): over 194 shapes errors of 0.61 to 1.0 of
+// those of the float kernels, but for two forward passes of 1.06 and 1.11 at errors of 1.4e-7 and 1.6e-7.
 #include <algorithm>
 #include <type_traits>
 
@@ -468,28 +469,68 @@ __global__ void __launch_bounds__(kPositions, 2) conv_forward_kernel(const ConvP
     for (int p = 0; p < kSplitPieces; ++p) *reinterpret_cast<u32x4*>(&lds[buffer][p][tile_at(left_row, left_chunk)]) = pieces[p];
   };
 
-  f32x16 sums[2][MT][2];   // the products of the leading pieces; all others
+  // The sums of a tile of 32 k: the ten small products of its halves, behind them the two large ones, so that few roundings
+  // are at the size of a tile's sum and none at that of the total but its own addition.  Summed through, the leading pieces
+  // apart from the others, the errors were 1.3 to 1.45 times the float kernel's over operands of one sign and up to 1.28 over
+  // long sums of either; now they are 0.66 to 0.92 (k 576, normal operands 1.35e-7 -> 0.93e-7, the float kernel's 1.27e-7;
+  // uniform ones 1.34e-7 -> 0.68e-7, 0.93e-7), for 0 to 4 % of the time.  Where there is one tile of rows the totals are added
+  // up a tile later: right behind the products they waited for them ([32, 32, 56, 56] under 32 36.5 us, later 32.8).
+  constexpr bool kLater = MT == 1;
+  f32x16 sums[MT][2], total[MT][2];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) sums[0][t][u] = sums[1][t][u] = zero16();
+    for (int u = 0; u < 2; ++u) sums[t][u] = total[t][u] = zero16();
+  auto add_up = [&] {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) total[t][u] += sums[t][u];
+  };
   float raw[2][16];
-  auto multiply = [&](int buffer, int part, const bf16x8 (&r)[2][kSplitPieces]) {
+  bf16x8 leading[2];   // of the positions, in the first half
+  auto multiply = [&](int buffer, int part, const bf16x8 (&r)[2][kSplitPieces], bool last) {
+    auto weights_at = [&](int t, int half_tile, int p) {
+      return *reinterpret_cast<const bf16x8*>(&lds[buffer][p][tile_at(t * 32 + row, half_tile * 2 + half)]);
+    };
     bf16x8 l[MT][kSplitPieces];
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int p = 0; p < kSplitPieces; ++p)
-        l[t][p] = *reinterpret_cast<const bf16x8*>(&lds[buffer][p][tile_at(t * 32 + row, part * 2 + half)]);
-#pragma unroll
-    for (int i = 0; i < kSplitProducts; ++i)
+      for (int p = 0; p < kSplitPieces; ++p) l[t][p] = weights_at(t, part, p);
+    if (part == 0) {
+      if (kLater) add_up();
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x16& sum = sums[i + 1 < kSplitProducts][t][u];
-          sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[t][kSplitLeft[i]], r[u][kSplitRight[i]], sum, 0, 0, 0);
-        }
+        for (int u = 0; u < 2; ++u) sums[t][u] = zero16();
+    }
+#pragma unroll
+    for (int i = 0; i + 1 < kSplitProducts; ++i)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          sums[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[t][kSplitLeft[i]], r[u][kSplitRight[i]], sums[t][u], 0, 0, 0);
+    if (part == 1) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const bf16x8 first = weights_at(t, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sums[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(first, leading[u], sums[t][u], 0, 0, 0);
+      }
+    }
+    if (part == 1 || last) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sums[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[t][0], r[u][0], sums[t][u], 0, 0, 0);
+      if (!kLater) add_up();
+    }
+    if (part == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) leading[u] = r[u][0];
+    }
   };
   load_left(0);
   gather(0, raw[0], kSixteen);
@@ -514,7 +555,7 @@ __global__ void __launch_bounds__(kPositions, 2) conv_forward_kernel(const ConvP
       split_positions(x, r, split_weights);
       gather(k + BK, x, kSixteen);
       if (part == 0) load_left(k0 + 2 * BK);
-      multiply(buffer, part, r);
+      multiply(buffer, part, r, false);
     }
     __syncthreads();
   }
@@ -537,21 +578,20 @@ __global__ void __launch_bounds__(kPositions, 2) conv_forward_kernel(const ConvP
       }
       bf16x8 r[2][kSplitPieces];
       split_positions(x, r, split_weights);
-      multiply(0, part, r);
+      multiply(0, part, r, k + 16 >= a.k);
     }
   }
 
+  if (kLater) add_up();
   bool found = false;
-  f32x16 total[MT][2];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const float sum = sums[0][t][u][e] + sums[1][t][u][e];
-        found |= not_finite(sum);
-        total[t][u][e] = sum * kSplitUnscale;
+        found |= not_finite(total[t][u][e]);
+        total[t][u][e] *= kSplitUnscale;
       }
   if (__syncthreads_or(found))
     product_in_float<MT>(
@@ -1373,7 +1413,9 @@ void conv_product(hipStream_t s, ConvProductArgs a, bool forward) {
 // ([20, 17, 17, 17] under 31, 23 blocks, 13 and 16): the more the shorter the sums ([67, 8, 71, 71] under 19 at stride 2, k
 // 72, 321 blocks, 15.2 and 17.5; from 384 on 0.84 to 1.0 of the float kernel's time).  Of more than 32 rows two blocks share a
 // unit, and short sums are over before a last round of few blocks is ([115, 73, 26, 26] under 104 of 1 x 1, k 73, 602 blocks,
-// 25 and 29; 12 of 14 such shapes of 513 to 640 blocks and up to 112 cells 0.96 to 1.14).
+// 25 and 29; 12 of 14 such shapes of 513 to 640 blocks and up to 112 cells 0.96 to 1.14).  Sums of 64 to 80 cells under 1 x 1
+// windows over 700 to 1600 blocks of full tiles take longer too (64 cells 1.07 to 1.18, [16, 64, 56, 56] under 256 27 and
+// 30.5; 80 up to 1.1; 88 and more 0.84 to 1.05) and stay here for their errors, two thirds of the float kernel's.
 // Input gradient (k out channels): with many of them the general split kernel throughout ([32, 256, 14, 14] under 256 103
 // and 85, [134, 94, 15, 15] under 145 122 and 107; of 65 to 80, a third tile mostly idle, 0.96 to 1.08 of the float kernel's
 // time); with up to 64 the kernel that keeps them in registers where the rows pay for that and the positions fill the chip

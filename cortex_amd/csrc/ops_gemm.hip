@@ -8,12 +8,13 @@
 //
 // Times of products, in us, the library's second: [1024, 4096] over 4096 k, b stored [n][k] 197 and 271, stored [k][n] 203
 // and 261; [4096, 4096] over 1024, both stored [k][.] 214 and 274; 4096 cubed 725 and 1121; 2048 cubed 94 and 133;
-// [64, 4096] over 4096 24 and 114; [128, 784] over 128 4.5 and 7.2; [128, 128] over 784 5.5 and 6.9.  Over 900 products of
-// layers of 1 to 4096 a side, whole calls one after the other: 1.47 times the library's speed in the geometric mean, 0.86 to
-// 4.3 in 98 % of them, 0.72 at the least.  Where it is below 0.9 they are of three kinds: a and b stored with their k side by
-// side, 500 to 1500 of them, over 70 to 700 tiles of 32 x 32 ([457, 132] over 1056 10.2 and 7.2); 65 to 275 k over 1 to 2
-// million results ([1682, 1039] over 93 9.9 and 7.5); and a chain of blocks that just misses a round.
-// Errors against 64 bits, of the library's: 0.05 to 1.0, 0.34 in the median.
+// [64, 4096] over 4096 24 and 114; [128, 784] over 128 4.5 and 7.2; [128, 128] over 784 5.5 and 6.9.  Over 1350 products of
+// layers of 1 to 4096 a side, whole calls one after the other: 1.62 times the library's speed in the geometric mean, 0.87 to
+// 7 in 98 % of them, 0.58 at the least.  60 are below 0.95: sums of 50 to 200 k over half a million results and more
+// ([878, 1290] over 66 9.2 and 6.3); of 400 to 1500 over 200 to 500 tiles of 32 x 32 ([851, 572] over 1451 27.7 and 16.1); a few
+// results over 2700 k and more, where two launches cost what they gain ([2, 56] over 3909 15.1 and 12.8); and chains of blocks
+// that just miss a round.  They are not handed back: the library's errors are two to seven times as large there.
+// Errors against 64 bits, of the library's: 0.05 to 1.0, 0.30 in the median.
 //
 // Tiles and their choice: below, at expected_time.
 #include <algorithm>

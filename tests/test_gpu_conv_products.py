@@ -398,6 +398,25 @@ def in_pieces(batch, m, k, n_rows, taps):
     return forward, weights, data_route(batch, k, m, n_rows) == "conv_product+conv_roll" and data
 
 
+@pytest.mark.parametrize("cout", [31, 33])     # one tile of rows and two
+@pytest.mark.parametrize("positive", [False, True])
+def test_outputs_in_pieces_round_as_short_chains_do(P, cout, positive):
+    """Of either sign and of one, whose sums grow with every product: the error of an output formed in pieces is no larger than
+    that of chains of eight products, the float kernel's."""
+    batch, cin, side, k = 30, 20, 50, 3
+    n_rows, n_cols = side * side, cin * k * k
+    desc, geometry = H.conv_desc(cin, cout, k, k, 1, 1, 1, 1), (batch, side, side, side, side)
+    rng = np.random.default_rng(cout)
+    values = lambda n: (rng.random(n) if positive else rng.standard_normal(n)).astype(np.float32)
+    inp, weights, out = P.buf(values(batch * cin * n_rows)), P.buf(values(cout * n_cols)), P.buf(np.zeros(batch * cout * n_rows, np.float32))
+    work = P.buf(np.zeros(batch * n_rows * n_cols, np.float32))
+    assert in_pieces(batch, cout, n_cols, n_rows, k * k)[0]
+    H.convolution(P.hip, "forward", vec(out), 0.0, vec(inp), vec(weights), vec(work), desc, *geometry)
+    unrolled = work.download()[:n_cols * n_rows].reshape(n_cols, n_rows)     # of the first image
+    exact, bound = rounding_error(weights.init.reshape(cout, n_cols), unrolled, 8)
+    assert np.linalg.norm(out.download()[:cout * n_rows].reshape(cout, n_rows) - exact) <= bound
+
+
 @pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: "x".join(map(str, c)))
 def test_which_products_are_formed_in_pieces(P, case):
     """Sums of one product of two floats and zeros: the float kernels and the library round it once.  The pieces leave out up to
