@@ -27,17 +27,19 @@ bool debug_sync();
 // slot; a call that needs two live temporaries uses two slots.
 enum ScratchSlot { kScratchReduce = 0, kScratchAccumA = 1, kScratchAccumB = 2, kScratchSlots = 3 };
 int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot = kScratchReduce);
-// The same where the caller can do without: null, and no error, if the block is too small and cannot grow, for want of memory
-// or because the stream is being captured.
-void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot = kScratchReduce);
 // The block as it is, if it is as large: null rather than another.
 void* stream_scratch_held(hipStream_t s, size_t bytes, int slot = kScratchReduce);
+// Whether ct_stream_reserve_scratch made it.
+bool stream_scratch_reserved(hipStream_t s, int slot);
+// Scratch for a caller that can do without, null if there is too little and no more to be had, for want of memory or because
+// the stream is being captured.  No call waits for it: a block that has become too small is kept until the stream is destroyed,
+// and the next is at least twice as large.
+void* stream_scratch_kept(hipStream_t s, size_t bytes);
 void release_stream_scratch(hipStream_t s);
 
 // Scratch of a stream for the partial sums of a matrix product, and the stream's right to launch what uses it: two threads may
-// form products on one stream, and one's launches must not come between the other's.  A block that has become too small is kept
-// until the stream is destroyed, for a recorded graph may still write to it: blocks double, so that all of them together stay
-// below twice kMostProductScratch.
+// form products on one stream, and one's launches must not come between the other's.  Blocks are kept as those above, for a
+// recorded graph may still write to them; all of them together stay below twice kMostProductScratch.
 constexpr size_t kMostProductScratch = size_t(256) << 20;
 class ProductScratch {
  public:

@@ -33,17 +33,17 @@ struct ScratchKey {
     return slot < o.slot;
   }
 };
-struct ScratchBlock { void* ptr; size_t bytes; };
+struct ScratchBlock { void* ptr; size_t bytes; bool reserved; };
 std::mutex g_scratch_mutex;
 std::map<ScratchKey, ScratchBlock> g_scratch;
 
-struct ProductBlocks {
-  std::mutex mutex;            // held while a product's launches are made
+struct KeptBlocks {
+  std::mutex mutex;            // of a product: held while its launches are made
   std::vector<void*> blocks;   // the last one is in use
   size_t bytes = 0;
 };
-constexpr int kProductKey = kScratchSlots;   // in the place of a slot
-std::map<ScratchKey, std::unique_ptr<ProductBlocks>> g_products;
+enum KeptKey { kKeptProduct = kScratchSlots, kKeptSort, kKeptEnd };   // in the place of a slot
+std::map<ScratchKey, std::unique_ptr<KeptBlocks>> g_kept;
 }  // namespace
 
 int stream_scratch(hipStream_t s, size_t bytes, void** out, int slot) {
@@ -88,57 +88,61 @@ void* stream_scratch_held(hipStream_t s, size_t bytes, int slot) {
   return it != g_scratch.end() && it->second.bytes >= bytes ? it->second.ptr : nullptr;
 }
 
-void* stream_scratch_if_any(hipStream_t s, size_t bytes, int slot) {
+bool stream_scratch_reserved(hipStream_t s, int slot) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  const auto it = g_scratch.find(ScratchKey{dev, s, slot});
+  return it != g_scratch.end() && it->second.reserved;
+}
+
+namespace {
+KeptBlocks* kept_blocks(hipStream_t s, KeptKey key) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  ScratchBlock& b = g_scratch[ScratchKey{dev, s, slot}];
-  if (b.bytes >= bytes) return b.ptr;
-  const size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
-  void* const grown = allocate_if_any(s, want);
-  if (!grown) return nullptr;   // the block stays what it was
-  if (b.ptr) {
-    // earlier kernels of this stream may still be reading the old block
-    if (hipStreamSynchronize(s) != hipSuccess) {
-      (void)hipFree(grown);
-      return nullptr;   // the error is the stream's and stays with it
-    }
-    (void)hipFree(b.ptr);
+  auto& entry = g_kept[ScratchKey{dev, s, key}];
+  if (!entry) entry = std::make_unique<KeptBlocks>();
+  return entry.get();
+}
+
+// Under the blocks' lock.
+void* last_block(KeptBlocks* k, hipStream_t s, size_t bytes) {
+  if (k->bytes < bytes) {
+    size_t want = std::max(size_t(1) << 20, 2 * k->bytes);
+    while (want < bytes) want *= 2;
+    void* const grown = allocate_if_any(s, want);
+    if (!grown) return nullptr;
+    k->blocks.push_back(grown);
+    k->bytes = want;
   }
-  b.ptr = grown;
-  b.bytes = want;
-  return grown;
+  return k->blocks.back();
+}
+}  // namespace
+
+void* stream_scratch_kept(hipStream_t s, size_t bytes) {
+  KeptBlocks* const k = kept_blocks(s, kKeptSort);
+  if (!k) return nullptr;
+  std::lock_guard<std::mutex> lock(k->mutex);
+  return last_block(k, s, bytes);
 }
 
 ProductScratch::ProductScratch(hipStream_t s, size_t bytes) {
-  int dev = 0;
-  if (bytes > kMostProductScratch || hipGetDevice(&dev) != hipSuccess) return;
-  ProductBlocks* p;
-  {
-    std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    auto& entry = g_products[ScratchKey{dev, s, kProductKey}];
-    if (!entry) entry = std::make_unique<ProductBlocks>();
-    p = entry.get();
-  }
-  lock_ = std::unique_lock<std::mutex>(p->mutex);
-  if (p->bytes < bytes) {
-    size_t want = std::max(size_t(1) << 20, 2 * p->bytes);
-    while (want < bytes) want *= 2;
-    void* const grown = allocate_if_any(s, want);
-    if (!grown) return;
-    p->blocks.push_back(grown);
-    p->bytes = want;
-  }
-  ptr_ = p->blocks.back();
+  KeptBlocks* const k = bytes > kMostProductScratch ? nullptr : kept_blocks(s, kKeptProduct);
+  if (!k) return;
+  lock_ = std::unique_lock<std::mutex>(k->mutex);
+  ptr_ = last_block(k, s, bytes);
 }
 
 void release_stream_scratch(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return;
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  if (auto it = g_products.find(ScratchKey{dev, s, kProductKey}); it != g_products.end()) {
+  for (int key = kKeptProduct; key < kKeptEnd; ++key) {
+    auto it = g_kept.find(ScratchKey{dev, s, key});
+    if (it == g_kept.end()) continue;
     for (void* block : it->second->blocks) (void)hipFree(block);
-    g_products.erase(it);
+    g_kept.erase(it);
   }
   for (int slot = 0; slot < kScratchSlots; ++slot) {
     auto it = g_scratch.find(ScratchKey{dev, s, slot});
@@ -301,6 +305,10 @@ int ct_stream_reserve_scratch(void* stream, size_t partial_bytes, size_t accumul
   if (accumulate_bytes) {
     if (int rc = stream_scratch((hipStream_t)stream, accumulate_bytes, &unused, kScratchAccumA)) return rc;
     if (int rc = stream_scratch((hipStream_t)stream, accumulate_bytes, &unused, kScratchAccumB)) return rc;
+    int dev = 0;
+    CT_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(g_scratch_mutex);
+    g_scratch[ScratchKey{dev, (hipStream_t)stream, kScratchAccumA}].reserved = true;
   }
   return CT_OK;
 }

@@ -505,14 +505,13 @@ int sort_index(hipStream_t s, const int32_t* index, uint32_t n, const int32_t** 
   };
   size_t needed = 0;
   if (n > kSortMinEntries && n <= kSortMaxEntries) {
-    // two bytes an entry more than the library's sort, for which no block that holds that one is replaced (a recorded graph
-    // may use it), nor where a stream that is being captured has no more
+    // Two bytes an entry more than the library's sort.  No block is replaced for them (a recorded graph may use it): they are
+    // in one of their own, but where a caller who wants no allocation has reserved what the library's sort needs, and where a
+    // stream that is being captured has no more.
     block = stream_scratch_held(s, index_sort_bytes(n), kScratchAccumA);
-    if (!block) {
+    if (!block && stream_scratch_reserved(s, kScratchAccumA))
       if (int rc = library_bytes(&needed)) return rc;
-      if (!stream_scratch_held(s, needed, kScratchAccumA))
-        block = stream_scratch_if_any(s, index_sort_bytes(n), kScratchAccumA);
-    }
+    if (!block && !(needed && stream_scratch_held(s, needed, kScratchAccumA))) block = stream_scratch_kept(s, index_sort_bytes(n));
     if (block) {
       index_sort(s, index, n, block, skey, perm);
       return CT_OK;

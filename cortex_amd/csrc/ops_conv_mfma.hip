@@ -35,9 +35,9 @@
 // same time.  Error against 64 bits, in units of the library's, geometric means and ranges over 280
 // shapes: outputs 0.87 (0.40 to 1.10), input gradients 0.80 (0.33 to 1.04), weight gradients 0.45
 // (0.07 to 1.08); those above 1.04 at errors of 3e-8 to 7e-8.  Chains of 128: up to 1.5, 1.3 and 1.6.
-// The bfloat16 matrix cores round once for sixteen products, the forward sums and those over up to 64 channels run through,
-// others end after 128 products, in the weight gradient after 64 (then in double): over 194 shapes errors of 0.61 to 1.0 of
-// those of the float kernels, but for two forward passes of 1.06 and 1.11 at errors of 1.4e-7 and 1.6e-7.
+// The bfloat16 matrix cores round once for eight products.  Forward sums end with a tile of 32 k, input gradients over up to
+// 64 channels run through, over more of them they end after 128 products, in the weight gradient after 64 (then in double):
+// over 194 shapes errors of 0.6 to 1.0 of those of the float kernels.
 #include <algorithm>
 #include <type_traits>
 

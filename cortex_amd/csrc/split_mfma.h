@@ -8,7 +8,7 @@
 // Higher-Precision Computations", 2019).  The last bracket is less than 2^-24 of the product (0.99 of that in the square of
 // 1 + 2^-8 - 2^-17, a sixth on average) and is left out: six products in place of one, each exact in the matrix cores' float
 // sums.  hi hi is summed apart from the rest, in two accumulators that are added at the end: the rounding errors of the five
-// small ones are 2^-8 of the large one's.  A float sum rounds after every product, these once for sixteen: from two terms on
+// small ones are 2^-8 of the large one's.  A float sum rounds after every product, these once for eight: from two terms on
 // that is more than what is left out, and a product by itself is formed from the floats.  Error against 64 bits, relative
 // 2-norm over normal operands (k terms; the library's float product in brackets): k 784 1.6e-7 (2.6e-7), 1024 1.9e-7
 // (5.7e-7), 4096 4.0e-7 (1.15e-6).

@@ -170,9 +170,10 @@ int ct_stream_destroy(void* stream);
  * those grow without synchronising, and the smaller ones stay until the stream is destroyed;
  * accumulate_bytes for each of the two blocks that accumulations into a broadcast or indexed
  * destination stage their temporaries through (at most the destination's size times the updates'
- * outermost extent; for indexed rows 18 bytes per index entry and 8 KiB up to 262144 entries (with 16, as the library's
- * sort needs, that one runs, in up to twice the time), beyond
- * that 8 bytes per entry plus the library sort's workspace, about as much again).
+ * outermost extent; for indexed rows 18 bytes per index entry and 8 KiB up to 262144 entries (with 16 reserved, as the
+ * library's sort needs, that one runs, in up to twice the time; with less, or nothing reserved, the sort has a block of
+ * its own that grows as those of products do), beyond that 8 bytes per entry plus the library sort's workspace, about as
+ * much again).
  * Zero leaves a block as it is. */
 int ct_stream_reserve_scratch(void* stream, size_t partial_bytes, size_t accumulate_bytes);
 

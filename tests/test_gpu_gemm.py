@@ -64,8 +64,8 @@ KERNELS = {(40, 40, 100): "gemm_small", (10, 20, 3700): "gemm_medium_pair+gemm_s
 def test_error_is_below_a_plain_sum_s(P, size):
     """The 2-norm of the error against 64 bits stays below that of the plain float sum, rounded after every product; the
     kernel that ran is the one that the sizes call for.  The plain sum rounds k times at the size of the sum so far; the
-    large products here once for 16 k, the five small ones, 2^-8 of them, as often each, and what is left out is below 2^-24 of
-    a product, a sixth of that on average and of either sign: a sixteenth of the roundings and a quarter of the error, of which
+    large products here once for 8 k, the five small ones, 2^-8 of them, as often each, and what is left out is below 2^-24 of
+    a product, a sixth of that on average and of either sign: an eighth of the roundings and a third of the error, of which
     half is asked for."""
     m, n, k = size
     rng = np.random.default_rng(k)
@@ -85,7 +85,7 @@ def test_error_is_below_a_plain_sum_s(P, size):
 def test_what_is_left_out_is_below_its_bound(P, size):
     """Every operand 1 + 2^-8 - 2^-17, whose pieces are 1, 2^-8 and -2^-17: the three products that are left out are the most
     that they can be, 0.99 * 2^-24 of a product, and of one sign.  The large products are ones, whose sums are exact.  Bar, in
-    2^-24 of the result: 1 for what is left out, 5 k / 16 roundings of the small sums, 2^-7 of the large one, and one each
+    2^-24 of the result: 1 for what is left out, 5 k / 8 roundings of the small sums, 2^-7 of the large one, and one each
     where the two sums, those of two groups of waves and the scale meet."""
     m, n, k = size
     x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
@@ -93,7 +93,7 @@ def test_what_is_left_out_is_below_its_bound(P, size):
     kernel, got, _ = run(P, a, b, np.zeros((m, n), np.float32), False, True, m, n, k)
     assert kernel in ("gemm_small", "gemm_medium", "gemm_medium_pair", "gemm_large"), kernel
     exact = k * float(x) ** 2
-    assert np.all(np.abs(got.astype(np.float64) - exact) <= (4 + 5 * k / 16 / 128) * 2.0 ** -24 * exact), kernel
+    assert np.all(np.abs(got.astype(np.float64) - exact) <= (4 + 5 * k / 8 / 128) * 2.0 ** -24 * exact), kernel
 
 
 @pytest.mark.parametrize("size", [(40, 50, 100), (640, 640, 50), (900, 900, 400), (2048, 2048, 256), (64, 2048, 4096), (650, 450, 255)],

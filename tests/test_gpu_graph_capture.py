@@ -275,19 +275,22 @@ def test_a_product_recorded_without_scratch_does_without(fresh):
     recorded.destroy()
 
 
-def test_a_recorded_sort_of_labels_keeps_its_scratch(fresh):
-    """Updates of 262144 rows chosen by labels, recorded on scratch that holds the library's sort of the labels (16 bytes an
-    entry) and not the kernels' own (18): eager calls between the replays take the block as it is.  Whole numbers."""
+@pytest.mark.parametrize("recorded_rows,reserved", [(262144, 4600 << 10), (262144, 0), (270000, 0)])     # more than 262144: the library's
+def test_a_recorded_sort_of_labels_keeps_its_scratch(fresh, recorded_rows, reserved):
+    """Updates of rows chosen by labels, recorded on scratch that holds the library's sort of the labels (16 bytes an entry) and
+    may not hold the kernels' own (18): eager calls of 262144 between the replays leave that block where it is.  Whole numbers."""
     stream, tensor = fresh
-    n, classes = 262144, 5000
-    capi.call("ct_stream_reserve_scratch", stream, 0, 4600 << 10)
+    classes, counts = 5000, (recorded_rows, 262144)
+    if reserved:
+        capi.call("ct_stream_reserve_scratch", stream, 0, reserved)
     rng = np.random.default_rng(5)
-    labels, y = tensor(rng.integers(0, classes, n).astype(np.int32)), tensor(whole(rng, n))
+    most = max(counts)
+    labels, y = tensor(rng.integers(0, classes, most).astype(np.int32)), tensor(whole(rng, most))
     sums = [tensor(np.zeros(classes, np.float32)) for _ in range(2)]
-    rows = [capi.make_dims([n, 1], [1, 1], [labels.ptr, None]) for _ in sums]
-    plain = dims([n, 1])
+    rows = [capi.make_dims([n, 1], [1, 1], [labels.ptr, None]) for n in counts]
 
     def add(side):
+        n, plain = counts[side], dims([counts[side], 1])
         capi.call("ct_memset", stream, sums[side].ptr, capi.F32, 0.0, classes)
         capi.call("ct_binary_accum", stream, sums[side].ptr, C.byref(rows[side]), 1.0, y.ptr, C.byref(plain), 1.0, n,
                   capi.BINARY_OPS["+"], 0, 1, capi.F32)
@@ -296,14 +299,14 @@ def test_a_recorded_sort_of_labels_keeps_its_scratch(fresh):
     capi.call("ct_stream_sync", stream)
     recorded = Recorded(hip_runtime(), stream, lambda: add(0))
     for replay in range(4):
-        host_labels, host = rng.integers(0, classes, n).astype(np.int32), whole(rng, n)
+        host_labels, host = rng.integers(0, classes, most).astype(np.int32), whole(rng, most)
         labels.upload(host_labels, stream)
         y.upload(host, stream)
         if replay:
             add(1)
         recorded.replay()
-        want = np.bincount(host_labels, weights=host, minlength=classes).astype(np.float32)
-        assert np.array_equal(sums[0].download(stream), want), replay
-        if replay:
-            assert np.array_equal(sums[1].download(stream), want), replay
+        for side in (0, 1) if replay else (0,):
+            n = counts[side]
+            want = np.bincount(host_labels[:n], weights=host[:n], minlength=classes).astype(np.float32)
+            assert np.array_equal(sums[side].download(stream), want), (replay, side)
     recorded.destroy()
