@@ -218,11 +218,16 @@ def check(status: int) -> None:
         raise CortexHipError(status, lib().ct_last_error().decode("utf-8", "replace"))
 
 
+_DIMS_AT = {name: tuple(at for at, t in enumerate(types) if t is _DP) for name, types in PROTOTYPES.items()}
+
+
 def call(name: str, *args) -> None:
     """Calls entry point ``name`` and raises on a non-zero status.  A ``ct_dims`` may also be given as its bytes."""
     if bytes in map(type, args):    # elsewhere, for instance as the source of a copy, bytes are an address
-        types = (*PROTOTYPES.get(name, ()), *[None] * len(args))
-        args = [C.byref(CtDims.from_buffer_copy(a)) if type(a) is bytes and t is _DP else a for a, t in zip(args, types)]
+        args = list(args)
+        for at in _DIMS_AT.get(name, ()):
+            if at < len(args) and type(args[at]) is bytes:
+                args[at] = C.byref(CtDims.from_buffer_copy(args[at]))
     status = getattr(_lib or lib(), name)(*args)
     if status != 0:
         check(status)
